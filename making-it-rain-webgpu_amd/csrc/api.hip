@@ -1087,9 +1087,9 @@ static void profile_group(md_group *g, int steps, double *ms) {
   for (md_system *s : g->reps) check_control(s);
 }
 
-// The autotuner: for each pair-kernel schedule in a small set (8, 16 or 32
-// list entries per work unit; 2, 3 or 4 resident waves per SIMD), rebuild
-// the lists with it and time `steps` steps launched phase by phase; keep the
+// The autotuner: for each pair-kernel schedule in a small set (list entries
+// per work unit, waves in the launch), rebuild the lists with it and time
+// `steps` steps launched phase by phase; keep the
 // fastest, record it in the cache under the group's key and report it with
 // the time of the schedule the group started with.  The schedule never
 // changes the bits (i-forces are rounded per 8 entries whatever the unit,
@@ -1111,10 +1111,11 @@ static void autotune_group(md_group *g, int steps, md_schedule *out) {
   auto add = [&](cand c) {
     if (std::find(candidates.begin(), candidates.end(), c) == candidates.end()) candidates.push_back(c);
   };
-  // the direct evaluation over unit lengths and resident waves (a longer
-  // unit means fewer i-force flushes, a shorter one finer load balance) ...
-  for (int seg : {8, 16, 32, 64, 128})
-    for (int per_simd : {2, 3, 4}) add(cand{seg, cus * 4 * per_simd, false});
+  // the direct evaluation over unit lengths and waves (four per SIMD are
+  // resident; more of them balance finer, fewer flush and load the i atoms of
+  // a super-cluster less often) ...
+  for (int seg : {8, 16, 32})
+    for (int per_simd : {4, 8, 16, 32, 64}) add(cand{seg, cus * 4 * per_simd, false});
   // ... and the compacted one at the usual shape
   add(cand{32, cus * 16, true});
   double ms[MD_PHASE_COUNT];

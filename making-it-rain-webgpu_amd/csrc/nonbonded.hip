@@ -131,6 +131,10 @@ struct md_pair_args {
   // each cluster's current bounding box in its frame (frame units; a cluster
   // of padding only holds an inverted box), written by k_nb_pack
   const int4 *cluster_lo, *cluster_hi;
+  // the energy, census and block counts of one evaluation, in MD_ENERGY_PARTS
+  // lines of their own: thousands of waves adding to one word would queue
+  // there (about 20 ns each); k_nb_forces sums the lines and clears them
+  int64_t *part;
   int64_t *energy;
   int64_t *census;  // in-cutoff pairs (md_control)
   int64_t *blocks;  // 8x8 cluster-pair blocks evaluated (md_control)
@@ -186,8 +190,8 @@ __device__ __forceinline__ const md_nb_args &md_nb_entry(const md_nb_args *T, co
 #define MD_FRAME_SHIFT 6  // Q32.32 -> 2^-26 nm
 #define MD_FRAME_UNIT 1.4901161193847656e-08f   // 2^-26 nm
 #define MD_FRAME_UNIT2 2.220446049250313e-16f   // 2^-52 nm^2
-// the pair kernel's per-atom scalings (see md_pair): charge (with sqrt K)
-// 2^26, sigma/2 2^26, 2 sqrt(eps) 2^13
+// the pair kernel's per-atom scalings (see md_pair), carried by slot_xyzq and
+// slot_lj: charge (with sqrt K) 2^26, sigma/2 2^26, 2 sqrt(eps) 2^13
 #define MD_PAIR_Q_SCALE 67108864.0f
 #define MD_PAIR_S_SCALE 67108864.0f
 #define MD_PAIR_E_SCALE 8192.0f
@@ -410,7 +414,7 @@ __global__ void k_nb_clusters(const md_nb_args *__restrict__ T, md_bmap map) {
     for (int d = 0; d < 3; ++d)
       slot_offset[d * c.nslots + slot] = (build_pos[d * c.np + a] - folded[d * c.np + a]) + origin[d];
     float4 p = atom_param[a];
-    slot_lj[slot] = make_float2(p.y, p.z);
+    slot_lj[slot] = make_float2(p.y * MD_PAIR_S_SCALE, p.z * MD_PAIR_E_SCALE);
   }
 }
 
@@ -824,15 +828,15 @@ __global__ void __launch_bounds__(64 * MD_MASK_GROUP) k_nb_masks(const md_nb_arg
   }
 }
 
-// the pair kernels' segment counters, one per XCD (md_seg_queue)
 #define MD_XCDS 8
-#define MD_CURSOR_STRIDE 16  // ints between two counters: one 64-byte line
+#define MD_PAIR_WAVES 32768
+#define MD_ENERGY_PARTS 64
+#define MD_ENERGY_STRIDE 8  // int64 words: one 64-byte line
 
 // Per step: each slot's position as f32 in its super-cluster's frame.
 // The launch's first thread also lays out the pair kernel's work: the start of
-// each replica's list segments in one numbering, and the counters the pair
-// kernel's waves take segments from, reset to 0.
-__global__ void k_nb_pack(const md_nb_args *__restrict__ T, md_bmap map, int *seg_start, int *cursor) {
+// each replica's list segments in one numbering.
+__global__ void k_nb_pack(const md_nb_args *__restrict__ T, md_bmap map, int *seg_start) {
   if (blockIdx.x == 0 && threadIdx.x < 64) {
     // the first wave: each lane one replica's segment count (two dependent
     // loads, issued by all lanes at once rather than one replica after
@@ -850,10 +854,7 @@ __global__ void k_nb_pack(const md_nb_args *__restrict__ T, md_bmap map, int *se
       if (r < map.R) seg_start[r] = run + incl - v;
       run += __shfl(incl, 63, 64);
     }
-    if (lane == 0) {
-      seg_start[map.R] = run;
-      for (int c = 0; c < MD_XCDS; ++c) cursor[c * MD_CURSOR_STRIDE] = 0;
-    }
+    if (lane == 0) seg_start[map.R] = run;
   }
   int blk;
   const md_nb_args &A = md_nb_entry(T, map, blk);
@@ -878,7 +879,7 @@ __global__ void k_nb_pack(const md_nb_args *__restrict__ T, md_bmap map, int *se
     int x = md_frame_coord(pos[a] - slot_offset[s], bad);
     int y = md_frame_coord(pos[np + a] - slot_offset[nslots + s], bad);
     int z = md_frame_coord(pos[2 * np + a] - slot_offset[2 * nslots + s], bad);
-    slot_xyzq[s] = make_int4(x, y, z, __float_as_int(A.atom_param[a].x));
+    slot_xyzq[s] = make_int4(x, y, z, __float_as_int(A.atom_param[a].x * MD_PAIR_Q_SCALE));
     if (bad) A.ctl->overflow = 3;
     lo[0] = hi[0] = x;
     lo[1] = hi[1] = y;
@@ -904,9 +905,19 @@ __global__ void k_nb_pack(const md_nb_args *__restrict__ T, md_bmap map, int *se
 // enough.
 // Blocks laid out XCD by XCD: neighbouring clusters read j-force records of
 // neighbouring entries, so they share one L2.
-__global__ void k_nb_forces(const md_nb_args *__restrict__ T, md_bmap map) {
+__global__ void k_nb_forces(const md_nb_args *__restrict__ T, md_bmap map, int energy) {
   int blk;
   const md_nb_args &A = T[md_locate(map, md_xcd_block(blockIdx.x, gridDim.x), blk)];
+  if (energy && blk == 0 && threadIdx.x < MD_ENERGY_PARTS) {
+    // the pair kernel's energy and counts: one wave, lane per part
+    int64_t *part = A.P.part + threadIdx.x * MD_ENERGY_STRIDE;
+    int64_t *const to[3] = {A.P.energy + MD_E_PAIR, A.P.census, A.P.blocks};
+    for (int k = 0; k < 3; ++k) {
+      const int64_t v = md_wave_sum_i64(part[k]);
+      part[k] = 0;
+      if (threadIdx.x == 0) *to[k] += v;
+    }
+  }
   const int nslots = A.c.nslots, np = A.c.np;
   const int s = blk * blockDim.x + threadIdx.x;
   if (s >= nslots) return;
@@ -1091,6 +1102,47 @@ __device__ __forceinline__ float md_sum_same_i(float x) {
   return x + md_dpp<HIGH ? MD_DPP_ROR4 : MD_DPP_ROR12>(x);
 }
 
+// md_sum_same_j of three values at once: after the first step lanes l and l^8
+// hold the same sums, so lanes 0-7 of each row go on with x and 8-15 with y;
+// after the second rows 0 and 1 do, so row 1 goes on with z.  Lane l < 24 gets
+// component l/8 of j atom l%8; the additions are md_sum_same_j's, in its order.
+__device__ __forceinline__ float md_sum_same_j3(float x, float y, float z, int lane) {
+  x += md_dpp<MD_DPP_ROR8>(x);
+  y += md_dpp<MD_DPP_ROR8>(y);
+  z += md_dpp<MD_DPP_ROR8>(z);
+  x = md_add_xor16((lane & 8) ? y : x);
+  z = md_add_xor16(z);
+  return md_add_xor32((lane & 16) ? z : x);
+}
+
+// lane l's partner l^4: the lanes of banks 0 and 2 of each row (l%8 < 4) take
+// lane l+4 (rotate right by 12), those of banks 1 and 3 lane l-4
+__device__ __forceinline__ float md_dpp_xor4(float x) {
+  const int v = __float_as_int(x);
+  const int r = __builtin_amdgcn_update_dpp(v, v, MD_DPP_ROR12, 0xf, 0x5, false);
+  return __int_as_float(__builtin_amdgcn_update_dpp(r, v, MD_DPP_ROR4, 0xf, 0xa, false));
+}
+
+// md_sum_same_i of f[0..7], lane jl keeping f[jl]'s sum: at each step a lane
+// keeps half of the values it still holds and hands its partner the other
+// half, so 7 additions replace 24.  Each addition is the butterfly's (x + x^1,
+// then ^2, then ^4), in its order.
+__device__ __forceinline__ float md_sum_i_transposed(const float (&f)[8], int jl) {
+  float a[4], b[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float keep = (jl & 1) ? f[2 * k + 1] : f[2 * k], give = (jl & 1) ? f[2 * k] : f[2 * k + 1];
+    a[k] = keep + md_dpp<MD_DPP_XOR1>(give);
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const float keep = (jl & 2) ? a[2 * k + 1] : a[2 * k], give = (jl & 2) ? a[2 * k] : a[2 * k + 1];
+    b[k] = keep + md_dpp<MD_DPP_XOR2>(give);
+  }
+  const float keep = (jl & 4) ? b[1] : b[0], give = (jl & 4) ? b[0] : b[1];
+  return keep + md_dpp_xor4(give);
+}
+
 // gap between boxes [ilo, ihi] and [jlo, jhi] on one axis, in frame units
 // (exact integer differences for boxes within 32 nm of each other)
 __device__ __forceinline__ float md_box_gap(int ilo, int ihi, int jlo, int jhi) {
@@ -1098,157 +1150,174 @@ __device__ __forceinline__ float md_box_gap(int ilo, int ihi, int jlo, int jhi) 
   return (float)max(0, max(a, b));
 }
 
-// One segment: consecutive list entries of super-cluster S against their j
+// The list records of one entry of a unit, in the lanes of its entry.
+struct md_unit_record {
+  int j, meta, x, y, z;  // the j-cluster, the meta word, J's frame origin in S's frame
+};
+__device__ __forceinline__ md_unit_record md_load_unit(const md_pair_args &A, int u, int ee, int il) {
+  const int e = min(u + il, ee - 1);
+  const int4 sh = A.entry_shift[e];
+  return md_unit_record{A.entry_j[e], A.entry_imask[e], sh.x, sh.y, sh.z};
+}
+// An entry's j atom of this lane, and the exclusion mask of S's cluster jl
+// against J (all ones for a clean entry, whose mask record is not read).
+struct md_j_record {
+  int4 p;
+  float2 lj;
+  int mask_lo, mask_hi;
+};
+__device__ __forceinline__ md_j_record md_load_j(const md_pair_args &A, int e, int J, int meta, int jl) {
+  md_j_record r{A.slot_xyzq[J * MD_CLUSTER + jl], A.slot_lj[J * MD_CLUSTER + jl], -1, -1};
+  if (!(meta & MD_META_CLEAN)) {
+    const int2 m = reinterpret_cast<const int2 *>(A.entry_excl)[(size_t)e * 8 + jl];
+    r.mask_lo = m.x;
+    r.mask_hi = m.y;
+  }
+  return r;
+}
+
+// One stretch: consecutive list entries of super-cluster S against their j
 // clusters, in units of MD_SEGMENT entries counted from S's first entry.  The
 // i forces and the energy are summed in f32 over one unit and rounded to
-// Q32.32 at its end, then summed as integers over the segment and added once:
-// the rounding never depends on the segment length, so every launch group
-// gives the same bits whatever length it picked.
+// Q32.32 at its end, then summed as integers over the stretch and added once:
+// the rounding never depends on how the entries are shared out, so every
+// launch gives the same bits.
+//
+// Bound by VALU issue: about 46 slots per block with a counted pair (12 for
+// its distances and ballot) and 45 per entry around its blocks, at four
+// cycles a slot, take nine tenths of its time on 64 replicas.  Hence the
+// reductions that share lanes (md_sum_same_j3, md_sum_i_transposed), the
+// eight entries' box tests in one pass, parameters stored scaled: 834 -> 788
+// us there.
 template <bool ENERGY, bool FIT>
-__device__ __forceinline__ void md_pair_segment(const md_pair_args &A, int seg, int lane, int il, int jl,
-                                                int64_t &efix, int &count, int &blocks) {
-  const int4 sg = md_uniform_xyz(A.segments + seg);
-  // wave-uniform by construction; readfirstlane tells the compiler, so the
-  // entry loop runs on scalar registers and its loads are scalar loads
-  const int S = __builtin_amdgcn_readfirstlane(sg.x), eb = __builtin_amdgcn_readfirstlane(sg.y),
-            ee = __builtin_amdgcn_readfirstlane(sg.z);
+__device__ __forceinline__ void md_pair_segment(const md_pair_args &A, int S, int eb, int ee, int lane, int il, int jl,
+                                                float4 *ipar, int64_t &efix, int &count, int &blocks) {
   // i data: lane's atom in each of S's 8 clusters (8 clusters x 8 atoms = 64
   // slots; lane il*8+jl reads slot S*64 + q*8 + il)
   int xi[8], yi[8], zi[8];
-  float qi[8], si[8], ei[8];
   float fx[8], fy[8], fz[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     int slot = S * MD_SUPER + q * MD_CLUSTER + il;
     int4 p = A.slot_xyzq[slot];
-    float2 lj = A.slot_lj[slot];
     xi[q] = p.x;
     yi[q] = p.y;
     zi[q] = p.z;
-    qi[q] = __int_as_float(p.w) * MD_PAIR_Q_SCALE;
-    si[q] = lj.x * MD_PAIR_S_SCALE;
-    ei[q] = lj.y * MD_PAIR_E_SCALE;
     fx[q] = fy[q] = fz[q] = 0.0f;
+  }
+  // the i atoms' scaled charge, sigma/2 and 2 sqrt(eps) sit in LDS (one read
+  // per block): 24 registers the prefetched records need at four waves per SIMD
+  {
+    const int4 p = A.slot_xyzq[S * MD_SUPER + lane];
+    const float2 lj = A.slot_lj[S * MD_SUPER + lane];
+    __syncthreads();  // one wave: orders these writes after the last stretch's reads
+    ipar[lane] = make_float4(__int_as_float(p.w), lj.x, lj.y, 0.0f);
+    __syncthreads();
   }
   float en = 0.0f;
   // lane (il, jl) keeps the i force of atom il of S's cluster q = jl
   int64_t ax = 0, ay = 0, az = 0;
-  int unit_end = min(eb + MD_SEGMENT, ee);
-  // lanes 0-7: the current box of S's cluster q = lane
-  int4 ilo = make_int4(0, 0, 0, 0), ihi = ilo;
-  if (lane < 8) {
-    ilo = A.cluster_lo[S * 8 + lane];
-    ihi = A.cluster_hi[S * 8 + lane];
-  }
+  // every lane: the current box of S's cluster q = jl
+  const int4 ilo = A.cluster_lo[S * 8 + jl], ihi = A.cluster_hi[S * 8 + jl];
   // the force polynomial's leading coefficient in a VGPR (an empty asm
   // with a VGPR operand puts it there once per segment)
   float top = A.fit_force[MD_EWALD_TERMS - 1];
   if (FIT) asm volatile("" : "+v"(top));
-  for (int e = eb; e < ee; ++e) {
-    const int J = md_uniform(A.entry_j + e);
-    const int meta = md_uniform(A.entry_imask + e);
-    const int4 sh = md_uniform_xyz(A.entry_shift + e);
+  // The records of a unit's 8 entries ride in lanes: lane (il, jl) holds entry
+  // il's, 8 copies, so one pass over the wave tests all 64 (entry, i-cluster)
+  // boxes of the unit, and an entry's words come out with v_readlane.  The
+  // next unit's records, the next entry's j atoms and exclusion masks are
+  // loaded while this entry is evaluated: a wave waits once per unit (for the
+  // boxes), not two or three times per entry, which was what bounded it.
+  md_unit_record rec = md_load_unit(A, eb, ee, il);
+  for (int u = eb; u < ee; u += MD_SEGMENT) {
+    const int n = min(MD_SEGMENT, ee - u);
+    const int J0 = __builtin_amdgcn_readlane(rec.j, 0);
+    md_j_record nxt = md_load_j(A, u, J0, __builtin_amdgcn_readlane(rec.meta, 0), jl);
     // Blocks whose current boxes lie more than the cutoff apart (by a 1e-5
     // relative margin over the f32 distance test) have no pair inside it and
-    // would add exactly zero: drop them before any pair arithmetic.  Lane q
-    // tests S's cluster q; integer box differences wrap exactly for boxes
-    // within 32 nm, and a box of padding only (inverted) may test either way,
-    // its pairs being masked.
-    int active = 0;
+    // would add exactly zero: drop them before any pair arithmetic.  Integer
+    // box differences wrap exactly for boxes within 32 nm, and a box of
+    // padding only (inverted) may test either way, its pairs being masked.
+    uint64_t near;
     {
-      const int4 jlo = md_uniform_xyz(A.cluster_lo + J), jhi = md_uniform_xyz(A.cluster_hi + J);
-      const float dx = md_box_gap(ilo.x, ihi.x, (int)((unsigned)jlo.x + (unsigned)sh.x),
-                                  (int)((unsigned)jhi.x + (unsigned)sh.x));
-      const float dy = md_box_gap(ilo.y, ihi.y, (int)((unsigned)jlo.y + (unsigned)sh.y),
-                                  (int)((unsigned)jhi.y + (unsigned)sh.y));
-      const float dz = md_box_gap(ilo.z, ihi.z, (int)((unsigned)jlo.z + (unsigned)sh.z),
-                                  (int)((unsigned)jhi.z + (unsigned)sh.z));
-      const bool near = lane < 8 && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < A.prune2;  // frame units^2
-      active = meta & (int)(__ballot(near) & 0xffu);
+      const int4 jlo = A.cluster_lo[rec.j], jhi = A.cluster_hi[rec.j];
+      const float dx = md_box_gap(ilo.x, ihi.x, (int)((unsigned)jlo.x + (unsigned)rec.x),
+                                  (int)((unsigned)jhi.x + (unsigned)rec.x));
+      const float dy = md_box_gap(ilo.y, ihi.y, (int)((unsigned)jlo.y + (unsigned)rec.y),
+                                  (int)((unsigned)jhi.y + (unsigned)rec.y));
+      const float dz = md_box_gap(ilo.z, ihi.z, (int)((unsigned)jlo.z + (unsigned)rec.z),
+                                  (int)((unsigned)jhi.z + (unsigned)rec.z));
+      near = __ballot(il < n && ((rec.meta >> jl) & 1) &&
+                      fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < A.prune2);  // frame units^2
     }
-    if (ENERGY) blocks += __popc(active);
-    float gx = 0.0f, gy = 0.0f, gz = 0.0f;
-    if (active) {
-      const int4 pj = A.slot_xyzq[J * MD_CLUSTER + jl];
-      const float2 lj = A.slot_lj[J * MD_CLUSTER + jl];
-      const float qj = __int_as_float(pj.w) * MD_PAIR_Q_SCALE, sj = lj.x * MD_PAIR_S_SCALE,
-                  ej = lj.y * MD_PAIR_E_SCALE;
-      // wrapping (unsigned) integer arithmetic: exact for every real pair; the
-      // padding slots far out may wrap, and their pairs are masked
-      unsigned xj = (unsigned)pj.x + (unsigned)sh.x, yj = (unsigned)pj.y + (unsigned)sh.y,
-               zj = (unsigned)pj.z + (unsigned)sh.z;
-      const uint64_t *ex = A.entry_excl + (size_t)e * 8;
+    for (int k = 0; k < n; ++k) {
+      const int active = (int)(near >> (8 * k)) & 0xff;
+      const md_j_record jr = nxt;
+      const bool clean = (__builtin_amdgcn_readlane(rec.meta, 8 * k) & MD_META_CLEAN) != 0;
+      const unsigned ox = (unsigned)__builtin_amdgcn_readlane(rec.x, 8 * k),
+                     oy = (unsigned)__builtin_amdgcn_readlane(rec.y, 8 * k),
+                     oz = (unsigned)__builtin_amdgcn_readlane(rec.z, 8 * k);
+      if (k + 1 < n)
+        nxt = md_load_j(A, u + k + 1, __builtin_amdgcn_readlane(rec.j, 8 * (k + 1)),
+                        __builtin_amdgcn_readlane(rec.meta, 8 * (k + 1)), jl);
+      else if (u + MD_SEGMENT < ee)
+        rec = md_load_unit(A, u + MD_SEGMENT, ee, il);
+      if (ENERGY) blocks += __popc(active);
+      float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+      if (active) {
+        const float qj = __int_as_float(jr.p.w), sj = jr.lj.x, ej = jr.lj.y;
+        // wrapping (unsigned) integer arithmetic: exact for every real pair; the
+        // padding slots far out may wrap, and their pairs are masked
+        const unsigned xj = (unsigned)jr.p.x + ox, yj = (unsigned)jr.p.y + oy, zj = (unsigned)jr.p.z + oz;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        if ((active >> q) & 1) {
-          // bit l of the mask allows lane l's pair: with the in-cutoff ballot
-          // it is the block's lane mask of counted pairs
-          const uint64_t allowed = (meta & MD_META_CLEAN) ? ~0ull : md_uniform(ex + q);
-          float dx = (float)(int)(xj - (unsigned)xi[q]), dy = (float)(int)(yj - (unsigned)yi[q]),
-                dz = (float)(int)(zj - (unsigned)zi[q]);
-          float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-          const uint64_t inc = allowed & __ballot(r2 < A.cutoff2);
-          // a block whose 64 pairs all lie beyond the cutoff (or are masked)
-          // adds exactly zero: skip its arithmetic, wave-uniformly
-          if (inc == 0) continue;
-          const bool counted = __builtin_amdgcn_inverse_ballot_w64(inc);
-          float fs = md_pair<ENERGY, FIT>(r2, qi[q], si[q], ei[q], qj, sj, ej, counted, top, A, en, count);
-          // the other lanes' fs is not a force: a divergent branch (the
-          // exec mask, scalar instructions) leaves them out without a select
-          if (counted) {
-            fx[q] = fmaf(-fs, dx, fx[q]);
-            fy[q] = fmaf(-fs, dy, fy[q]);
-            fz[q] = fmaf(-fs, dz, fz[q]);
-            gx = fmaf(fs, dx, gx);
-            gy = fmaf(fs, dy, gy);
-            gz = fmaf(fs, dz, gz);
+        for (int q = 0; q < 8; ++q) {
+          if ((active >> q) & 1) {
+            // bit l of the mask allows lane l's pair: with the in-cutoff ballot
+            // it is the block's lane mask of counted pairs
+            uint64_t allowed = ~0ull;
+            if (!clean)
+              allowed = (uint64_t)(unsigned)__builtin_amdgcn_readlane(jr.mask_lo, q) |
+                        (uint64_t)(unsigned)__builtin_amdgcn_readlane(jr.mask_hi, q) << 32;
+            float dx = (float)(int)(xj - (unsigned)xi[q]), dy = (float)(int)(yj - (unsigned)yi[q]),
+                  dz = (float)(int)(zj - (unsigned)zi[q]);
+            float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            const uint64_t inc = allowed & __ballot(r2 < A.cutoff2);
+            // a block whose 64 pairs all lie beyond the cutoff (or are masked)
+            // adds exactly zero: skip its arithmetic, wave-uniformly
+            if (inc == 0) continue;
+            const bool counted = __builtin_amdgcn_inverse_ballot_w64(inc);
+            const float4 pi = ipar[q * MD_CLUSTER + il];
+            float fs = md_pair<ENERGY, FIT>(r2, pi.x, pi.y, pi.z, qj, sj, ej, counted, top, A, en, count);
+            // the other lanes' fs is not a force: a divergent branch (the
+            // exec mask, scalar instructions) leaves them out without a select
+            if (counted) {
+              fx[q] = fmaf(-fs, dx, fx[q]);
+              fy[q] = fmaf(-fs, dy, fy[q]);
+              fz[q] = fmaf(-fs, dz, fz[q]);
+              gx = fmaf(fs, dx, gx);
+              gy = fmaf(fs, dy, gy);
+              gz = fmaf(fs, dz, gz);
+            }
           }
         }
+        gx = md_sum_same_j3(gx, gy, gz, lane);
       }
-      // j force: sum the 8 lanes that share j (lane%8), fixed order
-      gx = md_sum_same_j(gx);
-      gy = md_sum_same_j(gy);
-      gz = md_sum_same_j(gz);
+      // lanes 0-23 hold component lane/8 of j atom lane%8: one 96-byte record,
+      // j-major, so the slot thread that adds j's share reads 12 contiguous bytes
+      if (lane < 24) A.j_force[(size_t)(u + k) * 24 + (lane & 7) * 3 + (lane >> 3)] = gx;
     }
-    // lanes 0-7 hold (x, y, z) of j atoms 0-7: one 96-byte record, j-major,
-    // so the slot thread that adds j's share reads 12 contiguous bytes
-    if (lane < 8) {
-      float *r = A.j_force + (size_t)e * 24 + lane * 3;
-      r[0] = gx;
-      r[1] = gy;
-      r[2] = gz;
-    }
-    if (e + 1 == unit_end) {  // wave-uniform: the end of a unit
-      // i forces: sum the 8 lanes that share i (same il), fixed order; lane
-      // jl keeps q = jl's sum
-      float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+    // the unit's i forces: over the 8 lanes that share i (same il), lane jl
+    // keeping q = jl's sum
+    const float sx = md_sum_i_transposed(fx, jl), sy = md_sum_i_transposed(fy, jl), sz = md_sum_i_transposed(fz, jl);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        float x, y, z;
-        if (q < 4) {
-          x = md_sum_same_i<false>(fx[q]);
-          y = md_sum_same_i<false>(fy[q]);
-          z = md_sum_same_i<false>(fz[q]);
-        } else {
-          x = md_sum_same_i<true>(fx[q]);
-          y = md_sum_same_i<true>(fy[q]);
-          z = md_sum_same_i<true>(fz[q]);
-        }
-        if (jl == q) {
-          sx = x;
-          sy = y;
-          sz = z;
-        }
-        fx[q] = fy[q] = fz[q] = 0.0f;
-      }
-      ax += md_to_fixed(sx);
-      ay += md_to_fixed(sy);
-      az += md_to_fixed(sz);
-      if (ENERGY) {
-        efix += md_to_fixed(en * MD_FRAME_UNIT);  // the energy carried 2^26
-        en = 0.0f;
-      }
-      unit_end = min(unit_end + MD_SEGMENT, ee);
+    for (int q = 0; q < 8; ++q) fx[q] = fy[q] = fz[q] = 0.0f;
+    ax += md_to_fixed(sx);
+    ay += md_to_fixed(sy);
+    az += md_to_fixed(sz);
+    if (ENERGY) {
+      efix += md_to_fixed(en * MD_FRAME_UNIT);  // the energy carried 2^26
+      en = 0.0f;
     }
   }
   // 64 consecutive slots: S's cluster jl, atom il
@@ -1288,11 +1357,8 @@ struct md_pair_lds {
   float fs[MD_COMPACT_BATCH][512];               // the pair's force factor at (entry, block, lane)
 };
 
-__device__ __forceinline__ void md_pair_segment_compact(const md_pair_args &A, int seg, int lane, int il, int jl,
-                                                        md_pair_lds &L) {
-  const int4 sg = md_uniform_xyz(A.segments + seg);
-  const int S = __builtin_amdgcn_readfirstlane(sg.x), eb = __builtin_amdgcn_readfirstlane(sg.y),
-            ee = __builtin_amdgcn_readfirstlane(sg.z);
+__device__ __forceinline__ void md_pair_segment_compact(const md_pair_args &A, int S, int eb, int ee, int lane, int il,
+                                                        int jl, md_pair_lds &L) {
   int xi[8], yi[8], zi[8];
   float fx[8], fy[8], fz[8];
 #pragma unroll
@@ -1307,8 +1373,8 @@ __device__ __forceinline__ void md_pair_segment_compact(const md_pair_args &A, i
     // the i table: lane l holds slot S*64 + l (block l/8, atom l%8)
     const int4 p = A.slot_xyzq[S * MD_SUPER + lane];
     const float2 lj = A.slot_lj[S * MD_SUPER + lane];
-    L.ixyz[lane] = make_int4(p.x, p.y, p.z, __float_as_int(__int_as_float(p.w) * MD_PAIR_Q_SCALE));
-    L.ise[lane] = make_float2(lj.x * MD_PAIR_S_SCALE, lj.y * MD_PAIR_E_SCALE);
+    L.ixyz[lane] = p;
+    L.ise[lane] = lj;
   }
   int64_t ax = 0, ay = 0, az = 0;
   int unit_end = min(eb + MD_SEGMENT, ee);
@@ -1353,9 +1419,8 @@ __device__ __forceinline__ void md_pair_segment_compact(const md_pair_args &A, i
       zj[b] = (unsigned)pj.z + (unsigned)sh.z;
       if (lane < MD_CLUSTER) {  // lanes 0-7 hold j atoms 0-7
         const float2 lj = A.slot_lj[J * MD_CLUSTER + jl];
-        L.jxyz[b][jl] = make_int4((int)xj[b], (int)yj[b], (int)zj[b],
-                                  __float_as_int(__int_as_float(pj.w) * MD_PAIR_Q_SCALE));
-        L.jse[b][jl] = make_float2(lj.x * MD_PAIR_S_SCALE, lj.y * MD_PAIR_E_SCALE);
+        L.jxyz[b][jl] = make_int4((int)xj[b], (int)yj[b], (int)zj[b], pj.w);
+        L.jse[b][jl] = lj;
       }
       const uint64_t *ex = A.entry_excl + (size_t)e * 8;
 #pragma unroll
@@ -1469,60 +1534,59 @@ __device__ __forceinline__ void md_pair_segment_compact(const md_pair_args &A, i
   md_atomic_add_i64(&A.slot_force[2 * A.nslots + is], az);
 }
 
-// The pair kernels' work queue.  The segments, numbered replica by replica
-// and in list (Hilbert) order within each, are cut into MD_XCDS contiguous
-// ranges with a counter each (one 64-byte line apart).  A workgroup takes
-// segments from the range of the XCD it runs on first -- the dispatcher deals
-// workgroups to the XCDs in turn, workgroup b to XCD b mod 8 -- then from the
-// following ranges once that one is empty.  Each XCD's waves thus walk one
-// neighbourhood of the list at a time and its L2 keeps that neighbourhood's
-// j clusters, instead of all eight L2s fetching every cluster.  Which wave
-// takes which segment never changes a result (each segment's sums are
-// rounded to Q32.32 on their own).
+// The pair kernels' share of the work.  The segments, numbered replica by
+// replica and in list (Hilbert) order within each, are cut into MD_XCDS
+// contiguous ranges, one per XCD (the dispatcher deals workgroup b to XCD b
+// mod 8), and each range into equal contiguous runs, one per wave: an XCD's
+// waves walk one neighbourhood of the list and its L2 keeps that
+// neighbourhood's j clusters, and a wave keeps its i atoms and i forces in
+// registers across all segments of a super-cluster in its run.
 //
-// Every lane joins the atomic (lane 0 adds 1, the others 0) and readfirstlane
-// makes the index wave-uniform, so the exits are scalar branches.  A
-// lane-0-only atomic followed by a broadcast is not safe here: the optimiser
-// threads the per-segment `lane == 0` energy flush into the next `lane == 0`
-// atomic, after which lanes 1-63 loop back to the broadcast without lane 0
-// and never leave.  The counters only grow and a wave leaves a range at its
-// first index past the end, so every wave leaves.
-struct md_seg_queue {
-  int *cursor;
-  int nseg, home, range, lo, hi, lane;
-  __device__ md_seg_queue(int *c, int n, int l) : cursor(c), nseg(n), home((int)(blockIdx.x & (MD_XCDS - 1))),
-                                                  range(0), lane(l) {
-    bounds();
+// A launch has up to MD_PAIR_WAVES waves, eight times what is resident, so
+// the dispatcher evens out what the runs differ by (4,096 waves: 862 us on 64
+// replicas, 32,768: 788); a small list has a wave per segment.  No counter is
+// drawn from: a shared counter is one word at memory, each draw takes about
+// 20 ns of it, and with one counter per XCD drawn to exhaustion by every wave
+// the queue alone cost about 100 us a launch whatever the list (k_nb_pairs
+// with the counters and as it is: 2,168 atoms 100 -> 17 us, 31k 161 -> 60,
+// 243k 424 -> 310, 64 replicas of 2k-30k atoms 912 -> 788).
+struct md_seg_run {
+  int at, end;
+  __device__ explicit md_seg_run(int nseg) {
+    const int k = (int)(blockIdx.x & (MD_XCDS - 1)), w = (int)(blockIdx.x / MD_XCDS);
+    const int lo = (int)(((int64_t)nseg * k) / MD_XCDS), hi = (int)(((int64_t)nseg * (k + 1)) / MD_XCDS);
+    const int waves = ((int)gridDim.x + MD_XCDS - 1 - k) / MD_XCDS;  // workgroups of this XCD
+    at = lo + (int)((int64_t)(hi - lo) * w / waves);
+    end = lo + (int)((int64_t)(hi - lo) * (w + 1) / waves);
   }
-  __device__ void bounds() {
-    const int c = (home + range) & (MD_XCDS - 1);
-    lo = (int)(((int64_t)nseg * c) / MD_XCDS);
-    hi = (int)(((int64_t)nseg * (c + 1)) / MD_XCDS);
-  }
-  __device__ bool next(int &g) {
-    while (range < MD_XCDS) {
-      const int c = (home + range) & (MD_XCDS - 1);
-      g = lo + __builtin_amdgcn_readfirstlane(atomicAdd(cursor + c * MD_CURSOR_STRIDE, lane == 0 ? 1 : 0));
-      if (g < hi) return true;
-      if (++range < MD_XCDS) bounds();
-    }
-    return false;
+  // The next stretch of list entries of one super-cluster: S and [eb, ee) in
+  // replica r's list; false when the run is done.
+  __device__ bool next(const md_nb_args *T, const md_bmap &map, int &r, int &S, int &eb, int &ee) {
+    if (at >= end) return false;
+    int seg;
+    r = __builtin_amdgcn_readfirstlane(md_locate(map, at, seg));
+    const md_nb_args &A = T[r];
+    const int4 first = md_uniform_xyz(A.P.segments + seg);
+    S = __builtin_amdgcn_readfirstlane(first.x);
+    eb = __builtin_amdgcn_readfirstlane(first.y);
+    // S's segments are numbered up to the next super-cluster's first
+    const int stop = min(min(A.L.super_segs[S + 1], A.P.totals[1]), seg + end - at);
+    ee = __builtin_amdgcn_readfirstlane(md_uniform_xyz(A.P.segments + stop - 1).z);
+    at += __builtin_amdgcn_readfirstlane(stop) - seg;
+    return true;
   }
 };
 
 // The compacted schedule's kernel (forces only; energies use the direct one).
 template <bool BATCH>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_nb_pairs_compact(const md_nb_args *__restrict__ T, md_bmap seg_map, int *cursor) {
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_nb_pairs_compact(const md_nb_args *__restrict__ T, md_bmap seg_map) {
   __shared__ md_pair_lds L;
-  const int nseg = seg_map.start[seg_map.R];
   const int lane = threadIdx.x, il = lane >> 3, jl = lane & 7;
-  md_seg_queue Q(cursor, nseg, lane);
-  int g;
-  while (Q.next(g)) {
-    int seg;
-    const md_pair_args &A = T[md_locate(seg_map, g, seg)].P;
-    md_pair_segment_compact(A, seg, lane, il, jl, L);
-    __syncthreads();  // the next segment rewrites the i table
+  md_seg_run Q(seg_map.start[seg_map.R]);
+  int r, S, eb, ee;
+  while (Q.next(T, seg_map, r, S, eb, ee)) {
+    md_pair_segment_compact(T[r].P, S, eb, ee, lane, il, jl, L);
+    __syncthreads();  // the next super-cluster rewrites the i table
   }
 }
 
@@ -1530,31 +1594,29 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
 // k_nb_pairs<·, true>, one replica <·, false>, the same code, so a kernel
 // trace reports the batched launches on their own.
 template <bool ENERGY, bool BATCH = false>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_nb_pairs(const md_nb_args *__restrict__ T, md_bmap seg_map, int *cursor) {
-  const int nseg = seg_map.start[seg_map.R];
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ENERGY ? 3 : 4))) k_nb_pairs(const md_nb_args *__restrict__ T, md_bmap seg_map) {
+  __shared__ float4 ipar[MD_SUPER];
   const int lane = threadIdx.x, il = lane >> 3, jl = lane & 7;
-  // A resident grid of waves takes segments from the queue until none are
-  // left, across every replica's list.  Each segment's energy is rounded to
-  // Q32.32 and added on its own, so the sums do not depend on which wave took
-  // which segment.
-  md_seg_queue Q(cursor, nseg, lane);
-  int g;
-  while (Q.next(g)) {
-    int seg;
-    const md_pair_args &A = T[md_locate(seg_map, g, seg)].P;
+  // Each unit's energy is rounded to Q32.32 on its own, so the sums do not
+  // depend on which wave took which entries.
+  md_seg_run Q(seg_map.start[seg_map.R]);
+  int r, S, eb, ee;
+  while (Q.next(T, seg_map, r, S, eb, ee)) {
+    const md_pair_args &A = T[r].P;
     int64_t efix = 0;
     int count = 0, blocks = 0;
     if (A.ewald_fit)
-      md_pair_segment<ENERGY, true>(A, seg, lane, il, jl, efix, count, blocks);
+      md_pair_segment<ENERGY, true>(A, S, eb, ee, lane, il, jl, ipar, efix, count, blocks);
     else
-      md_pair_segment<ENERGY, false>(A, seg, lane, il, jl, efix, count, blocks);
+      md_pair_segment<ENERGY, false>(A, S, eb, ee, lane, il, jl, ipar, efix, count, blocks);
     if (ENERGY) {
       int64_t ef = md_wave_sum_i64(efix);
       int64_t cf = md_wave_sum_i64((int64_t)count);
       if (lane == 0) {
-        md_atomic_add_i64(A.energy + MD_E_PAIR, ef);
-        md_atomic_add_i64(A.census, cf);
-        md_atomic_add_i64(A.blocks, (int64_t)blocks);  // blocks is wave-uniform
+        int64_t *part = A.part + (blockIdx.x % MD_ENERGY_PARTS) * MD_ENERGY_STRIDE;
+        md_atomic_add_i64(part, ef);
+        md_atomic_add_i64(part + 1, cf);
+        md_atomic_add_i64(part + 2, (int64_t)blocks);  // blocks is wave-uniform
       }
     }
   }
@@ -1654,6 +1716,7 @@ struct md_nb_buffers {
   float *j_force = nullptr;
   int4 *cluster_lo = nullptr, *cluster_hi = nullptr;
   int *totals = nullptr;
+  int64_t *energy_part = nullptr;
   int nsuper = 0;
   int entry_capacity = 0, segment_capacity = 0, entries_per_super = 0;
   float half_min_width = 0, list_cutoff = 0;
@@ -1828,6 +1891,7 @@ void md_nb_setup(md_system *s) {
   B.super_count = md_alloc<int>(s, B.nsuper);
   B.super_segs = md_alloc<int>(s, B.nsuper + 1);
   B.totals = md_alloc<int>(s, 4);
+  B.energy_part = md_alloc<int64_t>(s, MD_ENERGY_PARTS * MD_ENERGY_STRIDE);
   // list capacity: the cluster pairs within the list radius plus the cluster
   // extents at the system's density, doubled for headroom
   double volume = std::fabs(s->box[0] * s->box[4] * s->box[8]);
@@ -1960,6 +2024,7 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   P.slot_lj = s->slot_lj;
   P.totals = B.totals;
   P.slot_force = B.slot_force;
+  P.part = B.energy_part;
   P.energy = s->energy;
   P.census = &s->ctl->pair_census;
   P.blocks = &s->ctl->pair_blocks;
@@ -2012,8 +2077,7 @@ struct md_nb_group {
   md_nb_args *table = nullptr;  // [R], device
   md_launch atoms, scan, clusters, supers, segments, masks, slots;
   md_launch seg;                // the pair kernel's segment numbering
-  int *cursor = nullptr;
-  int pair_grid[2] = {1, 1};
+  int pair_grid = 1;
   int seg_len = MD_SEGMENT;
   bool compact = false;  // forces through the compacted schedule
 };
@@ -2044,25 +2108,12 @@ void md_nb_group_setup(md_group *g) {
   G->slots = md_make_launch(g, slots);
   G->seg.map.start = md_group_alloc<int>(g, R + 1);
   G->seg.map.R = R;
-  G->cursor = md_group_alloc<int>(g, MD_XCDS * MD_CURSOR_STRIDE);
   G->table = md_group_alloc<md_nb_args>(g, R);
-  // the pair kernel keeps one resident grid busy from the segment counter
-  int cus = 1, per_cu[2] = {1, 1};
-  MD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
-  MD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[0], k_nb_pairs<false>, 64, 0));
-  MD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[1], k_nb_pairs<true>, 64, 0));
-  long capacity = 0;
-  for (md_system *s : g->reps) capacity += nbuf(s).segment_capacity;
-  for (int k = 0; k < 2; ++k)
-    G->pair_grid[k] = (int)std::max(1L, std::min(capacity, (long)std::max(1, cus) * std::max(1, per_cu[k])));
-  // Longer segments flush each i-force once per more entries (the flushes
-  // are half of the kernel's 64-bit atomics at 8 entries), but leave fewer
-  // units to share among the resident waves: double the length while at
-  // least 8 units per wave remain, at about 180 entries per super-cluster.
-  double entries = 0.0;
-  for (md_system *s : g->reps) entries += 180.0 * nbuf(s).nsuper;
-  const double waves = (double)G->pair_grid[0];
-  while (G->seg_len < 4 * MD_SEGMENT && entries / (2.0 * G->seg_len) >= 8.0 * waves) G->seg_len *= 2;
+  // The pair kernel's waves: one per segment of about 200 entries per
+  // super-cluster, at most MD_PAIR_WAVES
+  long units = 0;
+  for (md_system *s : g->reps) units += (long)nbuf(s).nsuper * (200 / MD_SEGMENT);
+  G->pair_grid = (int)std::min<long>(MD_PAIR_WAVES, std::max<long>(MD_XCDS, units));
   md_nb_group_refresh(g);
 }
 
@@ -2075,13 +2126,13 @@ void md_nb_set_schedule(md_group *g, int seg_len, int waves) {
   if (seg_len % MD_SEGMENT || seg_len < MD_SEGMENT || seg_len > 32 * MD_SEGMENT)
     throw md_error(MD_ERR_INVALID_ARGUMENT, "segment length must be a multiple of 8 entries, at most 256");
   G.seg_len = seg_len;
-  if (waves > 0) G.pair_grid[0] = waves;
+  if (waves > 0) G.pair_grid = waves;
   md_nb_group_refresh(g);
 }
 
 void md_nb_get_schedule(md_group *g, int *seg_len, int *waves) {
   *seg_len = nbg(g).seg_len;
-  *waves = nbg(g).pair_grid[0];
+  *waves = nbg(g).pair_grid;
 }
 
 void md_nb_set_compact(md_group *g, bool compact) { nbg(g).compact = compact; }
@@ -2137,27 +2188,27 @@ void md_nb_build(md_group *g) {
 void md_nb_pairs(md_group *g, bool energy) {
   auto &G = nbg(g);
   hipStream_t st = g->stream;
-  k_nb_pack<<<G.slots.total, 256, 0, st>>>(G.table, G.slots.map, const_cast<int *>(G.seg.map.start), G.cursor);
+  k_nb_pack<<<G.slots.total, 256, 0, st>>>(G.table, G.slots.map, const_cast<int *>(G.seg.map.start));
   md_mark(g, MD_PHASE_PAIRS);
   const bool batch = g->reps.size() > 1;
   if (energy) {
     if (batch)
-      k_nb_pairs<true, true><<<G.pair_grid[1], 64, 0, st>>>(G.table, G.seg.map, G.cursor);
+      k_nb_pairs<true, true><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
     else
-      k_nb_pairs<true, false><<<G.pair_grid[1], 64, 0, st>>>(G.table, G.seg.map, G.cursor);
+      k_nb_pairs<true, false><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
   } else if (G.compact) {
     if (batch)
-      k_nb_pairs_compact<true><<<G.pair_grid[0], 64, 0, st>>>(G.table, G.seg.map, G.cursor);
+      k_nb_pairs_compact<true><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
     else
-      k_nb_pairs_compact<false><<<G.pair_grid[0], 64, 0, st>>>(G.table, G.seg.map, G.cursor);
+      k_nb_pairs_compact<false><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
   } else {
     if (batch)
-      k_nb_pairs<false, true><<<G.pair_grid[0], 64, 0, st>>>(G.table, G.seg.map, G.cursor);
+      k_nb_pairs<false, true><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
     else
-      k_nb_pairs<false, false><<<G.pair_grid[0], 64, 0, st>>>(G.table, G.seg.map, G.cursor);
+      k_nb_pairs<false, false><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
   }
   md_mark(g, MD_PHASE_FORCES);
-  k_nb_forces<<<G.slots.total, 256, 0, st>>>(G.table, G.slots.map);
+  k_nb_forces<<<G.slots.total, 256, 0, st>>>(G.table, G.slots.map, energy ? 1 : 0);
   MD_HIP(hipGetLastError());
 }
 
