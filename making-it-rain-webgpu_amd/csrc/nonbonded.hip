@@ -1553,9 +1553,10 @@ __device__ __forceinline__ void md_pair_segment_compact(const md_pair_args &A, i
 struct md_seg_run {
   int at, end;
   __device__ explicit md_seg_run(int nseg) {
-    const int k = (int)(blockIdx.x & (MD_XCDS - 1)), w = (int)(blockIdx.x / MD_XCDS);
-    const int lo = (int)(((int64_t)nseg * k) / MD_XCDS), hi = (int)(((int64_t)nseg * (k + 1)) / MD_XCDS);
-    const int waves = ((int)gridDim.x + MD_XCDS - 1 - k) / MD_XCDS;  // workgroups of this XCD
+    const int ranges = min(MD_XCDS, (int)gridDim.x);  // every range has a wave
+    const int k = (int)blockIdx.x % ranges, w = (int)blockIdx.x / ranges;
+    const int lo = (int)(((int64_t)nseg * k) / ranges), hi = (int)(((int64_t)nseg * (k + 1)) / ranges);
+    const int waves = ((int)gridDim.x + ranges - 1 - k) / ranges;  // workgroups of this range
     at = lo + (int)((int64_t)(hi - lo) * w / waves);
     end = lo + (int)((int64_t)(hi - lo) * (w + 1) / waves);
   }
