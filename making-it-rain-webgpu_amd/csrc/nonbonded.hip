@@ -83,22 +83,17 @@ struct md_build_ctx {
 #define MD_MAX_IMAGE_SHELLS 4
 // candidate j super-clusters a list wave keeps in LDS (beyond: scan all)
 #define MD_LIST_CANDIDATES 1024
-// wavefronts that share one super-cluster's entries in the mask kernel, and
-// wavefronts per workgroup (a replica that did not rebuild dispatches
-// MD_MASK_WAVES / MD_MASK_GROUP workgroups per super-cluster that return at once)
-#define MD_MASK_WAVES 16
 // entry meta word: bits 0-7 the i-clusters of S that meet J, bits 8-15 those
 // that are J itself at the zero image, and MD_META_CLEAN when no active block
 // has an excluded, padding or lower-triangle pair (its masks are all ones and
 // the pair kernel does not read them)
 #define MD_META_CLEAN (1 << 16)
-#define MD_MASK_GROUP 4
 
 struct md_list_ptrs {
   const int64_t *cluster_center;
   const float4 *cluster_half;
   const int64_t *super_origin;
-  const float *super_radius;  // half diagonal of each super-cluster's bounding box (nm)
+  const float4 *super_sphere;  // each super-cluster's origin (f32) and half diagonal (nm)
   int *super_count;   // [nsuper] entries per super-cluster (in its region)
   int *super_segs;    // [nsuper+1] segments per super-cluster, then starts
   int *entry_j;
@@ -163,13 +158,12 @@ struct md_nb_args {
   int *cell_count, *cell_start, *cell_cursor, *atom_cell, *cell_member;
   int *slot_atom, *atom_slot;
   int64_t *folded, *build_pos, *slot_offset, *cluster_center, *super_origin;
-  float *super_radius;
+  float4 *super_sphere;
   float2 *slot_lj;
   int4 *slot_xyzq;
   float4 *cluster_half;
   const float4 *atom_param;
   const int *excl_start, *excl_list;
-  const uint64_t *excl_window;
   int64_t *force;  // the atoms' Q32.32 forces, [3][np]
   int4 *cluster_lo, *cluster_hi;
   int *totals;
@@ -247,29 +241,47 @@ __global__ void k_nb_assign(const md_nb_args *__restrict__ T, md_bmap map) {
 
 // Exclusive scan by one workgroup of 1024 threads over `count` values; the
 // total lands at out[count].  `in` may alias `out`.  Zeroes `clear` if given.
+// A pass takes MD_SCAN_ITEMS consecutive values per thread, scanned by wave
+// shuffles and once across the 16 waves, so a long scan is a few passes over
+// contiguous memory (85k cells: 157 us with one long run of values per thread,
+// 88 us so).
+#define MD_SCAN_ITEMS 8
 __device__ void md_block_scan(const int *in, int *out, int count, int *clear) {
-  __shared__ int partial[1024];
-  int t = threadIdx.x;
-  int per = (count + 1023) / 1024;
-  int begin = min(t * per, count), end = min(begin + per, count);
-  int sum = 0;
-  for (int k = begin; k < end; ++k) sum += in[k];
-  partial[t] = sum;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    int v = t >= off ? partial[t - off] : 0;
+  __shared__ int wave_sum[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int carry = 0;
+  for (int base = 0; base < count; base += 1024 * MD_SCAN_ITEMS) {
+    const int at = base + t * MD_SCAN_ITEMS;
+    int v[MD_SCAN_ITEMS], sum = 0;
+#pragma unroll
+    for (int k = 0; k < MD_SCAN_ITEMS; ++k) v[k] = at + k < count ? in[at + k] : 0;
+#pragma unroll
+    for (int k = 0; k < MD_SCAN_ITEMS; ++k) sum += v[k];
+    int incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int u = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += u;
+    }
+    if (lane == 63) wave_sum[wave] = incl;
     __syncthreads();
-    partial[t] += v;
-    __syncthreads();
+    int before = carry, total = 0;
+    for (int w = 0; w < 16; ++w) {
+      const int u = wave_sum[w];
+      if (w < wave) before += u;
+      total += u;
+    }
+    int run = before + incl - sum;
+#pragma unroll
+    for (int k = 0; k < MD_SCAN_ITEMS; ++k) {
+      if (at + k >= count) break;
+      out[at + k] = run;
+      run += v[k];
+      if (clear) clear[at + k] = 0;
+    }
+    carry += total;
+    __syncthreads();  // the next pass rewrites wave_sum
   }
-  int run = partial[t] - sum;
-  for (int k = begin; k < end; ++k) {
-    int v = in[k];
-    out[k] = run;
-    run += v;
-    if (clear) clear[k] = 0;
-  }
-  if (t == 1023) out[count] = partial[1023];
+  if (t == 0) out[count] = carry;
 }
 
 // one workgroup per replica
@@ -334,7 +346,7 @@ __global__ void k_nb_clusters(const md_nb_args *__restrict__ T, md_bmap map) {
   const int64_t *folded = A.folded, *build_pos = A.build_pos;
   const float4 *atom_param = A.atom_param;
   int64_t *cluster_center = A.cluster_center, *super_origin = A.super_origin, *slot_offset = A.slot_offset;
-  float *super_radius = A.super_radius;
+  float4 *super_sphere = A.super_sphere;
   float4 *cluster_half = A.cluster_half;
   float2 *slot_lj = A.slot_lj;
   // one thread per cluster; the 8 threads of a super-cluster cooperate
@@ -397,7 +409,7 @@ __global__ void k_nb_clusters(const md_nb_args *__restrict__ T, md_bmap map) {
     }
     // rounded up a little: the list test that uses it must stay conservative
     srad = sqrtf(r2) * 1.0001f + 1e-4f;
-    super_radius[s] = srad;
+    super_sphere[s] = make_float4(md_from_fixed(origin[0]), md_from_fixed(origin[1]), md_from_fixed(origin[2]), srad);
   }
   // the largest super-cluster radius, one atomic per wave as above
   for (int off = 32; off > 0; off >>= 1) srad = fmaxf(srad, __shfl_xor(srad, off, 64));
@@ -456,28 +468,50 @@ __device__ void md_for_each_image(const md_build_ctx &c, int64_t dx, int64_t dy,
   const int centre = (K[2] * nb + K[1]) * na + K[0];
   const float fx0 = md_from_fixed(dx), fy0 = md_from_fixed(dy), fz0 = md_from_fixed(dz);
   const float skip2 = skip * skip;
-  int code = 0;
-  for (int kc = -K[2]; kc <= K[2]; ++kc)
-    for (int kb = -K[1]; kb <= K[1]; ++kb)
-      for (int ka = -K[0]; ka <= K[0]; ++ka, ++code) {
-        const float gx = fmaf((float)kc, c.box.c[0], fmaf((float)kb, c.box.b[0], fmaf((float)ka, c.box.a[0], fx0)));
-        const float gy = fmaf((float)kc, c.box.c[1], fmaf((float)kb, c.box.b[1], fy0));
-        const float gz = fmaf((float)kc, c.box.c[2], fz0);
-        if (fmaf(gx, gx, fmaf(gy, gy, gz * gz)) >= skip2) continue;
-        int64_t ex = dx + ka * c.box.fa[0] + kb * c.box.fb[0] + kc * c.box.fc[0];
-        int64_t ey = dy + kb * c.box.fb[1] + kc * c.box.fc[1];
-        int64_t ez = dz + kc * c.box.fc[2];
-        visit(ex, ey, ez, code - centre);  // 0 = the reduced image itself
+  // Each lane walks on to its next image that is near enough, then the lanes
+  // visit together: in lockstep over the images, with a handful of lanes near
+  // at each, the wave would run the visit for nearly every one of them.
+  int ka = -K[0], kb = -K[1], kc = -K[2], code = -1;
+  for (;;) {
+    int va = 0, vb = 0, vc = 0;
+    bool hit = false;
+    while (kc <= K[2] && !hit) {
+      const float gx = fmaf((float)kc, c.box.c[0], fmaf((float)kb, c.box.b[0], fmaf((float)ka, c.box.a[0], fx0)));
+      const float gy = fmaf((float)kc, c.box.c[1], fmaf((float)kb, c.box.b[1], fy0));
+      const float gz = fmaf((float)kc, c.box.c[2], fz0);
+      hit = fmaf(gx, gx, fmaf(gy, gy, gz * gz)) < skip2;
+      va = ka;
+      vb = kb;
+      vc = kc;
+      ++code;
+      if (++ka > K[0]) {
+        ka = -K[0];
+        if (++kb > K[1]) {
+          kb = -K[1];
+          ++kc;
+        }
       }
+    }
+    if (!hit) return;
+    const int64_t ex = dx + va * c.box.fa[0] + vb * c.box.fb[0] + vc * c.box.fc[0];
+    const int64_t ey = dy + vb * c.box.fb[1] + vc * c.box.fc[1];
+    const int64_t ez = dz + vc * c.box.fc[2];
+    visit(ex, ey, ez, code - centre);  // 0 = the reduced image itself
+  }
 }
 
-// Super-cluster S as a list wave sees it: its clusters' boxes (wave-uniform,
-// indexed only by unrolled constants so they stay in registers), the frame
-// origin and the bounding-sphere radius of the whole super-cluster.
+// Super-cluster S as its list waves see it: its clusters' boxes (in LDS), the
+// frame origin and the bounding-sphere radius of the whole super-cluster.  A
+// j-cluster's image is placed exactly against the origin and rounded once to
+// f32; the box tests then run in f32 (within 1e-6 nm, by which they are
+// widened), not on int64 differences for each of the 8 boxes.
+struct md_super_boxes {
+  float4 cc[8];  // centres from the frame origin (nm)
+  float4 ch[8];  // half extents
+};
 struct md_super_view {
   int first, nlocal;
-  int64_t cx[8], cy[8], cz[8];
-  float4 ch[8];
+  const md_super_boxes *box;
   int64_t ox, oy, oz;
   float rs;
 };
@@ -507,6 +541,7 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
   float4 jh = L.cluster_half[J];
   const float reach = c.list_cutoff + V.rs + sqrtf(jh.x * jh.x + jh.y * jh.y + jh.z * jh.z) + 1e-3f;
   const float reach2 = reach * reach;
+  const float box2 = (c.list_cutoff + 1e-6f) * (c.list_cutoff + 1e-6f);
   // the image is chosen against S's origin and shared by the entry; S's own
   // clusters keep their unshifted frame (see md_for_each_image)
   int64_t dx = jx - V.ox, dy = jy - V.oy, dz = jz - V.oz;
@@ -518,17 +553,15 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
     if (ox * ox + oy * oy + oz * oz >= reach2) return;
     bool zero = shx == 0 && shy == 0 && shz == 0;
     int imask = 0, self = 0;
-#pragma unroll
+#pragma unroll 2
     for (int q = 0; q < 8; ++q) {
       int I = V.first + q;
       // within S, J >= I only; a cluster with its own images keeps one of
       // each +/- pair (J of another super-cluster comes only from one that
       // S lists, md_lists_pair)
       if (q < V.nlocal && (!own || J >= I) && !(J == I && !zero && code < 0)) {
-        float ddx = md_from_fixed(jx + shx - V.cx[q]);
-        float ddy = md_from_fixed(jy + shy - V.cy[q]);
-        float ddz = md_from_fixed(jz + shz - V.cz[q]);
-        if (md_boxes_within(ddx, ddy, ddz, V.ch[q], jh, c.list_cutoff2)) {
+        const float4 cc = V.box->cc[q];
+        if (md_boxes_within(ox - cc.x, oy - cc.y, oz - cc.z, V.box->ch[q], jh, box2)) {
           imask |= 1 << q;
           if (J == I && zero) self |= 1 << q;
         }
@@ -540,35 +573,60 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
 
 // Write the list entries of one super-cluster into its own region of the
 // entry arrays (entries_per_super entries from S * entries_per_super) and
-// their count: one wavefront per S, lanes over candidate J clusters,
-// compacted with a wavefront prefix count so the order is deterministic.  A
-// count past the region reports a list overflow.
-__global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T, md_bmap map) {
+// their count, and count each J's entries for the transposed list.  One
+// workgroup of MD_LIST_WAVES wavefronts per S, lanes over candidate J
+// clusters, each wave a chunk of 64; a prefix count over the round's waves
+// puts the entries in the order of one wave's scan (ascending J), so the list
+// does not depend on the number of waves.  The search of one S is a chain of
+// dependent loads and int64 arithmetic per chunk and the replica waits for
+// its slowest S, so the chunks run side by side (a rebuild's search with one wave per S, the
+// images in lockstep and int64 box tests: 157 us at 2,168 atoms, 241 at 243k;
+// so: 50 and 136).
+// A count past the region reports a list overflow.
+#define MD_LIST_WAVES 4
+__global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args *__restrict__ T, md_bmap map) {
   int S;
   const md_nb_args &A = md_nb_entry(T, map, S);
   md_control *ctl = A.ctl;
   if (!ctl->rebuild_active) return;
   const md_build_ctx &c = A.c;
   const md_list_ptrs &L = A.L;
-  int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (S >= c.nsuper) return;
+  __shared__ md_super_boxes boxes;
+  __shared__ int wave_count[MD_LIST_WAVES];
   md_super_view V;
   const int first = S * 8;
   V.first = first;
   V.nlocal = min(8, c.nclusters - first);
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    int k = min(first + q, c.nclusters - 1);
-    V.cx[q] = L.cluster_center[k];
-    V.cy[q] = L.cluster_center[c.nclusters + k];
-    V.cz[q] = L.cluster_center[2 * c.nclusters + k];
-    V.ch[q] = L.cluster_half[k];
+  V.box = &boxes;
+  if (threadIdx.x < 8) {
+    const int q = threadIdx.x, k = min(first + q, c.nclusters - 1);
+    boxes.cc[q] = make_float4(md_from_fixed(L.cluster_center[k] - L.super_origin[S]),
+                              md_from_fixed(L.cluster_center[c.nclusters + k] - L.super_origin[c.nsuper + S]),
+                              md_from_fixed(L.cluster_center[2 * c.nclusters + k] - L.super_origin[2 * c.nsuper + S]),
+                              0.0f);
+    boxes.ch[q] = L.cluster_half[k];
   }
+  __syncthreads();
+  // entries of the waves before this one in the round, and of all of them
+  auto round_counts = [&](int mine, int &before, int &all) {
+    if (lane == 0) wave_count[wave] = mine;
+    __syncthreads();
+    before = all = 0;
+    for (int w = 0; w < MD_LIST_WAVES; ++w) {
+      const int u = wave_count[w];
+      if (w < wave) before += u;
+      all += u;
+    }
+    __syncthreads();  // the next round rewrites the counts
+  };
   const int64_t ox = L.super_origin[S], oy = L.super_origin[c.nsuper + S], oz = L.super_origin[2 * c.nsuper + S];
   V.ox = ox;
   V.oy = oy;
   V.oz = oz;
-  V.rs = L.super_radius[S];
+  const float4 sphere = L.super_sphere[S];
+  V.rs = sphere.w;
   // Every image of a j-cluster that can come within the list radius of one of
   // S's clusters lies within R = list radius + largest cluster radius + r_S of
   // S's origin (some point of an i-cluster box, within r_S of the origin, comes
@@ -590,7 +648,7 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
       too_far |= k > MD_MAX_IMAGE_SHELLS;
       K[d] = min(k, MD_MAX_IMAGE_SHELLS);
     }
-  if (lane == 0 && too_far) ctl->overflow = 2;
+  if (threadIdx.x == 0 && too_far) ctl->overflow = 2;
   // Candidate j super-clusters SJ >= S, ascending.  A j-cluster of SJ can
   // reach an i-cluster of S only if the bounding spheres of the two
   // super-clusters come within the list radius at some image, so SJ is
@@ -617,21 +675,27 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
     }
   }
   if (prefilter) {
-    for (int sb = 0; sb < c.nsuper; sb += 64) {
-      const int SJ = sb + lane;
+    for (int sb = 0; sb < c.nsuper; sb += 64 * MD_LIST_WAVES) {
+      const int SJ = sb + (int)threadIdx.x;
       bool near = false;
       if (SJ < c.nsuper && (SJ == S || md_lists_pair(S, SJ))) {
-        const float lim = c.list_cutoff + rs + L.super_radius[SJ];
+        const float4 other = L.super_sphere[SJ];
+        const float lim = c.list_cutoff + rs + other.w;
         if (SJ == S) {
           near = true;
         } else {
-          int64_t dx = L.super_origin[SJ] - ox, dy = L.super_origin[c.nsuper + SJ] - oy,
-                  dz = L.super_origin[2 * c.nsuper + SJ] - oz;
-          md_min_image_fixed(dx, dy, dz, c.box);
-          // f32 images of the reduced difference, with a 1e-3 nm margin over
-          // their rounding (a candidate kept in excess makes no entry: each
-          // of its clusters still meets the exact tests below)
-          const float fx0 = md_from_fixed(dx), fy0 = md_from_fixed(dy), fz0 = md_from_fixed(dz);
+          // all in f32, with a 1e-3 nm margin over its rounding (a candidate
+          // kept in excess makes no entry: each of its clusters still meets
+          // the tests below)
+          float fx0 = other.x - sphere.x, fy0 = other.y - sphere.y, fz0 = other.z - sphere.z;
+          const float nc = floorf(fz0 / c.box.c[2] + 0.5f);
+          fx0 -= nc * c.box.c[0];
+          fy0 -= nc * c.box.c[1];
+          fz0 -= nc * c.box.c[2];
+          const float nb = floorf(fy0 / c.box.b[1] + 0.5f);
+          fx0 -= nb * c.box.b[0];
+          fy0 -= nb * c.box.b[1];
+          fx0 -= floorf(fx0 / c.box.a[0] + 0.5f) * c.box.a[0];
           const float limm = lim + 1e-3f, lim2 = limm * limm;
           for (int kc = -Kp[2]; kc <= Kp[2]; ++kc)
             for (int kb = -Kp[1]; kb <= Kp[1]; ++kb)
@@ -644,9 +708,11 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
         }
       }
       const uint64_t m = __ballot(near);
-      const int below = __popcll(m & ((uint64_t(1) << lane) - 1));
-      if (near && ncand + below < MD_LIST_CANDIDATES) cand[ncand + below] = SJ;
-      ncand += __popcll(m);
+      int before, all;
+      round_counts(__popcll(m), before, all);
+      const int at = ncand + before + __popcll(m & ((uint64_t(1) << lane) - 1));
+      if (near && at < MD_LIST_CANDIDATES) cand[at] = SJ;
+      ncand += all;
     }
     __syncthreads();
   }
@@ -655,9 +721,12 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
   const int chunks = scan_all ? (c.nclusters + 63) / 64 : (ncand + 7) / 8;
   int written = 0;
   const int base_out = S * c.entries_per_super, region_end = base_out + c.entries_per_super;
-  for (int chunk = 0; chunk < chunks; ++chunk) {
-    int J;
-    if (scan_all) {
+  for (int round = 0; round < chunks; round += MD_LIST_WAVES) {
+    const int chunk = round + wave;
+    int J = c.nclusters;
+    if (chunk >= chunks) {
+      // past the last chunk: this wave only takes part in the counting
+    } else if (scan_all) {
       J = 64 * chunk + lane;
       if (J < c.nclusters && J / 8 != S && !md_lists_pair(S, J / 8)) J = c.nclusters;
     } else {
@@ -682,8 +751,10 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
       int v = __shfl_up(incl, off, 64);
       if (lane >= off) incl += v;
     }
+    int before, all;
+    round_counts(__shfl(incl, 63, 64), before, all);
     if (valid && count) {
-      int at = base_out + written + incl - count;
+      int at = base_out + written + before + incl - count;
       int SJ = J / 8;
       int64_t jox = L.super_origin[SJ], joy = L.super_origin[c.nsuper + SJ], joz = L.super_origin[2 * c.nsuper + SJ];
       auto write = [&](int meta, int64_t shx, int64_t shy, int64_t shz) {
@@ -695,6 +766,7 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
           L.entry_shift[at] = make_int4(md_frame_coord(jox + shx - ox, bad), md_frame_coord(joy + shy - oy, bad),
                                         md_frame_coord(joz + shz - oz, bad), 0);
           if (bad) ctl->overflow = 3;
+          atomicAdd(&L.j_count[J], 1);
         }
         ++at;
       };
@@ -705,23 +777,24 @@ __global__ void __launch_bounds__(64) k_nb_list(const md_nb_args *__restrict__ T
           write(imask | (self << 8), shx, shy, shz);
         });
     }
-    written += __shfl(incl, 63, 64);
+    written += all;
   }
-  if (lane == 0) {
+  if (threadIdx.x == 0) {
     L.super_count[S] = written;
     if (written > c.entries_per_super) ctl->overflow = 1;
   }
 }
 
-// Starts of every super-cluster's entries and segments, and the totals.
-// one workgroup per replica
-__global__ void __launch_bounds__(1024) k_nb_list_scan(const md_nb_args *__restrict__ T, md_bmap map) {
+// Starts of every super-cluster's segments, the segments themselves, the
+// totals, and the starts of the transposed list.  One workgroup per replica.
+__global__ void __launch_bounds__(1024) k_nb_starts(const md_nb_args *__restrict__ T, md_bmap map) {
   int blk;
   const md_nb_args &A = md_nb_entry(T, map, blk);
   md_control *ctl = A.ctl;
   if (!ctl->rebuild_active) return;
   const md_list_ptrs &L = A.L;
   const int nsuper = A.c.nsuper, region = A.c.entries_per_super, segment_capacity = A.c.segment_capacity;
+  const int len = A.c.seg_len;
   int *totals = A.totals;
   __shared__ int entries;
   if (threadIdx.x == 0) entries = 0;
@@ -729,102 +802,112 @@ __global__ void __launch_bounds__(1024) k_nb_list_scan(const md_nb_args *__restr
   int mine = 0;
   for (int s = threadIdx.x; s < nsuper; s += 1024) {
     const int n = min(L.super_count[s], region);
-    L.super_segs[s] = (n + A.c.seg_len - 1) / A.c.seg_len;
+    L.super_segs[s] = (n + len - 1) / len;
     mine += n;
   }
   atomicAdd(&entries, mine);
   __syncthreads();
   md_block_scan(L.super_segs, L.super_segs, nsuper, nullptr);
+  md_block_scan(L.j_count, L.j_start, A.c.nclusters, L.j_count);
   __syncthreads();
   if (threadIdx.x == 0) {
-    int segs = L.super_segs[nsuper];
+    const int segs = L.super_segs[nsuper];
     if (segs > segment_capacity) ctl->overflow = 1;
     totals[0] = entries;
     totals[1] = min(segs, segment_capacity);
   }
-}
-
-__global__ void k_nb_segments(const md_nb_args *__restrict__ T, md_bmap map) {
-  int blk;
-  const md_nb_args &A = md_nb_entry(T, map, blk);
-  if (!A.ctl->rebuild_active) return;
-  const md_list_ptrs &L = A.L;
-  const int segment_capacity = A.c.segment_capacity, region = A.c.entries_per_super;
-  int S = blk * blockDim.x + threadIdx.x;
-  if (S >= A.c.nsuper) return;
-  const int b = S * region, e = b + min(L.super_count[S], region);
-  int sg = L.super_segs[S];
-  const int len = A.c.seg_len;
-  for (int at = b; at < e; at += len, ++sg) {
-    if (sg >= segment_capacity) break;
-    L.segments[sg] = make_int4(S, at, min(at + len, e), 0);
+  // 16 threads write one super-cluster's segments
+  for (int s = threadIdx.x >> 4; s < nsuper; s += 64) {
+    const int b = s * region, e = b + min(L.super_count[s], region), sg = L.super_segs[s];
+    for (int k = threadIdx.x & 15; b + k * len < e; k += 16) {
+      if (sg + k >= segment_capacity) break;
+      L.segments[sg + k] = make_int4(s, b + k * len, min(b + k * len + len, e), 0);
+    }
   }
 }
 
-// Exclusion masks: MD_MASK_WAVES wavefronts per super-cluster S, each taking
-// every MD_MASK_WAVES-th of S's entries, lane l = (i = l/8, j = l%8); for each
-// of S's 8 i-clusters a 64-bit mask of the pairs that interact.  Clears
-// padding, the lower triangle of a cluster with its own zero image, and every
-// excluded pair (the CSR holds both directions; nonbonded.ts:159-182).  An
-// exclusion is looked up in the i atom's 64-bit index window, and in the CSR
-// only for the rare atom flagged as having exclusions outside it.
-__global__ void __launch_bounds__(64 * MD_MASK_GROUP) k_nb_masks(const md_nb_args *__restrict__ T, md_bmap map) {
-  int blk;
-  const md_nb_args &A = md_nb_entry(T, map, blk);
+// Exclusion masks and the transposed list, one workgroup per super-cluster S.
+// An entry's mask for S's cluster q has bit (i = l/8, j = l%8) set when the
+// pair interacts: cleared for padding, for the lower triangle of a cluster
+// with its own zero image, and for every excluded pair (the CSR holds both
+// directions; nonbonded.ts:159-182).
+//
+// Driven by the exclusions, not by the pairs: S's 64 atoms have a few hundred
+// exclusions between them, each found in S's list by a binary search for its
+// j-cluster (the list ascends in J; the images of one J are adjacent), where
+// testing every pair of every entry against the exclusions is 512 tests per
+// entry (a rebuild's masks: 340 us at 243k atoms so tested, 30 this way).  The masks of MD_MASK_TILE entries at a time are put together
+// in LDS; a list longer than that takes several tiles.
+#define MD_MASK_TILE 256
+#define MD_MASK_THREADS 256
+__global__ void __launch_bounds__(MD_MASK_THREADS) k_nb_masks(const md_nb_args *__restrict__ T, md_bmap map) {
+  int S;
+  const md_nb_args &A = md_nb_entry(T, map, S);
   if (!A.ctl->rebuild_active) return;
   const md_build_ctx &c = A.c;
   const md_list_ptrs &L = A.L;
-  const int wave = blk * MD_MASK_GROUP + (int)(threadIdx.x >> 6);
-  const int S = wave / MD_MASK_WAVES, part = wave % MD_MASK_WAVES;
   if (S >= c.nsuper) return;
-  const int *slot_atom = A.slot_atom, *excl_start = A.excl_start, *excl_list = A.excl_list;
-  const int lane = threadIdx.x & 63, il = lane >> 3, jl = lane & 7;
-  int ia[8];
-  uint64_t iw[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int I = S * 8 + q;
-    ia[q] = I < c.nclusters ? slot_atom[I * MD_CLUSTER + il] : -1;
-    iw[q] = ia[q] >= 0 ? A.excl_window[ia[q]] : 0;
-  }
-  const int eb = S * c.entries_per_super, ee = eb + min(L.super_count[S], c.entries_per_super);
-  for (int e = eb + part; e < ee; e += MD_MASK_WAVES) {
-    const int J = L.entry_j[e];
-    const int meta = L.entry_imask[e];
-    if (lane == 0) atomicAdd(&L.j_count[J], 1);
-    const int ja = slot_atom[J * MD_CLUSTER + jl];
-    bool clean = true;
-    uint64_t masks[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      bool ok = ((meta >> q) & 1) && ia[q] >= 0 && ja >= 0;
-      if (ok && ((meta >> (8 + q)) & 1)) ok = jl > il;  // same cluster, zero image
-      if (ok) {
-        const int d = ja - ia[q];
-        if (d >= -32 && d < 32 && d != 0) {
-          ok = !((iw[q] >> (d + 32)) & 1);
-        } else if ((iw[q] >> 32) & 1) {
-          for (int k = excl_start[ia[q]]; k < excl_start[ia[q] + 1]; ++k)
-            if (excl_list[k] == ja) {
-              ok = false;
-              break;
-            }
-        }
+  __shared__ int tile_j[MD_MASK_TILE];
+  __shared__ int tile_meta[MD_MASK_TILE];
+  __shared__ unsigned long long mask[MD_MASK_TILE * 8];
+  const int eb = S * c.entries_per_super, count = min(L.super_count[S], c.entries_per_super);
+  const int *slot_atom = A.slot_atom, *atom_slot = A.atom_slot, *excl_start = A.excl_start, *excl_list = A.excl_list;
+  // four threads share one of S's atoms
+  const int slot = S * MD_SUPER + (int)(threadIdx.x >> 2), sub = threadIdx.x & 3;
+  const int a = slot_atom[slot];
+  const int q = (slot >> 3) & 7, il = slot & 7;
+  const int xb = a >= 0 ? excl_start[a] : 0, xe = a >= 0 ? excl_start[a + 1] : 0;
+  for (int t0 = 0; t0 < count; t0 += MD_MASK_TILE) {
+    const int nt = min(MD_MASK_TILE, count - t0);
+    for (int k = threadIdx.x; k < nt; k += MD_MASK_THREADS) {
+      const int J = L.entry_j[eb + t0 + k];
+      tile_j[k] = J;
+      tile_meta[k] = L.entry_imask[eb + t0 + k];
+      L.j_entries[L.j_start[J] + atomicAdd(&L.j_count[J], 1)] = eb + t0 + k;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < nt * 8; k += MD_MASK_THREADS) {
+      const int e = k >> 3, b = k & 7, meta = tile_meta[e];
+      uint64_t m = 0;
+      if ((meta >> b) & 1) {
+        // slots from n on are padding: the first ni rows, the first nj columns
+        const int ni = min(8, max(0, c.n - (S * 8 + b) * MD_CLUSTER)), nj = min(8, max(0, c.n - tile_j[e] * MD_CLUSTER));
+        m = ni >= 8 ? ~0ull : (1ull << (8 * ni)) - 1;
+        if (nj < 8) m &= 0x0101010101010101ull * (uint64_t)((1 << nj) - 1);
+        if ((meta >> (8 + b)) & 1) m &= 0x0080c0e0f0f8fcfeull;  // same cluster, zero image: j > i
       }
-      const uint64_t m = __ballot(ok);
-      masks[q] = m;
-      if ((meta >> q) & 1) clean = clean && m == ~0ull;
+      mask[k] = m;
     }
-    // a clean entry's masks are never read: only its meta word changes
-    if (clean) {
-      if (lane == 0) L.entry_imask[e] = meta | MD_META_CLEAN;
-    } else if (lane < 8) {
-      uint64_t m = masks[0];
-#pragma unroll
-      for (int q = 1; q < 8; ++q)
-        if (lane == q) m = masks[q];
-      L.entry_excl[(size_t)e * 8 + lane] = m;
+    __syncthreads();
+    for (int k = xb + sub; k < xe; k += 4) {
+      const int b = excl_list[k];
+      if (b == a) continue;
+      const int sb = atom_slot[b], J = sb / MD_CLUSTER;
+      int lo = 0, hi = nt;  // the first entry of the tile with a j-cluster >= J
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (tile_j[mid] < J)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      for (; lo < nt && tile_j[lo] == J; ++lo)
+        if ((tile_meta[lo] >> q) & 1) atomicAnd(&mask[lo * 8 + q], ~(1ull << (il * 8 + (sb & 7))));
     }
+    __syncthreads();
+    for (int k = threadIdx.x; k < nt * 8; k += MD_MASK_THREADS) {
+      // the 8 lanes of an entry agree on whether it is clean: every active
+      // block's mask all ones.  A clean entry's masks are never read: only its
+      // meta word changes.
+      const int e = k >> 3, b = k & 7, meta = tile_meta[e];
+      const uint64_t m = mask[k];
+      const uint64_t dirty = __ballot(((meta >> b) & 1) && m != ~0ull);
+      if ((dirty >> (threadIdx.x & 56)) & 0xff)
+        L.entry_excl[(size_t)(eb + t0 + e) * 8 + b] = m;
+      else if (b == 0)
+        L.entry_imask[eb + t0 + e] = meta | MD_META_CLEAN;
+    }
+    __syncthreads();  // the next tile rewrites the tables
   }
 }
 
@@ -954,31 +1037,6 @@ __global__ void k_nb_forces(const md_nb_args *__restrict__ T, md_bmap map, int e
     f[2] += md_to_fixed(e[2]);
   }
   for (int d = 0; d < 3; ++d) A.force[d * np + a] += f[d];
-}
-
-// The transposed list: starts from the counts k_nb_masks took (one
-// workgroup per replica), then each entry's number placed under its J.
-__global__ void __launch_bounds__(1024) k_nb_j_scan(const md_nb_args *__restrict__ T, md_bmap map) {
-  int blk;
-  const md_nb_args &A = md_nb_entry(T, map, blk);
-  if (!A.ctl->rebuild_active) return;
-  md_block_scan(A.L.j_count, A.L.j_start, A.c.nclusters, A.L.j_count);
-}
-
-// One wave per super-cluster (its ~200 entries are a few passes of 64
-// lanes): a launch over replicas that did not rebuild then dispatches 16
-// times fewer waves that return at once.
-__global__ void __launch_bounds__(64) k_nb_j_fill(const md_nb_args *__restrict__ T, md_bmap map) {
-  int S;
-  const md_nb_args &A = md_nb_entry(T, map, S);
-  if (!A.ctl->rebuild_active) return;
-  const md_list_ptrs &L = A.L;
-  if (S >= A.c.nsuper) return;
-  const int eb = S * A.c.entries_per_super, ee = eb + min(L.super_count[S], A.c.entries_per_super);
-  for (int e = eb + (int)threadIdx.x; e < ee; e += 64) {
-    const int J = L.entry_j[e];
-    L.j_entries[L.j_start[J] + atomicAdd(&L.j_count[J], 1)] = e;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1705,13 +1763,12 @@ std::vector<int> md_cell_walk(int W, int H, int D) {
 
 struct md_nb_buffers {
   int64_t *cluster_center = nullptr, *super_origin = nullptr;
-  float *super_radius = nullptr;
+  float4 *super_sphere = nullptr;
   int *super_count = nullptr, *super_segs = nullptr;
   int *entry_j = nullptr, *entry_imask = nullptr;
   int4 *entry_shift = nullptr;
   int4 *segments = nullptr;
   uint64_t *entry_excl = nullptr;
-  uint64_t *excl_window = nullptr;
   int64_t *slot_force = nullptr;
   int *j_count = nullptr, *j_start = nullptr, *j_entries = nullptr;
   float *j_force = nullptr;
@@ -1888,7 +1945,7 @@ void md_nb_setup(md_system *s) {
   s->cluster_half = md_alloc<float4>(s, nb.nclusters);
   B.cluster_center = md_alloc<int64_t>(s, 3 * (size_t)nb.nclusters);
   B.super_origin = md_alloc<int64_t>(s, 3 * (size_t)B.nsuper);
-  B.super_radius = md_alloc<float>(s, B.nsuper);
+  B.super_sphere = md_alloc<float4>(s, B.nsuper);
   B.super_count = md_alloc<int>(s, B.nsuper);
   B.super_segs = md_alloc<int>(s, B.nsuper + 1);
   B.totals = md_alloc<int>(s, 4);
@@ -1928,19 +1985,7 @@ void md_nb_setup(md_system *s) {
   if (!s->excl_list.empty())
     MD_HIP(hipMemcpyAsync(s->excl_list_d, s->excl_list.data(), sizeof(int) * s->excl_list.size(),
                           hipMemcpyHostToDevice, s->stream));
-  // each atom's exclusions within 32 indices as a bit window (bit d + 32 for
-  // atom i + d, d in [-32, 31], d != 0); bit 32 marks an atom that also has
-  // exclusions further away, which the mask kernel then looks up in the CSR
-  std::vector<uint64_t> window(s->n, 0);
-  for (int i = 0; i < s->n; ++i)
-    for (int k = s->excl_start[i]; k < s->excl_start[i + 1]; ++k) {
-      const int d = s->excl_list[k] - i;
-      if (d == 0) continue;
-      window[i] |= d >= -32 && d < 32 ? uint64_t(1) << (d + 32) : uint64_t(1) << 32;
-    }
-  B.excl_window = md_alloc<uint64_t>(s, s->n);
   B.slot_force = md_alloc<int64_t>(s, 3 * (size_t)nb.nslots);
-  MD_HIP(hipMemcpyAsync(B.excl_window, window.data(), sizeof(uint64_t) * s->n, hipMemcpyHostToDevice, s->stream));
   MD_HIP(hipStreamSynchronize(s->stream));
 }
 
@@ -2001,7 +2046,7 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   L.cluster_center = B.cluster_center;
   L.cluster_half = s->cluster_half;
   L.super_origin = B.super_origin;
-  L.super_radius = B.super_radius;
+  L.super_sphere = B.super_sphere;
   L.super_count = B.super_count;
   L.super_segs = B.super_segs;
   L.entry_j = B.entry_j;
@@ -2057,14 +2102,13 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   a.slot_offset = s->slot_offset;
   a.cluster_center = B.cluster_center;
   a.super_origin = B.super_origin;
-  a.super_radius = B.super_radius;
+  a.super_sphere = B.super_sphere;
   a.slot_lj = s->slot_lj;
   a.slot_xyzq = s->slot_xyzq;
   a.cluster_half = s->cluster_half;
   a.atom_param = s->atom_param;
   a.excl_start = s->excl_start_d;
   a.excl_list = s->excl_list_d;
-  a.excl_window = B.excl_window;
   a.force = s->force;
   a.cluster_lo = B.cluster_lo;
   a.cluster_hi = B.cluster_hi;
@@ -2076,7 +2120,7 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
 // a group's launch tables for the nonbonded kernels
 struct md_nb_group {
   md_nb_args *table = nullptr;  // [R], device
-  md_launch atoms, scan, clusters, supers, segments, masks, slots;
+  md_launch atoms, scan, clusters, supers, slots;
   md_launch seg;                // the pair kernel's segment numbering
   int pair_grid = 1;
   int seg_len = MD_SEGMENT;
@@ -2089,31 +2133,28 @@ void md_nb_group_setup(md_group *g) {
   auto *G = new md_nb_group();
   g->nb = G;
   const int R = (int)g->reps.size();
-  std::vector<int> atoms, one, clusters, supers, segments, masks, slots;
+  std::vector<int> atoms, one, clusters, supers, slots;
   for (md_system *s : g->reps) {
     auto &B = nbuf(s);
     atoms.push_back((s->n + 255) / 256);
     one.push_back(1);
     clusters.push_back((s->nb.nclusters + 63) / 64);
     supers.push_back(B.nsuper);
-    segments.push_back((B.nsuper + 63) / 64);
-    masks.push_back(B.nsuper * (MD_MASK_WAVES / MD_MASK_GROUP));
     slots.push_back((s->nb.nslots + 255) / 256);
   }
   G->atoms = md_make_launch(g, atoms);
   G->scan = md_make_launch(g, one);
   G->clusters = md_make_launch(g, clusters);
   G->supers = md_make_launch(g, supers);
-  G->segments = md_make_launch(g, segments);
-  G->masks = md_make_launch(g, masks);
   G->slots = md_make_launch(g, slots);
   G->seg.map.start = md_group_alloc<int>(g, R + 1);
   G->seg.map.R = R;
   G->table = md_group_alloc<md_nb_args>(g, R);
-  // The pair kernel's waves: one per segment of about 200 entries per
-  // super-cluster, at most MD_PAIR_WAVES
+  // The pair kernel's waves: one per segment the list has room for (waves
+  // without one leave at once; with fewer waves than segments some would take
+  // two and the launch wait for them), at most MD_PAIR_WAVES
   long units = 0;
-  for (md_system *s : g->reps) units += (long)nbuf(s).nsuper * (200 / MD_SEGMENT);
+  for (md_system *s : g->reps) units += (long)nbuf(s).entry_capacity / MD_SEGMENT;
   G->pair_grid = (int)std::min<long>(MD_PAIR_WAVES, std::max<long>(MD_XCDS, units));
   md_nb_group_refresh(g);
 }
@@ -2176,13 +2217,10 @@ void md_nb_build(md_group *g) {
   k_nb_rank<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
   k_nb_clusters<<<G.clusters.total, 64, 0, st>>>(T, G.clusters.map);
   md_mark(g, MD_PHASE_SEARCH);
-  k_nb_list<<<G.supers.total, 64, 0, st>>>(T, G.supers.map);
-  k_nb_list_scan<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
-  k_nb_segments<<<G.segments.total, 64, 0, st>>>(T, G.segments.map);
+  k_nb_list<<<G.supers.total, 64 * MD_LIST_WAVES, 0, st>>>(T, G.supers.map);
+  k_nb_starts<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
   md_mark(g, MD_PHASE_MASKS);
-  k_nb_masks<<<G.masks.total, 64 * MD_MASK_GROUP, 0, st>>>(T, G.masks.map);
-  k_nb_j_scan<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
-  k_nb_j_fill<<<G.supers.total, 64, 0, st>>>(T, G.supers.map);
+  k_nb_masks<<<G.supers.total, MD_MASK_THREADS, 0, st>>>(T, G.supers.map);
   MD_HIP(hipGetLastError());
 }
 
