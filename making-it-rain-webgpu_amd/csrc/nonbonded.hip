@@ -430,12 +430,12 @@ __global__ void k_nb_clusters(const md_nb_args *__restrict__ T, md_bmap map) {
   }
 }
 
-// AABB distance test between cluster boxes separated by d (nm, f32)
-__device__ __forceinline__ bool md_boxes_within(float dx, float dy, float dz, float4 h1, float4 h2, float r2) {
+// squared distance between cluster boxes whose centres are d apart (nm, f32)
+__device__ __forceinline__ float md_box_distance2(float dx, float dy, float dz, float4 h1, float4 h2) {
   float ex = fmaxf(fabsf(dx) - (h1.x + h2.x), 0.0f);
   float ey = fmaxf(fabsf(dy) - (h1.y + h2.y), 0.0f);
   float ez = fmaxf(fabsf(dz) - (h1.z + h2.z), 0.0f);
-  return ex * ex + ey * ey + ez * ez < r2;
+  return ex * ex + ey * ey + ez * ez;
 }
 
 // The candidate periodic images of cluster J relative to cluster c: the
@@ -503,9 +503,11 @@ __device__ void md_for_each_image(const md_build_ctx &c, int64_t dx, int64_t dy,
 // Super-cluster S as its list waves see it: its clusters' boxes (in LDS), the
 // frame origin and the bounding-sphere radius of the whole super-cluster.  A
 // j-cluster's image is placed exactly against the origin and rounded once to
-// f32; the box tests then run in f32 (within 1e-6 nm, by which they are
-// widened), not on int64 differences for each of the 8 boxes.
+// f32; the box tests run on that, and only one within 1e-5 nm^2 of the list
+// radius (f32 is within 2e-6) is decided on the int64 difference of the two
+// centres, so the list is the one those differences give.
 struct md_super_boxes {
+  int64_t cx[8], cy[8], cz[8];
   float4 cc[8];  // centres from the frame origin (nm)
   float4 ch[8];  // half extents
 };
@@ -541,7 +543,6 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
   float4 jh = L.cluster_half[J];
   const float reach = c.list_cutoff + V.rs + sqrtf(jh.x * jh.x + jh.y * jh.y + jh.z * jh.z) + 1e-3f;
   const float reach2 = reach * reach;
-  const float box2 = (c.list_cutoff + 1e-6f) * (c.list_cutoff + 1e-6f);
   // the image is chosen against S's origin and shared by the entry; S's own
   // clusters keep their unshifted frame (see md_for_each_image)
   int64_t dx = jx - V.ox, dy = jy - V.oy, dz = jz - V.oz;
@@ -561,7 +562,12 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
       // S lists, md_lists_pair)
       if (q < V.nlocal && (!own || J >= I) && !(J == I && !zero && code < 0)) {
         const float4 cc = V.box->cc[q];
-        if (md_boxes_within(ox - cc.x, oy - cc.y, oz - cc.z, V.box->ch[q], jh, box2)) {
+        const float near2 = md_box_distance2(ox - cc.x, oy - cc.y, oz - cc.z, V.box->ch[q], jh);
+        bool within = near2 < c.list_cutoff2;
+        if (fabsf(near2 - c.list_cutoff2) < 1e-5f)
+          within = md_box_distance2(md_from_fixed(jx + shx - V.box->cx[q]), md_from_fixed(jy + shy - V.box->cy[q]),
+                                    md_from_fixed(jz + shz - V.box->cz[q]), V.box->ch[q], jh) < c.list_cutoff2;
+        if (within) {
           imask |= 1 << q;
           if (J == I && zero) self |= 1 << q;
         }
@@ -602,10 +608,12 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
   V.box = &boxes;
   if (threadIdx.x < 8) {
     const int q = threadIdx.x, k = min(first + q, c.nclusters - 1);
-    boxes.cc[q] = make_float4(md_from_fixed(L.cluster_center[k] - L.super_origin[S]),
-                              md_from_fixed(L.cluster_center[c.nclusters + k] - L.super_origin[c.nsuper + S]),
-                              md_from_fixed(L.cluster_center[2 * c.nclusters + k] - L.super_origin[2 * c.nsuper + S]),
-                              0.0f);
+    boxes.cx[q] = L.cluster_center[k];
+    boxes.cy[q] = L.cluster_center[c.nclusters + k];
+    boxes.cz[q] = L.cluster_center[2 * c.nclusters + k];
+    boxes.cc[q] = make_float4(md_from_fixed(boxes.cx[q] - L.super_origin[S]),
+                              md_from_fixed(boxes.cy[q] - L.super_origin[c.nsuper + S]),
+                              md_from_fixed(boxes.cz[q] - L.super_origin[2 * c.nsuper + S]), 0.0f);
     boxes.ch[q] = L.cluster_half[k];
   }
   __syncthreads();
