@@ -344,11 +344,12 @@ enum {
   MD_PHASE_BONDED = 4,   /* bonds, angles, torsions, exceptions, restraints */
   MD_PHASE_SPREAD = 5,   /* PME charge spreading */
   MD_PHASE_FFT = 6,      /* PME forward FFT, convolution, inverse FFT */
-  MD_PHASE_GATHER = 7,   /* PME force interpolation */
+  MD_PHASE_GATHER = 7,   /* PME force interpolation (in one pass with MD_PHASE_FORCES,
+                            whose time the two share equally) */
   MD_PHASE_INTEGRATE = 8,/* LFMiddle/Verlet + SETTLE/SHAKE/RATTLE + COM */
   MD_PHASE_SEARCH = 9,   /* cluster-pair search, list starts, segments (gated) */
   MD_PHASE_MASKS = 10,   /* exclusion masks and the list by j-cluster (gated) */
-  MD_PHASE_FORCES = 11,  /* pair forces from slots and list entries onto the atoms */
+  MD_PHASE_FORCES = 11,  /* pair and bonded forces onto the atoms (see MD_PHASE_GATHER) */
   MD_PHASE_COUNT = 12
 };
 md_err md_profile_steps(md_system *sys, int32_t steps, double *ms);

@@ -565,15 +565,15 @@ static void create(md_system *s, const md_system_desc *d, const md_run_options *
         const int at[4] = {ta[t].x, ta[t].y, ta[t].z, ta[t].w};
         for (int j = 0; j < per[k]; ++j) owner.push_back(at[j]);
       }
-    std::vector<int> start(np + 1, 0), list(owner.size());
+    std::vector<int> start(np + 1, 0), at_piece(owner.size());
     for (int a : owner) ++start[a + 1];
     for (int a = 0; a < np; ++a) start[a + 1] += start[a];
     std::vector<int> fill(start.begin(), start.end() - 1);
-    for (size_t q = 0; q < owner.size(); ++q) list[fill[owner[q]]++] = (int)q;
+    for (size_t q = 0; q < owner.size(); ++q) at_piece[q] = fill[owner[q]]++;
     s->n_pieces = (int)owner.size();
     s->term_piece = md_alloc<int64_t>(s, std::max<size_t>(1, 3 * owner.size()));
     s->atom_piece_start = upload(s, start);
-    s->atom_piece = upload(s, list);
+    s->piece_at = upload(s, at_piece);
   }
   s->restraint_ref = upload(s, rref);
   s->water_atoms = upload(s, R.waters);
@@ -633,6 +633,8 @@ static void launch_step(md_group *g) {
   if (nb) {
     md_mark(g, MD_PHASE_SPREAD);
     md_pme(g, false);
+  } else {
+    md_bonded_forces(g);
   }
   md_mark(g, MD_PHASE_INTEGRATE);
   md_integrate(g);
@@ -746,7 +748,6 @@ static void run_group(md_group *g, int64_t steps) {
   if (steps <= 0) return;
   MD_HIP(hipSetDevice(g->device));
   group_prepare(g);
-  md_zero_forces(g, false);
   const int stride = g->max_batch > 0 ? g->max_batch : STRIDE_STEPS;
   if (g->graph_stale) drop_graphs(g);
   g->graph_stale = false;
@@ -807,7 +808,6 @@ static void evaluate(md_system *s, double *forces, double *groups, double *total
   fault_tick(s, 1);
   md_group *grp = s->self;
   group_prepare(grp);
-  md_zero_forces(grp, true);
   if (census) {
     MD_HIP(hipMemsetAsync(&s->ctl->pair_census, 0, sizeof(int64_t), s->stream));
     MD_HIP(hipMemsetAsync(&s->ctl->pair_blocks, 0, sizeof(int64_t), s->stream));
@@ -818,7 +818,10 @@ static void evaluate(md_system *s, double *forces, double *groups, double *total
     md_nb_pairs(grp, true);
   }
   md_bonded(grp, true);
-  if (s->has_nonbonded) md_pme(grp, true);
+  if (s->has_nonbonded)
+    md_pme(grp, true);
+  else
+    md_bonded_forces(grp);
   int64_t e[MD_E_SLOTS];
   MD_HIP(hipMemcpyAsync(e, s->energy, sizeof e, hipMemcpyDeviceToHost, s->stream));
   std::vector<int64_t> f;
@@ -1061,7 +1064,6 @@ static void profile_group(md_group *g, int steps, double *ms) {
   MD_HIP(hipSetDevice(g->device));
   for (int k = 0; k < MD_PHASE_COUNT; ++k) ms[k] = 0.0;
   group_prepare(g);
-  md_zero_forces(g, false);
   for (int r = 0; r < steps; ++r) {
     g->profiling = true;
     try {
@@ -1083,6 +1085,7 @@ static void profile_group(md_group *g, int steps, double *ms) {
     g->prof_phase.clear();
   }
   for (int k = 0; k < MD_PHASE_COUNT; ++k) ms[k] /= steps;
+  if (g->nb) ms[MD_PHASE_GATHER] = ms[MD_PHASE_FORCES] = 0.5 * ms[MD_PHASE_FORCES];  // one pass (k_forces)
   for (md_system *s : g->reps) s->steps_done += steps;
   for (md_system *s : g->reps) check_control(s);
 }

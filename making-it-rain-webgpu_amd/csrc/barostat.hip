@@ -206,14 +206,16 @@ __global__ void k_baro_restore(const md_baro_dev *B, int64_t *pos, const int64_t
 
 // the step's force kernels with energies on, into the energy slots
 static void baro_energy(md_group *g, bool nb) {
-  md_zero_forces(g, true);
   md_step_prologue(g, false);
   if (nb) {
     md_nb_build(g);
     md_nb_pairs(g, true);
   }
   md_bonded(g, true);
-  if (nb) md_pme(g, true);
+  if (nb)
+    md_pme(g, true);
+  else
+    md_bonded_forces(g);
 }
 
 static void baro_box_constants(md_group *g, const double *box, bool nb) {
@@ -239,7 +241,6 @@ void md_baro_attempt(md_system *s) {
   k_baro_decide<<<1, 1, 0, g->stream>>>(B.dev, s->energy, ek, B.seed, B.pressure, B.kt, B.nmol, s->ctl);
   k_baro_restore<<<(s->n + 255) / 256, 256, 0, g->stream>>>(B.dev, s->pos, B.saved, s->n, s->np);
   baro_box_constants(g, dev_box(B), nb);
-  md_zero_forces(g, false);
   MD_HIP(hipGetLastError());
 }
 

@@ -27,8 +27,8 @@ struct md_term_args {
   const int64_t *pos;
   int64_t *force;
   int64_t *energy;
-  int64_t *piece;  // [pieces][3]: each (term, atom) force in Q32.32
-  const int *piece_start, *piece_list;  // by atom: [np + 1], then piece numbers
+  int64_t *piece;  // [pieces][3]: each (term, atom) force in Q32.32, by atom
+  const int *piece_start, *piece_at;  // an atom's pieces [np + 1]; a term's piece's place
   int np;
   int n_bonds, n_angles, n_torsions, n_exceptions, n_restraints;
   double alpha;
@@ -38,10 +38,12 @@ struct md_term_args {
 __device__ __forceinline__ int64_t md_d_to_fixed(double v) { return (int64_t)rint(v * 4294967296.0); }
 
 // Piece p of the term list takes one atom's force from one term, stored
-// plainly: atoms shared by many terms (a torsion's four atoms sit in a dozen
-// other terms) would otherwise serialise their 64-bit atomics at memory.
+// plainly at its place among the atom's pieces: atoms shared by many terms (a
+// torsion's four atoms sit in a dozen other terms) would otherwise serialise
+// their 64-bit atomics at memory, and the scattered stores cost nothing to
+// wait for where scattered reads would.
 __device__ __forceinline__ void md_put_piece(const md_term_args &A, int p, double fx, double fy, double fz) {
-  int64_t *q = A.piece + 3 * (size_t)p;
+  int64_t *q = A.piece + 3 * (size_t)A.piece_at[p];
   q[0] = md_d_to_fixed(fx);
   q[1] = md_d_to_fixed(fy);
   q[2] = md_d_to_fixed(fz);
@@ -203,33 +205,21 @@ __global__ void __launch_bounds__(256) k_terms(const md_term_args *__restrict__ 
   }
 }
 
-// Each atom's share of the terms: the sum of its pieces added to its force.
-// Kernels on one stream run in order and a thread is the only one holding
-// its atom here, so a plain read-add-write is enough; integer sums make the
-// order of the pieces irrelevant to the bits.
+// The forces of systems without a NonbondedForce: the sum of each atom's
+// pieces (the others' are summed with the pair and mesh forces, k_forces).
 __global__ void k_terms_gather(const md_term_args *__restrict__ T, md_bmap map) {
   int blk;
   const md_term_args &A = T[md_locate(map, blockIdx.x, blk)];
   const int a = blk * blockDim.x + threadIdx.x;
   if (a >= A.np) return;
-  const int b = A.piece_start[a], e = A.piece_start[a + 1];
-  if (b == e) return;
   int64_t f[3] = {0, 0, 0};
-  for (int k = b; k < e; ++k) {
-    const int64_t *q = A.piece + 3 * (size_t)A.piece_list[k];
+  for (int k = A.piece_start[a]; k < A.piece_start[a + 1]; ++k) {
+    const int64_t *q = A.piece + 3 * (size_t)k;
     f[0] += q[0];
     f[1] += q[1];
     f[2] += q[2];
   }
-  for (int d = 0; d < 3; ++d) A.force[d * A.np + a] += f[d];
-}
-
-__global__ void k_zero_forces(const md_term_args *__restrict__ T, md_bmap map, int zero_energy) {
-  int blk;
-  const md_term_args &A = T[md_locate(map, blockIdx.x, blk)];
-  int i = blk * blockDim.x + threadIdx.x;
-  if (i < 3 * A.np) A.force[i] = 0;
-  if (zero_energy && i < MD_E_SLOTS) A.energy[i] = 0;
+  for (int d = 0; d < 3; ++d) A.force[d * A.np + a] = f[d];
 }
 
 static md_term_args term_args(md_system *s) {
@@ -241,7 +231,7 @@ static md_term_args term_args(md_system *s) {
   A.force = s->force;
   A.piece = s->term_piece;
   A.piece_start = s->atom_piece_start;
-  A.piece_list = s->atom_piece;
+  A.piece_at = s->piece_at;
   A.energy = s->energy;
   A.np = s->np;
   A.n_bonds = s->n_bonds;
@@ -256,7 +246,7 @@ static md_term_args term_args(md_system *s) {
 
 struct md_bonded_group {
   md_term_args *table = nullptr;
-  md_launch zero, terms, atoms;
+  md_launch terms, atoms;
 };
 
 static md_bonded_group &bg(md_group *g) { return *reinterpret_cast<md_bonded_group *>(g->bonded); }
@@ -264,14 +254,12 @@ static md_bonded_group &bg(md_group *g) { return *reinterpret_cast<md_bonded_gro
 void md_bonded_group_setup(md_group *g) {
   auto *G = new md_bonded_group();
   g->bonded = G;
-  std::vector<int> zero, terms, atoms;
+  std::vector<int> terms, atoms;
   for (md_system *s : g->reps) {
-    zero.push_back((3 * s->np + 255) / 256);
-    atoms.push_back(s->n_pieces > 0 ? (s->np + 255) / 256 : 0);
+    atoms.push_back((s->np + 255) / 256);
     int total = s->n_bonds + s->n_angles + s->n_torsions + s->n_exceptions + s->n_restraints;
     terms.push_back((total + 255) / 256);
   }
-  G->zero = md_make_launch(g, zero);
   G->terms = md_make_launch(g, terms);
   G->atoms = md_make_launch(g, atoms);
   G->table = md_group_alloc<md_term_args>(g, g->reps.size());
@@ -304,12 +292,6 @@ void md_bonded_group_free(md_group *g) {
   g->bonded = nullptr;
 }
 
-void md_zero_forces(md_group *g, bool energies) {
-  auto &G = bg(g);
-  k_zero_forces<<<G.zero.total, 256, 0, g->stream>>>(G.table, G.zero.map, energies ? 1 : 0);
-  MD_HIP(hipGetLastError());
-}
-
 void md_bonded(md_group *g, bool energy) {
   auto &G = bg(g);
   if (G.terms.total == 0) return;
@@ -317,6 +299,11 @@ void md_bonded(md_group *g, bool energy) {
     k_terms<true><<<G.terms.total, 256, 0, g->stream>>>(G.table, G.terms.map);
   else
     k_terms<false><<<G.terms.total, 256, 0, g->stream>>>(G.table, G.terms.map);
+  MD_HIP(hipGetLastError());
+}
+
+void md_bonded_forces(md_group *g) {
+  auto &G = bg(g);
   k_terms_gather<<<G.atoms.total, 256, 0, g->stream>>>(G.table, G.atoms.map);
   MD_HIP(hipGetLastError());
 }

@@ -255,21 +255,21 @@ struct md_system {
   int n_bonds = 0, n_angles = 0, n_torsions = 0, n_exceptions = 0, n_restraints = 0;
   int4 *term_atoms = nullptr;
   double4 *term_param = nullptr;
-  // the terms' forces as pieces, one Q32.32 triple per (term, atom) in term
-  // order (2, 3, 4, 2, 1 atoms for a bond, angle, torsion, exception,
-  // restraint), and by atom the pieces to sum: k_terms stores pieces,
-  // k_terms_gather adds each atom's sum to its force (no atomics)
+  // the terms' forces as pieces, one Q32.32 triple per (term, atom), an
+  // atom's pieces side by side: k_terms stores each where `piece_at` says (in
+  // term order: 2, 3, 4, 2, 1 atoms for a bond, angle, torsion, exception,
+  // restraint), and the pass that makes the atom's force reads them in a row
   int n_pieces = 0;
-  int64_t *term_piece = nullptr;    // [n_pieces][3]
+  int64_t *term_piece = nullptr;    // [n_pieces][3], by atom
   int *atom_piece_start = nullptr;  // [np + 1]
-  int *atom_piece = nullptr;        // [n_pieces]
+  int *piece_at = nullptr;          // [n_pieces]
   int64_t *restraint_ref = nullptr;  // [3][n_restraints] Q32.32
 
   // ---- PME ------------------------------------------------------------
   int pme_nx = 0, pme_ny = 0, pme_nz = 0, pme_nzc = 0;
   int64_t *pme_grid = nullptr;  // [nx][ny][nz] Q32.32 charge
   float2 *pme_cgrid = nullptr;  // [nx][ny][nz/2+1]
-  float *pme_phi = nullptr;     // [nx][ny][nz] dE/dQ
+  float *pme_phi = nullptr;     // [nx][ny][nz + 4] dE/dQ, rows continued periodically
   void *pme_ext = nullptr;
 
   // ---- constraints / integrator work items -----------------------------
@@ -322,10 +322,24 @@ T *md_alloc(md_system *s, size_t count) {
 // starts a phase; outside md_profile_steps it does nothing.
 void md_mark(md_group *g, int phase);
 
+// What the pair kernel leaves for the pass that makes the atoms' forces.
+struct md_pair_forces {
+  int64_t *slot_force;  // [3][nslots] i forces, cleared behind the pass
+  const float *j_force;
+  const int *j_start, *j_entries;
+  int64_t *part;  // the evaluation's energy and counts, MD_ENERGY_PARTS lines
+  int64_t *census, *blocks;
+};
+// lines the pair kernel's energy sums are spread over: thousands of waves
+// adding to one word would queue there (about 20 ns each)
+#define MD_ENERGY_PARTS 64
+#define MD_ENERGY_STRIDE 8  // int64 words: one 64-byte line
+
 // ---- per-system setup (each in its own .hip file) ---------------------------
 void md_nb_setup(md_system *s);                 // nonbonded.hip: buffers of one system
 std::vector<int> md_cell_walk(int W, int H, int D);  // nonbonded.hip: cell sort order
 void md_nb_free(md_system *s);
+md_pair_forces md_nb_pair_forces(md_system *s);
 int64_t md_nb_entries(md_system *s);
 int64_t md_nb_capacity(md_system *s);
 void md_pme_setup(md_system *s);                // pme.hip
@@ -353,10 +367,11 @@ bool md_nb_get_compact(md_group *g);
 void md_nb_build(md_group *g);                  // rebuild kernels, gated per replica
 void md_nb_pairs(md_group *g, bool energy);
 void md_bonded(md_group *g, bool energy);       // bonded.hip
-void md_zero_forces(md_group *g, bool energies);
-void md_pme(md_group *g, bool energy);          // pme.hip
-// integrate.hip: advance the step counters and latch each replica's rebuild
-// request (its own displacement test, or `force_pending` set by the host)
+void md_bonded_forces(md_group *g);             // the terms' forces alone (no NonbondedForce)
+void md_pme(md_group *g, bool energy);          // pme.hip: the mesh, then every atom's force
+// integrate.hip: advance the step counters (or, for an evaluation, clear the
+// energies) and latch each replica's rebuild request (its own displacement
+// test, or `force_pending` set by the host)
 void md_step_prologue(md_group *g, bool advance);
 void md_integrate(md_group *g);
 void md_momentum(md_group *g);

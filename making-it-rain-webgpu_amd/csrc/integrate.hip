@@ -34,6 +34,7 @@ struct md_int_args {
   const int64_t *build_pos;
   md_control *ctl;
   uint32_t *group_status;  // the launch group's error word (see k_step_prologue)
+  int64_t *energy;         // [MD_E_SLOTS]
   int np;
   float dt, half_dt, inv_dt;
   float vscale, noise_scale, kt;
@@ -152,7 +153,6 @@ __device__ __forceinline__ void md_load_kick(const md_int_args &A, md_item<MAXA>
       it.x[a][d] = A.pos[d * A.np + i];
       float v = A.vel[d * A.np + i];
       int64_t f = A.force[d * A.np + i];
-      A.force[d * A.np + i] = 0;  // consumed: the next step accumulates afresh
       if (it.im[a] != 0.0f) {
         v -= vcom[d];
         v = v + A.dt * it.im[a] * md_from_fixed(f);
@@ -861,8 +861,8 @@ __global__ void __launch_bounds__(256) k_constrain(const md_int_args *__restrict
 
 // start of a step, one thread per replica: advance the device step counter,
 // latch the rebuild request (the displacement test's, or the host's),
-// clear the momentum slot this step's integrator fills, and raise the group's
-// status word when an earlier step left an error in the control block
+// clear the momentum slot this step's integrator fills (or, not advancing, the
+// energies an evaluation sums), and raise the group's status word when an earlier step left an error in the control block
 __global__ void k_step_prologue(const md_int_args *__restrict__ T, int R, int advance) {
   int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= R) return;
@@ -873,6 +873,8 @@ __global__ void k_step_prologue(const md_int_args *__restrict__ T, int R, int ad
     ctl->step_next = ctl->step_next + 1;
     int64_t s = ctl->step_current;
     for (int d = 0; d < 3; ++d) ctl->momentum[(s + 1) & 1][d] = 0;
+  } else {
+    for (int k = 0; k < MD_E_SLOTS; ++k) T[r].energy[k] = 0;
   }
   ctl->rebuild_active = ctl->rebuild_request[0] | ctl->force_pending;
   ctl->rebuild_request[0] = 0;
@@ -912,6 +914,7 @@ static md_int_args int_args(md_system *s) {
   A.mass = s->mass_f;
   A.build_pos = s->build_pos;
   A.ctl = s->ctl;
+  A.energy = s->energy;
   A.np = s->np;
   double dt = s->opt.time_step;
   A.dt = (float)dt;

@@ -117,22 +117,18 @@ struct md_pair_args {
   const int *totals;
   // Q32.32 forces by slot, [3][nslots]: a cluster's 8 atoms are 8 adjacent
   // words, so the 8 or 64 lanes of one atomic instruction hit one or a few
-  // cache lines instead of as many random atoms; k_nb_forces moves them to
+  // cache lines instead of as many random atoms; k_forces moves them to
   // the atoms
   int64_t *slot_force;
   // per list entry, the f32 force on each of J's 8 atoms, [entry][x|y|z][8]:
-  // one plain store per entry instead of 24 atomics; k_nb_forces sums them
+  // one plain store per entry instead of 24 atomics; k_forces sums them
   float *j_force;
   // each cluster's current bounding box in its frame (frame units; a cluster
   // of padding only holds an inverted box), written by k_nb_pack
   const int4 *cluster_lo, *cluster_hi;
-  // the energy, census and block counts of one evaluation, in MD_ENERGY_PARTS
-  // lines of their own: thousands of waves adding to one word would queue
-  // there (about 20 ns each); k_nb_forces sums the lines and clears them
+  // energy, in-cutoff pairs and 8x8 blocks evaluated, in MD_ENERGY_PARTS
+  // lines; k_forces sums the lines and clears them
   int64_t *part;
-  int64_t *energy;
-  int64_t *census;  // in-cutoff pairs (md_control)
-  int64_t *blocks;  // 8x8 cluster-pair blocks evaluated (md_control)
   int nslots, nclusters;
   // in the pair kernel's frame units (see md_pair): cutoff^2 in 2^-52 nm^2;
   // alpha/2 and 2 alpha / sqrt(pi) times 2^-26; -alpha^2 / ln 2 times 2^-52
@@ -164,7 +160,6 @@ struct md_nb_args {
   float4 *cluster_half;
   const float4 *atom_param;
   const int *excl_start, *excl_list;
-  int64_t *force;  // the atoms' Q32.32 forces, [3][np]
   int4 *cluster_lo, *cluster_hi;
   int *totals;
   md_control *ctl;
@@ -921,8 +916,6 @@ __global__ void __launch_bounds__(MD_MASK_THREADS) k_nb_masks(const md_nb_args *
 
 #define MD_XCDS 8
 #define MD_PAIR_WAVES 32768
-#define MD_ENERGY_PARTS 64
-#define MD_ENERGY_STRIDE 8  // int64 words: one 64-byte line
 
 // Per step: each slot's position as f32 in its super-cluster's frame.
 // The launch's first thread also lays out the pair kernel's work: the start of
@@ -986,65 +979,6 @@ __global__ void k_nb_pack(const md_nb_args *__restrict__ T, md_bmap map, int *se
     A.cluster_lo[s / MD_CLUSTER] = make_int4(lo[0], lo[1], lo[2], 0);
     A.cluster_hi[s / MD_CLUSTER] = make_int4(hi[0], hi[1], hi[2], 0);
   }
-}
-
-// After the pair kernel: each slot's force onto its atom -- its i-force sums
-// plus, as j atom, the force of every list entry naming its cluster, each
-// rounded to Q32.32 on its own (the value an atomic per entry would add) --
-// and the slot cleared for the next step.  Kernels on one stream run in order
-// and a slot is the only one holding its atom, so a plain read-add-write is
-// enough.
-// Blocks laid out XCD by XCD: neighbouring clusters read j-force records of
-// neighbouring entries, so they share one L2.
-__global__ void k_nb_forces(const md_nb_args *__restrict__ T, md_bmap map, int energy) {
-  int blk;
-  const md_nb_args &A = T[md_locate(map, md_xcd_block(blockIdx.x, gridDim.x), blk)];
-  if (energy && blk == 0 && threadIdx.x < MD_ENERGY_PARTS) {
-    // the pair kernel's energy and counts: one wave, lane per part
-    int64_t *part = A.P.part + threadIdx.x * MD_ENERGY_STRIDE;
-    int64_t *const to[3] = {A.P.energy + MD_E_PAIR, A.P.census, A.P.blocks};
-    for (int k = 0; k < 3; ++k) {
-      const int64_t v = md_wave_sum_i64(part[k]);
-      part[k] = 0;
-      if (threadIdx.x == 0) *to[k] += v;
-    }
-  }
-  const int nslots = A.c.nslots, np = A.c.np;
-  const int s = blk * blockDim.x + threadIdx.x;
-  if (s >= nslots) return;
-  int64_t *slot_force = A.P.slot_force;
-  const int a = A.slot_atom[s];
-  int64_t f[3];
-  for (int d = 0; d < 3; ++d) {
-    f[d] = slot_force[d * nslots + s];
-    slot_force[d * nslots + s] = 0;
-  }
-  if (a < 0) return;
-  const int J = s / MD_CLUSTER, q = s - J * MD_CLUSTER;
-  const float *jf = A.P.j_force + q * 3;
-  const int *je = A.L.j_entries;
-  int k = A.L.j_start[J];
-  const int end = A.L.j_start[J + 1];
-  // four entries' records in flight at a time: each iteration's loads are
-  // independent of the last, so the loop waits once per four entries on the
-  // entry index and once on the records (integer sums: order-free)
-  for (; k + 4 <= end; k += 4) {
-    const int e0 = je[k], e1 = je[k + 1], e2 = je[k + 2], e3 = je[k + 3];
-    const float *r0 = jf + (size_t)e0 * 24, *r1 = jf + (size_t)e1 * 24, *r2 = jf + (size_t)e2 * 24,
-                *r3 = jf + (size_t)e3 * 24;
-    const float x0 = r0[0], y0 = r0[1], z0 = r0[2], x1 = r1[0], y1 = r1[1], z1 = r1[2];
-    const float x2 = r2[0], y2 = r2[1], z2 = r2[2], x3 = r3[0], y3 = r3[1], z3 = r3[2];
-    f[0] += md_to_fixed(x0) + md_to_fixed(x1) + md_to_fixed(x2) + md_to_fixed(x3);
-    f[1] += md_to_fixed(y0) + md_to_fixed(y1) + md_to_fixed(y2) + md_to_fixed(y3);
-    f[2] += md_to_fixed(z0) + md_to_fixed(z1) + md_to_fixed(z2) + md_to_fixed(z3);
-  }
-  for (; k < end; ++k) {
-    const float *e = jf + (size_t)je[k] * 24;
-    f[0] += md_to_fixed(e[0]);
-    f[1] += md_to_fixed(e[1]);
-    f[2] += md_to_fixed(e[2]);
-  }
-  for (int d = 0; d < 3; ++d) A.force[d * np + a] += f[d];
 }
 
 // ---------------------------------------------------------------------------
@@ -2079,9 +2013,6 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   P.totals = B.totals;
   P.slot_force = B.slot_force;
   P.part = B.energy_part;
-  P.energy = s->energy;
-  P.census = &s->ctl->pair_census;
-  P.blocks = &s->ctl->pair_blocks;
   P.nslots = s->nb.nslots;
   P.nclusters = s->nb.nclusters;
   P.cutoff2 = std::ldexp(s->nb.cutoff2, 52);
@@ -2117,7 +2048,6 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   a.atom_param = s->atom_param;
   a.excl_start = s->excl_start_d;
   a.excl_list = s->excl_list_d;
-  a.force = s->force;
   a.cluster_lo = B.cluster_lo;
   a.cluster_hi = B.cluster_hi;
   a.totals = B.totals;
@@ -2254,9 +2184,13 @@ void md_nb_pairs(md_group *g, bool energy) {
     else
       k_nb_pairs<false, false><<<G.pair_grid, 64, 0, st>>>(G.table, G.seg.map);
   }
-  md_mark(g, MD_PHASE_FORCES);
-  k_nb_forces<<<G.slots.total, 256, 0, st>>>(G.table, G.slots.map, energy ? 1 : 0);
   MD_HIP(hipGetLastError());
+}
+
+md_pair_forces md_nb_pair_forces(md_system *s) {
+  auto &B = nbuf(s);
+  return md_pair_forces{B.slot_force, B.j_force, B.j_start, B.j_entries, B.energy_part, &s->ctl->pair_census,
+                        &s->ctl->pair_blocks};
 }
 
 int64_t md_nb_entries(md_system *s) {
