@@ -227,35 +227,61 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
+// idx / m for 0 <= idx < 2^20 by an f32 reciprocal (an integer division is some
+// 30 instructions, more than a radix-4 butterfly): (idx + 1/2) / m is at least
+// 1/(2m) from an integer, and the product is within 3.6e-7 of it relatively.
+__device__ __forceinline__ float md_inverse(int m) { return __builtin_amdgcn_rcpf((float)m); }
+__device__ __forceinline__ int md_div(int idx, float inv) { return (int)(((float)idx + 0.5f) * inv); }
+
+// Where a stage finds its input and puts its output: lines of LDS (element e
+// of line l at l * line + e * elem; a transposed read swaps the strides), or
+// the kernel's own memory through its Ext.
+struct md_fft_io {
+  const float2 *in;
+  int in_line, in_elem;
+  float2 *out;
+  int out_line;
+  bool ext_in, ext_out;
+};
+
 // One Stockham stage of radix R (a compile-time constant, so a butterfly's R
 // values stay in registers): output j of sub-transform k gathers the R
 // inputs j + q m, multiplies input q by the twiddle w^(k q n / (ns R)) (an
-// index below n, as k < ns and q < R), and takes their length-R DFT.
-template <int R>
-__device__ __forceinline__ void md_fft_stage(const float2 *in, float2 *out, int nlines, int n, int ns,
+// index below n, as k < ns and q < R), and takes their length-R DFT.  A stage
+// that touches the kernel's memory walks it in the order of its addresses
+// (Ext::line_fast: consecutive threads on consecutive lines).
+template <int R, class Ext>
+__device__ __forceinline__ void md_fft_stage(const md_fft_io &io, Ext &ext, int nlines, int n, int ns,
                                              const float2 *tw, float sign) {
   const int m = n / R;
-  const int twstride = n / (ns * R);
-  const int dftstride = n / R;
+  const int twstride = m / ns;
+  const int dftstride = m;
+  const bool lines_first = (io.ext_in || io.ext_out) && Ext::line_fast;
+  const float inv = md_inverse(lines_first ? nlines : m), inv_ns = md_inverse(ns);
   for (int idx = threadIdx.x; idx < nlines * m; idx += blockDim.x) {
-    const int line = idx / m, j = idx - line * m;
-    const int k = j % ns;
-    float2 v[R];
-    const float2 *src = in + line * n;
+    const int hi = md_div(idx, inv);
+    const int line = lines_first ? idx - hi * nlines : hi, j = lines_first ? hi : idx - hi * m;
+    const int k = j - md_div(j, inv_ns) * ns;
+    float2 v[R], o[R];
+    if (io.ext_in) {
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-      float2 x = src[j + q * m];
-      if (q > 0 && k > 0) {
+      for (int q = 0; q < R; ++q) v[q] = ext.load(line, j + q * m);
+    } else {
+      const float2 *src = io.in + line * io.in_line + j * io.in_elem;
+#pragma unroll
+      for (int q = 0; q < R; ++q) v[q] = src[q * m * io.in_elem];
+    }
+    if (k > 0) {
+#pragma unroll
+      for (int q = 1; q < R; ++q) {
         float2 w = tw[k * q * twstride];
         w.y *= -sign;  // table holds exp(-2 pi i t/n); inverse conjugates
-        x = cmul(x, w);
+        v[q] = cmul(v[q], w);
       }
-      v[q] = x;
     }
-    float2 *dst = out + line * n + (j / ns) * ns * R + k;
     if constexpr (R == 2) {
-      dst[0] = make_float2(v[0].x + v[1].x, v[0].y + v[1].y);
-      dst[ns] = make_float2(v[0].x - v[1].x, v[0].y - v[1].y);
+      o[0] = make_float2(v[0].x + v[1].x, v[0].y + v[1].y);
+      o[1] = make_float2(v[0].x - v[1].x, v[0].y - v[1].y);
     } else if constexpr (R == 4) {
       float2 s0 = make_float2(v[0].x + v[2].x, v[0].y + v[2].y);
       float2 s1 = make_float2(v[0].x - v[2].x, v[0].y - v[2].y);
@@ -263,10 +289,10 @@ __device__ __forceinline__ void md_fft_stage(const float2 *in, float2 *out, int 
       float2 s3 = make_float2(v[1].x - v[3].x, v[1].y - v[3].y);
       // multiply s3 by sign*i: forward (-i), inverse (+i)
       float2 t3 = make_float2(-sign * s3.y, sign * s3.x);
-      dst[0] = make_float2(s0.x + s2.x, s0.y + s2.y);
-      dst[ns] = make_float2(s1.x + t3.x, s1.y + t3.y);
-      dst[2 * ns] = make_float2(s0.x - s2.x, s0.y - s2.y);
-      dst[3 * ns] = make_float2(s1.x - t3.x, s1.y - t3.y);
+      o[0] = make_float2(s0.x + s2.x, s0.y + s2.y);
+      o[1] = make_float2(s1.x + t3.x, s1.y + t3.y);
+      o[2] = make_float2(s0.x - s2.x, s0.y - s2.y);
+      o[3] = make_float2(s1.x - t3.x, s1.y - t3.y);
     } else {
 #pragma unroll
       for (int qo = 0; qo < R; ++qo) {
@@ -279,39 +305,60 @@ __device__ __forceinline__ void md_fft_stage(const float2 *in, float2 *out, int 
           acc.x += p.x;
           acc.y += p.y;
         }
-        dst[qo * ns] = acc;
+        o[qo] = acc;
       }
+    }
+    const int to = (j - k) * R + k;
+    if (io.ext_out) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) ext.store(line, to + q * ns, o[q]);
+    } else {
+      float2 *dst = io.out + line * io.out_line + to;
+#pragma unroll
+      for (int q = 0; q < R; ++q) dst[q * ns] = o[q];
     }
   }
 }
 
-// `nlines` contiguous lines of length P.n in `a` (pitch P.n), transformed with
-// sign -1 (forward) or +1 (inverse); returns the buffer holding the result.
-// Each stage dispatches on its radix to the specialised butterfly.
-__device__ __forceinline__ float2 *md_lds_fft(float2 *a, float2 *b, int nlines, const md_fft_plan &P,
-                                              const float2 *tw_all, float sign) {
-  const int n = P.n;
-  const float2 *tw = tw_all + P.tw;
+// pitch of a line of n values in LDS: odd, so that a transposed read of
+// consecutive lines meets each bank once
+__host__ __device__ inline int md_pitch(int n) { return n | 1; }
+
+// `nlines` lines of length P.n, transformed with sign -1 (forward) or +1
+// (inverse) through the LDS buffers a and b.  The input is `src` (one of the
+// two, with its line and element strides) or, with a null src, the kernel's
+// memory through ext.load; the output is a buffer (returned, lines md_pitch
+// apart) or, with `out`, the kernel's memory through ext.store.  Twiddles come
+// from LDS.  Ends with a barrier unless it ends in ext.store.
+template <class Ext>
+__device__ __forceinline__ float2 *md_fft(float2 *a, float2 *b, const float2 *src, int line, int elem, bool out,
+                                          Ext &ext, int nlines, const md_fft_plan &P, const float2 *tw, float sign) {
+  const int n = P.n, pitch = md_pitch(n);
   int ns = 1;
-  float2 *in = a, *out = b;
+  md_fft_io io{src, line, elem, src == a ? b : a, pitch, src == nullptr, false};
   for (int s = 0; s < P.nstages; ++s) {
     const int r = P.radix[s];
+    io.ext_out = out && s + 1 == P.nstages;
     switch (r) {
-      case 2: md_fft_stage<2>(in, out, nlines, n, ns, tw, sign); break;
-      case 3: md_fft_stage<3>(in, out, nlines, n, ns, tw, sign); break;
-      case 4: md_fft_stage<4>(in, out, nlines, n, ns, tw, sign); break;
-      case 5: md_fft_stage<5>(in, out, nlines, n, ns, tw, sign); break;
-      case 7: md_fft_stage<7>(in, out, nlines, n, ns, tw, sign); break;
-      case 11: md_fft_stage<11>(in, out, nlines, n, ns, tw, sign); break;
-      default: md_fft_stage<13>(in, out, nlines, n, ns, tw, sign); break;
+      case 2: md_fft_stage<2>(io, ext, nlines, n, ns, tw, sign); break;
+      case 3: md_fft_stage<3>(io, ext, nlines, n, ns, tw, sign); break;
+      case 4: md_fft_stage<4>(io, ext, nlines, n, ns, tw, sign); break;
+      case 5: md_fft_stage<5>(io, ext, nlines, n, ns, tw, sign); break;
+      case 7: md_fft_stage<7>(io, ext, nlines, n, ns, tw, sign); break;
+      case 11: md_fft_stage<11>(io, ext, nlines, n, ns, tw, sign); break;
+      default: md_fft_stage<13>(io, ext, nlines, n, ns, tw, sign); break;
     }
-    __syncthreads();
-    float2 *t = in;
-    in = out;
-    out = t;
+    if (!io.ext_out) __syncthreads();
+    float2 *done = io.out;
+    io = md_fft_io{done, pitch, 1, done == a ? b : a, pitch, false, false};
     ns *= r;
   }
-  return in;
+  return const_cast<float2 *>(io.in);
+}
+
+// this length's twiddles into LDS (visible after the next barrier)
+__device__ __forceinline__ void md_load_twiddles(float2 *to, const md_fft_plan &P, const float2 *tw_all) {
+  for (int k = threadIdx.x; k < P.n; k += blockDim.x) to[k] = tw_all[P.tw + k];
 }
 
 // The potential's rows are MD_PHI_PAD values longer than the mesh, the row's
@@ -332,6 +379,49 @@ __device__ __forceinline__ void md_put_phi(float *row, int z, int nz, float v) {
   if (z < MD_PHI_PAD) row[nz + z] = v;
 }
 
+// The kernels' memory as their transforms' first and last stages see it.
+//
+// The charge grid's rows as lines (row r0 + line), read as f32 and cleared.
+struct md_ext_charge {
+  static constexpr bool line_fast = false;
+  int64_t *grid;
+  float2 *out;  // k_pme_z_forward's half rows
+  int nz, nzc;
+  __device__ float2 load(int line, int z) const {
+    int64_t *p = grid + (size_t)line * nz + z;
+    const int64_t v = *p;
+    *p = 0;
+    return make_float2((float)((double)v * 2.3283064365386963e-10), 0.0f);
+  }
+  __device__ void store(int line, int z, float2 v) const {
+    if (z < nzc) out[(size_t)line * nzc + z] = v;
+  }
+};
+// lines along a strided axis, `line` the consecutive index
+struct md_ext_lines {
+  static constexpr bool line_fast = true;
+  const float2 *in;
+  float2 *out;
+  size_t stride;
+  __device__ float2 load(int line, int e) const { return in[e * stride + line]; }
+  __device__ void store(int line, int e, float2 v) const { out[e * stride + line] = v; }
+};
+// the Hermitian half rows of a real line (x and y are back in real space, so
+// g(x, y, -kz) = conj(g(x, y, kz)) in the same row), and its real values
+struct md_ext_potential {
+  static constexpr bool line_fast = false;
+  const float2 *in;  // the half rows: element kz of line l at l * line + kz * elem
+  int line, elem;
+  float *phi;
+  int nz, nzc;
+  __device__ float2 load(int l, int z) const {
+    if (z < nzc) return in[l * line + z * elem];
+    const float2 w = in[l * line + (nz - z) * elem];
+    return make_float2(w.x, -w.y);
+  }
+  __device__ void store(int l, int z, float2 v) const { md_put_phi(phi + (size_t)l * (nz + MD_PHI_PAD), z, nz, v.x); }
+};
+
 // z pass, forward: int64 rows -> f32 -> complex FFT -> first nz/2+1 values.
 // Clears the integer grid behind it.  Block = PME_BATCH rows.
 __global__ void __launch_bounds__(256) k_pme_z_forward(const md_pme_table *__restrict__ T, md_bmap map) {
@@ -339,50 +429,41 @@ __global__ void __launch_bounds__(256) k_pme_z_forward(const md_pme_table *__res
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  int64_t *grid = E.grid;
-  float2 *cgrid = E.cgrid;
-  int rows = P.nx * P.ny;
-  int r0 = blk * PME_BATCH;
-  int nl = min(PME_BATCH, rows - r0);
-  float2 *a = lds, *b = lds + PME_BATCH * P.nz;
-  for (int idx = threadIdx.x; idx < nl * P.nz; idx += blockDim.x) {
-    int l = idx / P.nz, z = idx - l * P.nz;
-    size_t at = (size_t)(r0 + l) * P.nz + z;
-    int64_t v = grid[at];
-    grid[at] = 0;
-    a[l * P.nz + z] = make_float2((float)((double)v * 2.3283064365386963e-10), 0.0f);
-  }
+  const int rows = P.nx * P.ny, r0 = blk * PME_BATCH, nl = min(PME_BATCH, rows - r0);
+  float2 *a = lds, *b = a + PME_BATCH * md_pitch(P.nz), *tw = b + PME_BATCH * md_pitch(P.nz);
+  md_load_twiddles(tw, P.pz, P.tw);
   __syncthreads();
-  float2 *res = md_lds_fft(a, b, nl, P.pz, P.tw, -1.0f);
-  for (int idx = threadIdx.x; idx < nl * P.nzc; idx += blockDim.x) {
-    int l = idx / P.nzc, z = idx - l * P.nzc;
-    cgrid[(size_t)(r0 + l) * P.nzc + z] = res[l * P.nz + z];
-  }
+  md_ext_charge ext{E.grid + (size_t)r0 * P.nz, E.cgrid + (size_t)r0 * P.nzc, P.nz, P.nzc};
+  md_fft(a, b, nullptr, 0, 0, true, ext, nl, P.pz, tw, -1.0f);
 }
 
-// y pass: lines along y at fixed (x, kz); a block takes PME_BATCH
-// consecutive kz at one x, so global reads are contiguous runs.
+// Lines along y or x are taken a run of consecutive kz at a time, at most
+// PME_BATCH, the runs of one row of equal length (33 values as three runs of
+// 11, not 16, 16 and 1).
+__host__ __device__ inline int md_kz_runs(int nzc) { return (nzc + PME_BATCH - 1) / PME_BATCH; }
+__device__ __forceinline__ void md_kz_run(int nzc, int run, int &z0, int &nl) {
+  const int runs = md_kz_runs(nzc), per = (nzc + runs - 1) / runs;
+  z0 = run * per;
+  nl = max(0, min(per, nzc - z0));
+}
+
+// y pass: lines along y at fixed (x, kz)
 __global__ void __launch_bounds__(256) k_pme_y(const md_pme_table *__restrict__ T, md_bmap map, float sign) {
   extern __shared__ float2 lds[];
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  float2 *cgrid = E.cgrid;
-  int kzb = (P.nzc + PME_BATCH - 1) / PME_BATCH;
-  int x = blk / kzb;
-  int z0 = (blk - x * kzb) * PME_BATCH;
-  int nl = min(PME_BATCH, P.nzc - z0);
-  float2 *a = lds, *b = lds + PME_BATCH * P.ny;
-  for (int idx = threadIdx.x; idx < nl * P.ny; idx += blockDim.x) {
-    int y = idx / nl, l = idx - y * nl;
-    a[l * P.ny + y] = cgrid[((size_t)x * P.ny + y) * P.nzc + z0 + l];
-  }
+  const int runs = md_kz_runs(P.nzc), x = blk / runs;
+  int z0, nl;
+  md_kz_run(P.nzc, blk - x * runs, z0, nl);
+  float2 *a = lds, *b = a + PME_BATCH * md_pitch(P.ny), *tw = b + PME_BATCH * md_pitch(P.ny);
+  md_load_twiddles(tw, P.py, P.tw);
   __syncthreads();
-  float2 *res = md_lds_fft(a, b, nl, P.py, P.tw, sign);
-  for (int idx = threadIdx.x; idx < nl * P.ny; idx += blockDim.x) {
-    int y = idx / nl, l = idx - y * nl;
-    cgrid[((size_t)x * P.ny + y) * P.nzc + z0 + l] = res[l * P.ny + y];
-  }
+  float2 *plane = E.cgrid + (size_t)x * P.ny * P.nzc + z0;
+  md_ext_lines ext{plane, plane, (size_t)P.nzc};
+  // (one butterfly of a single-stage plan owns its whole line, so a line is
+  // read before it is written either way)
+  md_fft(a, b, nullptr, 0, 0, true, ext, nl, P.py, tw, sign);
 }
 
 // x pass with the convolution: forward transform along x, multiply by the
@@ -393,29 +474,27 @@ __global__ void __launch_bounds__(256) k_pme_x_convolve(const md_pme_table *__re
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  float2 *cgrid = E.cgrid;
   int64_t *energy = E.energy;
-  int kzb = (P.nzc + PME_BATCH - 1) / PME_BATCH;
-  int y = blk / kzb;
-  int z0 = (blk - y * kzb) * PME_BATCH;
-  int nl = min(PME_BATCH, P.nzc - z0);
-  float2 *a = lds, *b = lds + PME_BATCH * P.nx;
-  size_t xstride = (size_t)P.ny * P.nzc;
-  for (int idx = threadIdx.x; idx < nl * P.nx; idx += blockDim.x) {
-    int x = idx / nl, l = idx - x * nl;
-    a[l * P.nx + x] = cgrid[x * xstride + (size_t)y * P.nzc + z0 + l];
-  }
+  const int runs = md_kz_runs(P.nzc), y = blk / runs;
+  int z0, nl;
+  md_kz_run(P.nzc, blk - y * runs, z0, nl);
+  const int pitch = md_pitch(P.nx);
+  float2 *a = lds, *b = a + PME_BATCH * pitch, *tw = b + PME_BATCH * pitch;
+  md_load_twiddles(tw, P.px, P.tw);
   __syncthreads();
-  float2 *res = md_lds_fft(a, b, nl, P.px, P.tw, -1.0f);
-  float e = 0.0f;
+  float2 *const at = E.cgrid + (size_t)y * P.nzc + z0;
+  md_ext_lines ext{at, at, (size_t)P.ny * P.nzc};
+  float2 *res = md_fft(a, b, nullptr, 0, 0, false, ext, nl, P.px, tw, -1.0f);
+  double e = 0.0;
   int mb = y <= P.ny / 2 ? y : y - P.ny;
   const float two_pi = 6.283185307179586f;
+  const float inv_nx = md_inverse(P.nx);
   for (int idx = threadIdx.x; idx < nl * P.nx; idx += blockDim.x) {
-    int l = idx / P.nx, x = idx - l * P.nx;
+    const int l = md_div(idx, inv_nx), x = idx - l * P.nx;
     int kz = z0 + l;
     int ma = x <= P.nx / 2 ? x : x - P.nx;
     int mc = kz;
-    float2 v = res[l * P.nx + x];
+    float2 v = res[l * pitch + x];
     float2 outv = make_float2(0.0f, 0.0f);
     if (!(x == 0 && y == 0 && kz == 0)) {
       float kx = two_pi * (ma * P.invf[0]);
@@ -428,21 +507,16 @@ __global__ void __launch_bounds__(256) k_pme_x_convolve(const md_pme_table *__re
         // the half grid stands for both k and -k except on the kz = 0 and
         // kz = nz/2 planes, which are their own partners
         float weight = (kz == 0 || (2 * kz == P.nz)) ? 1.0f : 2.0f;
-        e += weight * factor * (v.x * v.x + v.y * v.y);
+        e += (double)(weight * factor * (v.x * v.x + v.y * v.y));
       }
       outv = make_float2(2.0f * factor * v.x, 2.0f * factor * v.y);
     }
-    res[l * P.nx + x] = outv;
+    res[l * pitch + x] = outv;
   }
   __syncthreads();
-  float2 *other = res == a ? b : a;
-  float2 *res2 = md_lds_fft(res, other, nl, P.px, P.tw, 1.0f);
-  for (int idx = threadIdx.x; idx < nl * P.nx; idx += blockDim.x) {
-    int x = idx / nl, l = idx - x * nl;
-    cgrid[x * xstride + (size_t)y * P.nzc + z0 + l] = res2[l * P.nx + x];
-  }
+  md_fft(a, b, res, pitch, 1, true, ext, nl, P.px, tw, 1.0f);
   if (ENERGY) {
-    int64_t f = md_wave_sum_i64(md_to_fixed(e));
+    int64_t f = md_wave_sum_i64((int64_t)rint(e * 4294967296.0));
     if ((threadIdx.x & 63) == 0) md_atomic_add_i64(energy + MD_E_RECIPROCAL, f);
   }
 }
@@ -453,104 +527,64 @@ __global__ void __launch_bounds__(256) k_pme_z_inverse(const md_pme_table *__res
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  const float2 *cgrid = E.cgrid;
-  float *phi = E.phi;
-  int rows = P.nx * P.ny;
-  int r0 = blk * PME_BATCH;
-  int nl = min(PME_BATCH, rows - r0);
-  float2 *a = lds, *b = lds + PME_BATCH * P.nz;
-  for (int idx = threadIdx.x; idx < nl * P.nz; idx += blockDim.x) {
-    int l = idx / P.nz, z = idx - l * P.nz;
-    float2 v;
-    if (z < P.nzc) {
-      v = cgrid[(size_t)(r0 + l) * P.nzc + z];
-    } else {
-      // x and y are back in real space, so each row is the z transform of a
-      // real line: g(x, y, -kz) = conj(g(x, y, kz)), same row
-      float2 w = cgrid[(size_t)(r0 + l) * P.nzc + (P.nz - z)];
-      v = make_float2(w.x, -w.y);
-    }
-    a[l * P.nz + z] = v;
-  }
+  const int rows = P.nx * P.ny, r0 = blk * PME_BATCH, nl = min(PME_BATCH, rows - r0);
+  float2 *a = lds, *b = a + PME_BATCH * md_pitch(P.nz), *tw = b + PME_BATCH * md_pitch(P.nz);
+  md_load_twiddles(tw, P.pz, P.tw);
   __syncthreads();
-  float2 *res = md_lds_fft(a, b, nl, P.pz, P.tw, 1.0f);
-  for (int idx = threadIdx.x; idx < nl * P.nz; idx += blockDim.x) {
-    int l = idx / P.nz, z = idx - l * P.nz;
-    md_put_phi(phi + (size_t)(r0 + l) * (P.nz + MD_PHI_PAD), z, P.nz, res[l * P.nz + z].x);
-  }
+  md_ext_potential ext{E.cgrid + (size_t)r0 * P.nzc, P.nzc, 1, E.phi + (size_t)r0 * (P.nz + MD_PHI_PAD), P.nz, P.nzc};
+  md_fft(a, b, nullptr, 0, 0, true, ext, nl, P.pz, tw, 1.0f);
+}
+
+// values of one LDS buffer for a whole x-plane: ny lines along z, then nz/2+1
+// along y
+__host__ __device__ inline int md_plane_buffer(int ny, int nz) {
+  const int rows = ny * md_pitch(nz), columns = (nz / 2 + 1) * md_pitch(ny);
+  return rows > columns ? rows : columns;
 }
 
 // The z and y passes of one x-plane in one workgroup, the plane kept in LDS
-// between them (meshes whose plane fits: 2 ny nz complex values).  The same
-// line transforms as k_pme_z_forward then k_pme_y, with the same inputs, so
-// the same bits; one launch and one trip through memory fewer.
-__global__ void __launch_bounds__(256) k_pme_yz_forward(const md_pme_table *__restrict__ T, md_bmap map) {
+// between them (meshes whose plane fits).  The same line transforms as
+// k_pme_z_forward then k_pme_y, with the same inputs, so the same bits; one
+// launch and one trip through memory fewer.  The first stage reads the grid
+// and the last writes the spectrum; the y lines' first stage reads the z
+// lines' output transposed, so nothing is copied in between.
+#define MD_PLANE_THREADS 512
+__global__ void __launch_bounds__(MD_PLANE_THREADS) k_pme_yz_forward(const md_pme_table *__restrict__ T, md_bmap map) {
   extern __shared__ float2 lds[];
   int x;
   const md_pme_table &E = md_pme_entry(T, map, x);
   const md_pme_args &P = E.P;
-  int64_t *grid = E.grid;
-  float2 *cgrid = E.cgrid;
-  const int ny = P.ny, nz = P.nz, nzc = P.nzc;
-  float2 *a = lds, *b = lds + ny * nz;
-  for (int idx = threadIdx.x; idx < ny * nz; idx += blockDim.x) {
-    const int y = idx / nz, z = idx - y * nz;
-    const size_t at = ((size_t)x * ny + y) * nz + z;
-    const int64_t v = grid[at];
-    grid[at] = 0;
-    a[y * nz + z] = make_float2((float)((double)v * 2.3283064365386963e-10), 0.0f);
-  }
+  const int ny = P.ny, nz = P.nz, nzc = P.nzc, size = md_plane_buffer(ny, nz);
+  float2 *a = lds, *b = lds + size, *twz = b + size, *twy = twz + nz;
+  md_load_twiddles(twz, P.pz, P.tw);
+  md_load_twiddles(twy, P.py, P.tw);
   __syncthreads();
-  float2 *res = md_lds_fft(a, b, ny, P.pz, P.tw, -1.0f);  // [y][kz]
-  float2 *other = res == a ? b : a;
-  for (int idx = threadIdx.x; idx < nzc * ny; idx += blockDim.x) {
-    const int kz = idx / ny, y = idx - kz * ny;
-    other[kz * ny + y] = res[y * nz + kz];
-  }
-  __syncthreads();
-  float2 *res2 = md_lds_fft(other, res, nzc, P.py, P.tw, -1.0f);  // [kz][ky]
-  for (int idx = threadIdx.x; idx < ny * nzc; idx += blockDim.x) {
-    const int ky = idx / nzc, kz = idx - ky * nzc;
-    cgrid[((size_t)x * ny + ky) * nzc + kz] = res2[kz * ny + ky];
-  }
+  md_ext_charge rows{E.grid + (size_t)x * ny * nz, nullptr, nz, nzc};
+  float2 *res = md_fft(a, b, nullptr, 0, 0, false, rows, ny, P.pz, twz, -1.0f);  // [y][kz]
+  float2 *plane = E.cgrid + (size_t)x * ny * nzc;
+  md_ext_lines columns{plane, plane, (size_t)nzc};
+  md_fft(a, b, res, 1, md_pitch(nz), true, columns, nzc, P.py, twy, -1.0f);  // [ky][kz]
 }
 
 // The inverse y and z passes of one x-plane (k_pme_y with +1, then
 // k_pme_z_inverse), the plane kept in LDS between them.
-__global__ void __launch_bounds__(256) k_pme_yz_inverse(const md_pme_table *__restrict__ T, md_bmap map) {
+__global__ void __launch_bounds__(MD_PLANE_THREADS) k_pme_yz_inverse(const md_pme_table *__restrict__ T, md_bmap map) {
   extern __shared__ float2 lds[];
   int x;
   const md_pme_table &E = md_pme_entry(T, map, x);
   const md_pme_args &P = E.P;
-  const float2 *cgrid = E.cgrid;
-  float *phi = E.phi;
-  const int ny = P.ny, nz = P.nz, nzc = P.nzc;
-  float2 *a = lds, *b = lds + ny * nz;
-  for (int idx = threadIdx.x; idx < nzc * ny; idx += blockDim.x) {
-    const int kz = idx / ny, y = idx - kz * ny;
-    a[kz * ny + y] = cgrid[((size_t)x * ny + y) * nzc + kz];
-  }
+  const int ny = P.ny, nz = P.nz, nzc = P.nzc, size = md_plane_buffer(ny, nz);
+  float2 *a = lds, *b = lds + size, *twz = b + size, *twy = twz + nz;
+  md_load_twiddles(twz, P.pz, P.tw);
+  md_load_twiddles(twy, P.py, P.tw);
   __syncthreads();
-  float2 *res = md_lds_fft(a, b, nzc, P.py, P.tw, 1.0f);  // [kz][y]
-  float2 *other = res == a ? b : a;
-  for (int idx = threadIdx.x; idx < ny * nz; idx += blockDim.x) {
-    const int y = idx / nz, z = idx - y * nz;
-    float2 v;
-    if (z < nzc) {
-      v = res[z * ny + y];
-    } else {
-      // x and y are back in real space: g(x, y, -kz) = conj(g(x, y, kz))
-      const float2 w = res[(nz - z) * ny + y];
-      v = make_float2(w.x, -w.y);
-    }
-    other[y * nz + z] = v;
-  }
-  __syncthreads();
-  float2 *res2 = md_lds_fft(other, res, ny, P.pz, P.tw, 1.0f);  // [y][z]
-  for (int idx = threadIdx.x; idx < ny * nz; idx += blockDim.x) {
-    const int y = idx / nz, z = idx - y * nz;
-    md_put_phi(phi + ((size_t)x * ny + y) * (nz + MD_PHI_PAD), z, nz, res2[y * nz + z].x);
-  }
+  float2 *plane = E.cgrid + (size_t)x * ny * nzc;
+  md_ext_lines columns{plane, plane, (size_t)nzc};
+  float2 *res = md_fft(a, b, nullptr, 0, 0, false, columns, nzc, P.py, twy, 1.0f);  // [kz][y]
+  md_ext_potential rows{res, 1, md_pitch(ny), E.phi + (size_t)x * ny * (nz + MD_PHI_PAD), nz, nzc};
+  float2 *free_buffer = res == a ? b : a;
+  // the rows' first stage reads res through `rows`, so it writes the other
+  md_fft(free_buffer, res, nullptr, 0, 0, true, rows, ny, P.pz, twz, 1.0f);
 }
 
 // Every atom's force, one thread per slot of the nonbonded list's spatial
@@ -831,7 +865,7 @@ void md_pme_group_setup(md_group *g) {
   int mx = 0, my = 0, mz = 0;
   for (md_system *s : g->reps) {
     bool on = s->has_nonbonded;
-    int nx = s->pme_nx, ny = s->pme_ny, nz = s->pme_nz, kzb = (s->pme_nzc + PME_BATCH - 1) / PME_BATCH;
+    int nx = s->pme_nx, ny = s->pme_ny, nz = s->pme_nz, kzb = md_kz_runs(s->pme_nzc);
     spread.push_back(on ? s->nb.nslots / 64 : 0);
     zrows.push_back(on ? (nx * ny + PME_BATCH - 1) / PME_BATCH : 0);
     ylines.push_back(on ? nx * kzb : 0);
@@ -850,17 +884,20 @@ void md_pme_group_setup(md_group *g) {
   G->xlines = md_make_launch(g, xlines);
   G->gather = md_make_launch(g, gather);
   G->planes = md_make_launch(g, planes);
-  G->lyz = sizeof(float2) * 2 * (size_t)my * mz;
-  G->fused_yz = G->lyz <= 64 * 1024;  // up to 64^3 meshes
-  G->lz = sizeof(float2) * 2 * PME_BATCH * mz;
-  G->ly = sizeof(float2) * 2 * PME_BATCH * my;
-  G->lx = sizeof(float2) * 2 * PME_BATCH * mx;
-  size_t lds = std::max(G->lz, std::max(G->ly, G->lx));
-  if (lds > 64 * 1024) {
-    for (auto *k : {(const void *)k_pme_z_forward, (const void *)k_pme_y, (const void *)k_pme_x_convolve<true>,
-                    (const void *)k_pme_x_convolve<false>, (const void *)k_pme_z_inverse})
-      MD_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  }
+  // planes of up to about 64^2 in LDS, two workgroups to a CU
+  G->lyz = sizeof(float2) * (2 * (size_t)md_plane_buffer(my, mz) + my + mz);
+  G->fused_yz = G->lyz <= 68 * 1024;
+  G->lz = sizeof(float2) * (2 * PME_BATCH * md_pitch(mz) + mz);
+  G->ly = sizeof(float2) * (2 * PME_BATCH * md_pitch(my) + my);
+  G->lx = sizeof(float2) * (2 * PME_BATCH * md_pitch(mx) + mx);
+  auto allow = [](std::initializer_list<const void *> kernels, size_t lds) {
+    if (lds > 64 * 1024)
+      for (auto *k : kernels) MD_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  };
+  allow({(const void *)k_pme_z_forward, (const void *)k_pme_z_inverse}, G->lz);
+  allow({(const void *)k_pme_y}, G->ly);
+  allow({(const void *)k_pme_x_convolve<true>, (const void *)k_pme_x_convolve<false>}, G->lx);
+  if (G->fused_yz) allow({(const void *)k_pme_yz_forward, (const void *)k_pme_yz_inverse}, G->lyz);
   G->table = md_group_alloc<md_pme_table>(g, g->reps.size());
   md_pme_group_refresh(g);
 }
@@ -900,7 +937,7 @@ void md_pme(md_group *g, bool energy) {
   k_pme_spread<<<G.spread.total, MD_SPREAD_THREADS, 0, st>>>(T, G.spread.map);
   md_mark(g, MD_PHASE_FFT);
   if (G.fused_yz) {
-    k_pme_yz_forward<<<G.planes.total, 256, G.lyz, st>>>(T, G.planes.map);
+    k_pme_yz_forward<<<G.planes.total, MD_PLANE_THREADS, G.lyz, st>>>(T, G.planes.map);
   } else {
     k_pme_z_forward<<<G.zrows.total, 256, G.lz, st>>>(T, G.zrows.map);
     k_pme_y<<<G.ylines.total, 256, G.ly, st>>>(T, G.ylines.map, -1.0f);
@@ -910,7 +947,7 @@ void md_pme(md_group *g, bool energy) {
   else
     k_pme_x_convolve<false><<<G.xlines.total, 256, G.lx, st>>>(T, G.xlines.map);
   if (G.fused_yz) {
-    k_pme_yz_inverse<<<G.planes.total, 256, G.lyz, st>>>(T, G.planes.map);
+    k_pme_yz_inverse<<<G.planes.total, MD_PLANE_THREADS, G.lyz, st>>>(T, G.planes.map);
   } else {
     k_pme_y<<<G.ylines.total, 256, G.ly, st>>>(T, G.ylines.map, 1.0f);
     k_pme_z_inverse<<<G.zrows.total, 256, G.lz, st>>>(T, G.zrows.map);
