@@ -621,12 +621,12 @@ void md_mark(md_group *g, int phase) {
 static void launch_step(md_group *g) {
   const bool nb = g->nb != nullptr;
   md_mark(g, MD_PHASE_PROLOGUE);
-  md_step_prologue(g, true);
   if (nb) {
-    md_mark(g, MD_PHASE_BUILD);
-    md_nb_build(g);
+    md_nb_build(g, true);
     md_mark(g, MD_PHASE_PACK);
     md_nb_pairs(g, false);
+  } else {
+    md_step_prologue(g, true);
   }
   md_mark(g, MD_PHASE_BONDED);
   md_bonded(g, false);
@@ -812,10 +812,11 @@ static void evaluate(md_system *s, double *forces, double *groups, double *total
     MD_HIP(hipMemsetAsync(&s->ctl->pair_census, 0, sizeof(int64_t), s->stream));
     MD_HIP(hipMemsetAsync(&s->ctl->pair_blocks, 0, sizeof(int64_t), s->stream));
   }
-  md_step_prologue(grp, false);
   if (s->has_nonbonded) {
-    md_nb_build(grp);
+    md_nb_build(grp, false);
     md_nb_pairs(grp, true);
+  } else {
+    md_step_prologue(grp, false);
   }
   md_bonded(grp, true);
   if (s->has_nonbonded)

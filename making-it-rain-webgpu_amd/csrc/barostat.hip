@@ -206,10 +206,11 @@ __global__ void k_baro_restore(const md_baro_dev *B, int64_t *pos, const int64_t
 
 // the step's force kernels with energies on, into the energy slots
 static void baro_energy(md_group *g, bool nb) {
-  md_step_prologue(g, false);
   if (nb) {
-    md_nb_build(g);
+    md_nb_build(g, false);
     md_nb_pairs(g, true);
+  } else {
+    md_step_prologue(g, false);
   }
   md_bonded(g, true);
   if (nb)

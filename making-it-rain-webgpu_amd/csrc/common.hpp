@@ -227,6 +227,14 @@ __device__ inline int64_t md_wave_sum_i64(int64_t v) {
   return v;
 }
 
+// Raise a shared word to a non-negative float (they order as their bits).  Most
+// callers find it high enough already and leave it: thousands of waves with an
+// atomic each on one word would queue there.
+__device__ inline void md_raise(uint32_t *word, float v) {
+  const uint32_t bits = __float_as_uint(v);
+  if (bits > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(word, bits);
+}
+
 __device__ inline void md_atomic_add_i64(int64_t *p, int64_t v) {
   atomicAdd(reinterpret_cast<unsigned long long *>(p), (unsigned long long)v);
 }

@@ -57,6 +57,26 @@ struct md_control {
                                    // cutoff, 2 a scaled position left the fixed-point range
 };
 
+// The start of a step, by one thread per replica: advance the device step
+// counter, latch the rebuild request (the displacement test's, or the host's),
+// clear the momentum slot this step's integrator fills (or, not advancing, the
+// energies an evaluation sums), and raise the group's status word when an
+// earlier step left an error in the control block.
+__device__ __forceinline__ void md_prologue(md_control *ctl, uint32_t *group_status, int64_t *energy, int advance) {
+  if (ctl->overflow | ctl->diverged | ctl->barostat_error) atomicOr(group_status, 1u);
+  if (advance) {
+    ctl->step_current = ctl->step_next;
+    ctl->step_next = ctl->step_next + 1;
+    const int64_t s = ctl->step_current;
+    for (int d = 0; d < 3; ++d) ctl->momentum[(s + 1) & 1][d] = 0;
+  } else {
+    for (int k = 0; k < MD_E_SLOTS; ++k) energy[k] = 0;
+  }
+  ctl->rebuild_active = ctl->rebuild_request[0] | ctl->force_pending;
+  ctl->rebuild_request[0] = 0;
+  ctl->force_pending = 0;
+}
+
 // The per-group energies of the energy slots and the host constants
 // (dispersion, self and net-charge terms), and their total -- the same on the
 // host (md_evaluate) and on the device (the barostat's Metropolis test).
@@ -241,10 +261,10 @@ struct md_system {
 
   // ---- neighbour list (buffers private to nonbonded.hip in nb_ext) -----
   md_nb_params nb{};
-  int *cell_rank = nullptr, *cell_count = nullptr, *cell_cursor = nullptr, *cell_start = nullptr;
+  int *cell_rank = nullptr, *cell_count = nullptr, *cell_start = nullptr;
   int *atom_cell = nullptr, *cell_member = nullptr;
   int *slot_atom = nullptr, *atom_slot = nullptr;
-  int64_t *atom_folded = nullptr, *build_pos = nullptr, *slot_offset = nullptr;
+  int64_t *build_pos = nullptr, *slot_offset = nullptr;
   float2 *slot_lj = nullptr;
   int4 *slot_xyzq = nullptr;      // pair-kernel frame coordinates + charge bits
   float4 *cluster_half = nullptr;
@@ -364,7 +384,7 @@ void md_nb_set_schedule(md_group *g, int seg_len, int waves);  // pair-kernel sc
 void md_nb_get_schedule(md_group *g, int *seg_len, int *waves);
 void md_nb_set_compact(md_group *g, bool compact);  // forces through the compacted pair schedule
 bool md_nb_get_compact(md_group *g);
-void md_nb_build(md_group *g);                  // rebuild kernels, gated per replica
+void md_nb_build(md_group *g, bool advance);    // the step's prologue, then the rebuild, gated per replica
 void md_nb_pairs(md_group *g, bool energy);
 void md_bonded(md_group *g, bool energy);       // bonded.hip
 void md_bonded_forces(md_group *g);             // the terms' forces alone (no NonbondedForce)

@@ -33,7 +33,7 @@ struct md_int_args {
   const float *mass;
   const int64_t *build_pos;
   md_control *ctl;
-  uint32_t *group_status;  // the launch group's error word (see k_step_prologue)
+  uint32_t *group_status;  // the launch group's error word (see md_prologue)
   int64_t *energy;         // [MD_E_SLOTS]
   int np;
   float dt, half_dt, inv_dt;
@@ -859,26 +859,10 @@ __global__ void __launch_bounds__(256) k_constrain(const md_int_args *__restrict
   }
 }
 
-// start of a step, one thread per replica: advance the device step counter,
-// latch the rebuild request (the displacement test's, or the host's),
-// clear the momentum slot this step's integrator fills (or, not advancing, the
-// energies an evaluation sums), and raise the group's status word when an earlier step left an error in the control block
+// the start of a step, where no other kernel runs it (md_nb_build)
 __global__ void k_step_prologue(const md_int_args *__restrict__ T, int R, int advance) {
   int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  md_control *ctl = T[r].ctl;
-  if (ctl->overflow | ctl->diverged | ctl->barostat_error) atomicOr(T[r].group_status, 1u);
-  if (advance) {
-    ctl->step_current = ctl->step_next;
-    ctl->step_next = ctl->step_next + 1;
-    int64_t s = ctl->step_current;
-    for (int d = 0; d < 3; ++d) ctl->momentum[(s + 1) & 1][d] = 0;
-  } else {
-    for (int k = 0; k < MD_E_SLOTS; ++k) T[r].energy[k] = 0;
-  }
-  ctl->rebuild_active = ctl->rebuild_request[0] | ctl->force_pending;
-  ctl->rebuild_request[0] = 0;
-  ctl->force_pending = 0;
+  if (r < R) md_prologue(T[r].ctl, T[r].group_status, T[r].energy, advance);
 }
 
 // momentum of the current velocities, into the slot the next step reads

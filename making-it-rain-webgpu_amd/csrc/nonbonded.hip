@@ -151,9 +151,9 @@ struct md_nb_args {
   md_pair_args P;
   const int64_t *pos;
   const int *cell_rank;
-  int *cell_count, *cell_start, *cell_cursor, *atom_cell, *cell_member;
+  int *cell_count, *cell_start, *atom_cell, *cell_member;
   int *slot_atom, *atom_slot;
-  int64_t *folded, *build_pos, *slot_offset, *cluster_center, *super_origin;
+  int64_t *build_pos, *slot_offset, *cluster_center, *super_origin;
   float4 *super_sphere;
   float2 *slot_lj;
   int4 *slot_xyzq;
@@ -163,6 +163,8 @@ struct md_nb_args {
   int4 *cluster_lo, *cluster_hi;
   int *totals;
   md_control *ctl;
+  uint32_t *group_status;
+  int64_t *energy;
 };
 
 // this block's replica entry and its block index inside the replica
@@ -191,31 +193,23 @@ __device__ __forceinline__ int md_frame_coord(int64_t v, bool &bad) {
   return (int)u;
 }
 
-// Fold each atom into the cell and bucket it (cell-list.wgsl:139-250).  The
-// fractional coordinate is computed in f64 from the exact fixed-point
-// position; the folding subtracts whole lattice vectors in Q32.32.
-__global__ void k_nb_assign(const md_nb_args *__restrict__ T, md_bmap map) {
-  int blk;
-  const md_nb_args &A = md_nb_entry(T, map, blk);
-  if (!A.ctl->rebuild_active) return;
+// Fold a position into the cell: the folded position (whole lattice vectors
+// subtracted in Q32.32) and its sorting cell's number along the cell walk.
+// The fractional coordinate is computed in f64 from the exact fixed-point
+// position (cell-list.wgsl:139-250).
+__device__ __forceinline__ int md_fold(const md_nb_args &A, const int64_t *x, int64_t *folded) {
   const md_build_ctx &c = A.c;
-  int i = blk * blockDim.x + threadIdx.x;
-  if (i >= c.n) return;
-  const int64_t *pos = A.pos;
-  int *atom_cell = A.atom_cell;
-  int64_t *folded = A.folded, *build_pos = A.build_pos;
-  int64_t x = pos[i], y = pos[c.np + i], z = pos[2 * c.np + i];
   const double s = 2.3283064365386963e-10;
-  double rx = (double)x * s, ry = (double)y * s, rz = (double)z * s;
+  double rx = (double)x[0] * s, ry = (double)x[1] * s, rz = (double)x[2] * s;
   const double *M = c.box.invd;
   double fa = rx * M[0] + ry * M[3] + rz * M[6];
   double fb = ry * M[4] + rz * M[7];
   double fc = rz * M[8];
   double na = floor(fa), nb = floor(fb), nc = floor(fc);
   int64_t ia = (int64_t)na, ib = (int64_t)nb, ic = (int64_t)nc;
-  int64_t fx = x - ia * c.box.fa[0] - ib * c.box.fb[0] - ic * c.box.fc[0];
-  int64_t fy = y - ib * c.box.fb[1] - ic * c.box.fc[1];
-  int64_t fz = z - ic * c.box.fc[2];
+  folded[0] = x[0] - ia * c.box.fa[0] - ib * c.box.fb[0] - ic * c.box.fc[0];
+  folded[1] = x[1] - ib * c.box.fb[1] - ic * c.box.fc[1];
+  folded[2] = x[2] - ic * c.box.fc[2];
   double ua = fa - na, ub = fb - nb, uc = fc - nc;
   int ga = min((int)(ua * c.gdim0), c.gdim0 - 1);
   int gb = min((int)(ub * c.gdim1), c.gdim1 - 1);
@@ -223,19 +217,37 @@ __global__ void k_nb_assign(const md_nb_args *__restrict__ T, md_bmap map) {
   ga = max(ga, 0);
   gb = max(gb, 0);
   gc = max(gc, 0);
-  int key = A.cell_rank[(ga * c.gdim1 + gb) * c.gdim2 + gc];
-  atom_cell[i] = key;
-  atomicAdd(&A.cell_count[key], 1);
-  folded[i] = fx;
-  folded[c.np + i] = fy;
-  folded[2 * c.np + i] = fz;
-  build_pos[i] = x;
-  build_pos[c.np + i] = y;
-  build_pos[2 * c.np + i] = z;
+  return A.cell_rank[(ga * c.gdim1 + gb) * c.gdim2 + gc];
+}
+
+// The start of a rebuild, by one thread per replica
+__device__ __forceinline__ void md_rebuild_begins(md_control *ctl) {
+  ctl->rebuilds += 1;
+  ctl->max_disp2_bits[0] = 0;
+  ctl->cluster_radius_bits = 0;
+  ctl->super_radius_bits = 0;
+}
+
+// Bucket each atom; its number among its cell's arrivals goes to atom_slot
+// until k_nb_rank gives it its slot.
+__global__ void k_nb_assign(const md_nb_args *__restrict__ T, md_bmap map) {
+  int blk;
+  const md_nb_args &A = md_nb_entry(T, map, blk);
+  if (!A.ctl->rebuild_active) return;
+  const md_build_ctx &c = A.c;
+  int i = blk * blockDim.x + threadIdx.x;
+  if (i >= c.n) return;
+  const int64_t x[3] = {A.pos[i], A.pos[c.np + i], A.pos[2 * c.np + i]};
+  int64_t folded[3];
+  const int key = md_fold(A, x, folded);
+  A.atom_cell[i] = key;
+  A.atom_slot[i] = atomicAdd(&A.cell_count[key], 1);
+  for (int d = 0; d < 3; ++d) A.build_pos[d * c.np + i] = x[d];
 }
 
 // Exclusive scan by one workgroup of 1024 threads over `count` values; the
-// total lands at out[count].  `in` may alias `out`.  Zeroes `clear` if given.
+// total lands at out[count].  `in` may alias `out` or `clear`, which is zeroed
+// if given; all three are 16-byte aligned.
 // A pass takes MD_SCAN_ITEMS consecutive values per thread, scanned by wave
 // shuffles and once across the 16 waves, so a long scan is a few passes over
 // contiguous memory (85k cells: 157 us with one long run of values per thread,
@@ -248,8 +260,15 @@ __device__ void md_block_scan(const int *in, int *out, int count, int *clear) {
   for (int base = 0; base < count; base += 1024 * MD_SCAN_ITEMS) {
     const int at = base + t * MD_SCAN_ITEMS;
     int v[MD_SCAN_ITEMS], sum = 0;
+    const bool whole = at + MD_SCAN_ITEMS <= count;  // by 16-byte loads and stores
+    if (whole) {
+      const int4 *p = reinterpret_cast<const int4 *>(in + at);
+      const int4 x = p[0], y = p[1];
+      v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w, v[4] = y.x, v[5] = y.y, v[6] = y.z, v[7] = y.w;
+    } else {
 #pragma unroll
-    for (int k = 0; k < MD_SCAN_ITEMS; ++k) v[k] = at + k < count ? in[at + k] : 0;
+      for (int k = 0; k < MD_SCAN_ITEMS; ++k) v[k] = at + k < count ? in[at + k] : 0;
+    }
 #pragma unroll
     for (int k = 0; k < MD_SCAN_ITEMS; ++k) sum += v[k];
     int incl = sum;
@@ -268,10 +287,22 @@ __device__ void md_block_scan(const int *in, int *out, int count, int *clear) {
     int run = before + incl - sum;
 #pragma unroll
     for (int k = 0; k < MD_SCAN_ITEMS; ++k) {
-      if (at + k >= count) break;
-      out[at + k] = run;
-      run += v[k];
-      if (clear) clear[at + k] = 0;
+      const int u = v[k];
+      v[k] = run;
+      run += u;
+    }
+    if (whole) {
+      int4 *p = reinterpret_cast<int4 *>(out + at), *z = reinterpret_cast<int4 *>(clear + at);
+      p[0] = make_int4(v[0], v[1], v[2], v[3]);
+      p[1] = make_int4(v[4], v[5], v[6], v[7]);
+      if (clear) z[0] = z[1] = make_int4(0, 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int k = 0; k < MD_SCAN_ITEMS; ++k) {
+        if (at + k >= count) break;
+        out[at + k] = v[k];
+        if (clear) clear[at + k] = 0;
+      }
     }
     carry += total;
     __syncthreads();  // the next pass rewrites wave_sum
@@ -283,21 +314,9 @@ __device__ void md_block_scan(const int *in, int *out, int count, int *clear) {
 __global__ void __launch_bounds__(1024) k_nb_scan_cells(const md_nb_args *__restrict__ T, md_bmap map) {
   int blk;
   const md_nb_args &A = md_nb_entry(T, map, blk);
-  md_control *ctl = A.ctl;
-  if (!ctl->rebuild_active) return;
-  int ncells = A.c.ncells;
-  md_block_scan(A.cell_count, A.cell_start, ncells, nullptr);
-  __syncthreads();
-  for (int k = threadIdx.x; k < ncells; k += 1024) {
-    A.cell_count[k] = 0;
-    A.cell_cursor[k] = 0;
-  }
-  if (threadIdx.x == 0) {
-    ctl->rebuilds += 1;
-    ctl->max_disp2_bits[0] = 0;
-    ctl->cluster_radius_bits = 0;
-    ctl->super_radius_bits = 0;
-  }
+  if (!A.ctl->rebuild_active) return;
+  md_block_scan(A.cell_count, A.cell_start, A.c.ncells, A.cell_count);
+  if (threadIdx.x == 0) md_rebuild_begins(A.ctl);
 }
 
 __global__ void k_nb_scatter(const md_nb_args *__restrict__ T, md_bmap map) {
@@ -306,9 +325,7 @@ __global__ void k_nb_scatter(const md_nb_args *__restrict__ T, md_bmap map) {
   if (!A.ctl->rebuild_active) return;
   int i = blk * blockDim.x + threadIdx.x;
   if (i >= A.c.n) return;
-  int key = A.atom_cell[i];
-  int at = A.cell_start[key] + atomicAdd(&A.cell_cursor[key], 1);
-  A.cell_member[at] = i;
+  A.cell_member[A.cell_start[A.atom_cell[i]] + A.atom_slot[i]] = i;
 }
 
 // Deterministic order inside a cell: rank by atom index over the cell's
@@ -328,101 +345,189 @@ __global__ void k_nb_rank(const md_nb_args *__restrict__ T, md_bmap map) {
   A.atom_slot[i] = slot;
 }
 
-// Per 8-atom cluster: bounding box of the folded build positions.  Per
-// 64-atom super-cluster: a frame origin, and for each slot the fixed-point
-// offset that takes a current position to f32 coordinates in that frame.
-__global__ void k_nb_clusters(const md_nb_args *__restrict__ T, md_bmap map) {
-  int blk;
-  const md_nb_args &A = md_nb_entry(T, map, blk);
-  md_control *ctl = A.ctl;
-  if (!ctl->rebuild_active) return;
+// One wave per super-cluster S, lane = slot, `a` its atom (or -1): the bounding
+// boxes of its 8-atom clusters over the folded positions, S's frame origin
+// (the centre of its bounding box) and radius, and for each slot the
+// fixed-point offset that takes a current position to coordinates in that
+// frame.  Raises `most` to S's largest cluster radius and its own radius.
+struct md_radii {
+  float cluster, super;
+};
+__device__ __forceinline__ void md_super_frame(const md_nb_args &A, int S, int a, md_radii &most) {
   const md_build_ctx &c = A.c;
-  const int *slot_atom = A.slot_atom;
-  const int64_t *folded = A.folded, *build_pos = A.build_pos;
-  const float4 *atom_param = A.atom_param;
-  int64_t *cluster_center = A.cluster_center, *super_origin = A.super_origin, *slot_offset = A.slot_offset;
-  float4 *super_sphere = A.super_sphere;
-  float4 *cluster_half = A.cluster_half;
-  float2 *slot_lj = A.slot_lj;
-  // one thread per cluster; the 8 threads of a super-cluster cooperate
-  int k = blk * blockDim.x + threadIdx.x;  // cluster index
-  int lane = threadIdx.x & 63;
-  bool live = k < c.nclusters;
-  int64_t lo[3] = {INT64_MAX, INT64_MAX, INT64_MAX}, hi[3] = {INT64_MIN, INT64_MIN, INT64_MIN};
-  if (live) {
-    for (int q = 0; q < MD_CLUSTER; ++q) {
-      int a = slot_atom[k * MD_CLUSTER + q];
-      if (a < 0) continue;
-      for (int d = 0; d < 3; ++d) {
-        int64_t v = folded[d * c.np + a];
-        lo[d] = min(lo[d], v);
-        hi[d] = max(hi[d], v);
-      }
-    }
+  const int lane = threadIdx.x & 63, slot = S * MD_SUPER + lane, k = slot / MD_CLUSTER;
+  int64_t x[3] = {0, 0, 0}, folded[3] = {0, 0, 0};
+  if (a >= 0) {
+    for (int d = 0; d < 3; ++d) x[d] = A.pos[d * c.np + a];
+    md_fold(A, x, folded);
   }
-  int64_t cen[3];
-  float half[3];
+  int64_t lo[3], hi[3], slo[3], shi[3];
   for (int d = 0; d < 3; ++d) {
-    cen[d] = live && lo[d] <= hi[d] ? lo[d] + ((hi[d] - lo[d]) >> 1) : 0;
-    half[d] = live && lo[d] <= hi[d] ? md_from_fixed(hi[d] - lo[d]) * 0.5f : 0.0f;
+    int64_t l = a >= 0 ? folded[d] : INT64_MAX, h = a >= 0 ? folded[d] : INT64_MIN;
+    for (int off = 1; off < 8; off <<= 1) {
+      l = min(l, (int64_t)__shfl_xor(l, off, 64));
+      h = max(h, (int64_t)__shfl_xor(h, off, 64));
+    }
+    lo[d] = l;
+    hi[d] = h;
+    for (int off = 8; off < 64; off <<= 1) {
+      l = min(l, (int64_t)__shfl_xor(l, off, 64));
+      h = max(h, (int64_t)__shfl_xor(h, off, 64));
+    }
+    slo[d] = l;
+    shi[d] = h;
+  }
+  const bool live = lo[0] <= hi[0];  // the cluster has an atom
+  int64_t cen[3], origin[3];
+  float half[3], r2 = 0.0f;
+  for (int d = 0; d < 3; ++d) {
+    cen[d] = live ? lo[d] + ((hi[d] - lo[d]) >> 1) : 0;
+    half[d] = live ? md_from_fixed(hi[d] - lo[d]) * 0.5f : 0.0f;
+    origin[d] = slo[d] + ((shi[d] - slo[d]) >> 1);  // S holds at least one atom
+    const float h = 0.5f * md_from_fixed(shi[d] - slo[d]);
+    r2 += h * h;
   }
   float radius = sqrtf(half[0] * half[0] + half[1] * half[1] + half[2] * half[2]);
-  if (live) {
-    for (int d = 0; d < 3; ++d) cluster_center[d * c.nclusters + k] = cen[d];
-    cluster_half[k] = make_float4(half[0], half[1], half[2], 0.0f);
+  for (int off = 8; off < 64; off <<= 1) radius = fmaxf(radius, __shfl_xor(radius, off, 64));
+  // rounded up a little: the list test that uses it must stay conservative
+  const float srad = sqrtf(r2) * 1.0001f + 1e-4f;
+  if (lane == 0) {
+    for (int d = 0; d < 3; ++d) A.super_origin[d * c.nsuper + S] = origin[d];
+    A.super_sphere[S] = make_float4(md_from_fixed(origin[0]), md_from_fixed(origin[1]), md_from_fixed(origin[2]), srad);
+  }
+  most.cluster = fmaxf(most.cluster, radius);
+  most.super = fmaxf(most.super, srad);
+  if ((lane & 7) == 0 && k < c.nclusters) {
+    for (int d = 0; d < 3; ++d) A.cluster_center[d * c.nclusters + k] = cen[d];
+    A.cluster_half[k] = make_float4(half[0], half[1], half[2], 0.0f);
     A.L.j_count[k] = 0;
   }
-  // the largest cluster radius (non-negative floats order as their bits):
-  // reduced over the wave first, one atomic per wave on the shared word
-  // rather than one per cluster, which all queue on one address
-  {
-    float rmax = live ? radius : -1.0f;
-    for (int off = 32; off > 0; off >>= 1) rmax = fmaxf(rmax, __shfl_xor(rmax, off, 64));
-    if (lane == 0 && rmax >= 0.0f) atomicMax(&ctl->cluster_radius_bits, __float_as_uint(rmax));
+  for (int d = 0; d < 3; ++d) A.slot_offset[d * c.nslots + slot] = a >= 0 ? (x[d] - folded[d]) + origin[d] : 0;
+  float2 lj = make_float2(0.0f, 0.0f);
+  if (a >= 0) {
+    const float4 p = A.atom_param[a];
+    lj = make_float2(p.y * MD_PAIR_S_SCALE, p.z * MD_PAIR_E_SCALE);
   }
-  // super-cluster frame: the bounding box centre over its 8 clusters
-  int64_t slo[3], shi[3];
-  for (int d = 0; d < 3; ++d) {
-    int64_t a = lo[d], b = hi[d];
-    for (int off = 1; off < 8; off <<= 1) {
-      a = min(a, (int64_t)__shfl_xor(a, off, 64));
-      b = max(b, (int64_t)__shfl_xor(b, off, 64));
+  A.slot_lj[slot] = lj;
+}
+
+// The workgroup's radii into the control words: one atomic at most per word.
+__device__ __forceinline__ void md_raise_radii(md_control *ctl, const md_radii &mine, md_radii *waves) {
+  const int wave = threadIdx.x >> 6, count = blockDim.x >> 6;
+  if ((threadIdx.x & 63) == 0) waves[wave] = mine;  // the lanes of a wave agree
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  md_radii most = waves[0];
+  for (int w = 1; w < count; ++w) {
+    most.cluster = fmaxf(most.cluster, waves[w].cluster);
+    most.super = fmaxf(most.super, waves[w].super);
+  }
+  md_raise(&ctl->cluster_radius_bits, most.cluster);
+  md_raise(&ctl->super_radius_bits, most.super);
+}
+
+#define MD_FRAME_WAVES 4
+__global__ void __launch_bounds__(64 * MD_FRAME_WAVES) k_nb_clusters(const md_nb_args *__restrict__ T, md_bmap map) {
+  __shared__ md_radii waves[MD_FRAME_WAVES];
+  int blk;
+  const md_nb_args &A = md_nb_entry(T, map, blk);
+  if (!A.ctl->rebuild_active) return;
+  const int S = blk * MD_FRAME_WAVES + (int)(threadIdx.x >> 6);
+  md_radii most{0.0f, 0.0f};
+  if (S < A.c.nsuper) md_super_frame(A, S, A.slot_atom[S * MD_SUPER + (int)(threadIdx.x & 63)], most);
+  md_raise_radii(A.ctl, most, waves);
+}
+
+// The step's prologue and, for a replica that rebuilds, the whole cell sort in
+// one workgroup: launch groups of small replicas, whose step is a chain of
+// launches (4.5 us each, whether or not a replica rebuilds).  Cells' counts and
+// members stay in LDS, an atom's cell and arrival in registers; the result is
+// that of k_nb_assign to k_nb_clusters.  At
+// 2,168 atoms the five launches and the prologue took 31 us of a step on
+// average, this takes 8.  At 31k atoms one workgroup would take longer over a
+// rebuild than the launches it saves.
+#define MD_SORT_THREADS 1024
+#define MD_SORT_ITEMS 12  // atoms a thread holds
+#define MD_SORT_CELLS 12288
+__global__ void __launch_bounds__(MD_SORT_THREADS) k_nb_sort(const md_nb_args *__restrict__ T, int advance, int cells) {
+  extern __shared__ int sort_lds[];
+  __shared__ int active, wave_sum[16];
+  const md_nb_args &A = T[blockIdx.x];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (t == 0) {
+    md_prologue(A.ctl, A.group_status, A.energy, advance);
+    active = (int)A.ctl->rebuild_active;
+    if (active) md_rebuild_begins(A.ctl);
+  }
+  __syncthreads();
+  if (!active) return;
+  const md_build_ctx &c = A.c;
+  int *count = sort_lds, *member = sort_lds + cells;
+  for (int k = t; k <= c.ncells; k += MD_SORT_THREADS) count[k] = 0;
+  __syncthreads();
+  int key[MD_SORT_ITEMS], at[MD_SORT_ITEMS];
+#pragma unroll
+  for (int u = 0; u < MD_SORT_ITEMS; ++u) {
+    const int i = u * MD_SORT_THREADS + t;
+    key[u] = -1;
+    at[u] = 0;
+    if (i < c.n) {
+      const int64_t x[3] = {A.pos[i], A.pos[c.np + i], A.pos[2 * c.np + i]};
+      int64_t folded[3];
+      key[u] = md_fold(A, x, folded);
+      at[u] = atomicAdd(&count[key[u]], 1);
+      for (int d = 0; d < 3; ++d) A.build_pos[d * c.np + i] = x[d];
     }
-    slo[d] = a;
-    shi[d] = b;
   }
-  int s = k / 8;
-  int64_t origin[3];
-  for (int d = 0; d < 3; ++d) origin[d] = slo[d] <= shi[d] ? slo[d] + ((shi[d] - slo[d]) >> 1) : 0;
-  float srad = -1.0f;
-  if (live && (lane & 7) == 0 && s < c.nsuper) {
-    float r2 = 0.0f;
-    for (int d = 0; d < 3; ++d) {
-      super_origin[d * c.nsuper + s] = origin[d];
-      float h = 0.5f * md_from_fixed(shi[d] - slo[d]);
-      r2 += h * h;
+  __syncthreads();
+  // exclusive scan of the counts in place, count[ncells] the total
+  const int per = (c.ncells + MD_SORT_THREADS) / MD_SORT_THREADS;  // covers ncells + 1
+  int sum = 0;
+  for (int k = t * per; k < min((t + 1) * per, c.ncells + 1); ++k) sum += count[k];
+  int incl = sum;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += u;
+  }
+  if (lane == 63) wave_sum[wave] = incl;
+  __syncthreads();
+  int run = incl - sum;
+  for (int w = 0; w < wave; ++w) run += wave_sum[w];
+  for (int k = t * per; k < min((t + 1) * per, c.ncells + 1); ++k) {
+    const int v = count[k];
+    count[k] = run;
+    run += v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < MD_SORT_ITEMS; ++u)
+    if (key[u] >= 0) member[count[key[u]] + at[u]] = u * MD_SORT_THREADS + t;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < MD_SORT_ITEMS; ++u)
+    if (key[u] >= 0) {
+      const int i = u * MD_SORT_THREADS + t, b = count[key[u]], e = count[key[u] + 1];
+      int rank = 0;
+      for (int k = b; k < e; ++k) rank += member[k] < i;
+      at[u] = b + rank;
     }
-    // rounded up a little: the list test that uses it must stay conservative
-    srad = sqrtf(r2) * 1.0001f + 1e-4f;
-    super_sphere[s] = make_float4(md_from_fixed(origin[0]), md_from_fixed(origin[1]), md_from_fixed(origin[2]), srad);
-  }
-  // the largest super-cluster radius, one atomic per wave as above
-  for (int off = 32; off > 0; off >>= 1) srad = fmaxf(srad, __shfl_xor(srad, off, 64));
-  if (lane == 0 && srad >= 0.0f) atomicMax(&ctl->super_radius_bits, __float_as_uint(srad));
-  if (!live) return;
-  for (int q = 0; q < MD_CLUSTER; ++q) {
-    int slot = k * MD_CLUSTER + q;
-    int a = slot_atom[slot];
-    if (a < 0) {
-      for (int d = 0; d < 3; ++d) slot_offset[d * c.nslots + slot] = 0;
-      slot_lj[slot] = make_float2(0.0f, 0.0f);
-      continue;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < MD_SORT_ITEMS; ++u)
+    if (key[u] >= 0) {
+      const int i = u * MD_SORT_THREADS + t;
+      member[at[u]] = i;
+      A.slot_atom[at[u]] = i;
+      A.atom_slot[i] = at[u];
     }
-    for (int d = 0; d < 3; ++d)
-      slot_offset[d * c.nslots + slot] = (build_pos[d * c.np + a] - folded[d * c.np + a]) + origin[d];
-    float4 p = atom_param[a];
-    slot_lj[slot] = make_float2(p.y * MD_PAIR_S_SCALE, p.z * MD_PAIR_E_SCALE);
+  __syncthreads();
+  __shared__ md_radii waves[MD_SORT_THREADS / 64];
+  md_radii most{0.0f, 0.0f};
+  for (int S = wave; S < c.nsuper; S += MD_SORT_THREADS / 64) {
+    const int slot = S * MD_SUPER + lane;
+    md_super_frame(A, S, slot < c.n ? member[slot] : -1, most);
   }
+  md_raise_radii(A.ctl, most, waves);
 }
 
 // squared distance between cluster boxes whose centres are d apart (nm, f32)
@@ -548,8 +653,8 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
     float ox = md_from_fixed(jx + shx - V.ox), oy = md_from_fixed(jy + shy - V.oy), oz = md_from_fixed(jz + shz - V.oz);
     if (ox * ox + oy * oy + oz * oz >= reach2) return;
     bool zero = shx == 0 && shy == 0 && shz == 0;
-    int imask = 0, self = 0;
-#pragma unroll 2
+    int imask = 0, self = 0, border = 0;
+#pragma unroll 4
     for (int q = 0; q < 8; ++q) {
       int I = V.first + q;
       // within S, J >= I only; a cluster with its own images keeps one of
@@ -558,16 +663,19 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
       if (q < V.nlocal && (!own || J >= I) && !(J == I && !zero && code < 0)) {
         const float4 cc = V.box->cc[q];
         const float near2 = md_box_distance2(ox - cc.x, oy - cc.y, oz - cc.z, V.box->ch[q], jh);
-        bool within = near2 < c.list_cutoff2;
-        if (fabsf(near2 - c.list_cutoff2) < 1e-5f)
-          within = md_box_distance2(md_from_fixed(jx + shx - V.box->cx[q]), md_from_fixed(jy + shy - V.box->cy[q]),
-                                    md_from_fixed(jz + shz - V.box->cz[q]), V.box->ch[q], jh) < c.list_cutoff2;
-        if (within) {
-          imask |= 1 << q;
-          if (J == I && zero) self |= 1 << q;
-        }
+        if (near2 < c.list_cutoff2) imask |= 1 << q;
+        if (fabsf(near2 - c.list_cutoff2) < 1e-5f) border |= 1 << q;
+        if (J == I && zero) self |= 1 << q;
       }
     }
+    for (; border; border &= border - 1) {
+      const int q = __ffs(border) - 1;
+      const bool within =
+          md_box_distance2(md_from_fixed(jx + shx - V.box->cx[q]), md_from_fixed(jy + shy - V.box->cy[q]),
+                           md_from_fixed(jz + shz - V.box->cz[q]), V.box->ch[q], jh) < c.list_cutoff2;
+      imask = within ? imask | 1 << q : imask & ~(1 << q);
+    }
+    self &= imask;
     if (imask) emit(imask, self, shx, shy, shz);
   });
 }
@@ -788,8 +896,8 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
   }
 }
 
-// Starts of every super-cluster's segments, the segments themselves, the
-// totals, and the starts of the transposed list.  One workgroup per replica.
+// Starts of every super-cluster's segments, the totals, and the starts of the
+// transposed list.  One workgroup per replica.
 __global__ void __launch_bounds__(1024) k_nb_starts(const md_nb_args *__restrict__ T, md_bmap map) {
   int blk;
   const md_nb_args &A = md_nb_entry(T, map, blk);
@@ -819,17 +927,10 @@ __global__ void __launch_bounds__(1024) k_nb_starts(const md_nb_args *__restrict
     totals[0] = entries;
     totals[1] = min(segs, segment_capacity);
   }
-  // 16 threads write one super-cluster's segments
-  for (int s = threadIdx.x >> 4; s < nsuper; s += 64) {
-    const int b = s * region, e = b + min(L.super_count[s], region), sg = L.super_segs[s];
-    for (int k = threadIdx.x & 15; b + k * len < e; k += 16) {
-      if (sg + k >= segment_capacity) break;
-      L.segments[sg + k] = make_int4(s, b + k * len, min(b + k * len + len, e), 0);
-    }
-  }
 }
 
-// Exclusion masks and the transposed list, one workgroup per super-cluster S.
+// Exclusion masks, the transposed list and the segments, one workgroup per
+// super-cluster S.
 // An entry's mask for S's cluster q has bit (i = l/8, j = l%8) set when the
 // pair interacts: cleared for padding, for the lower triangle of a cluster
 // with its own zero image, and for every excluded pair (the CSR holds both
@@ -860,6 +961,12 @@ __global__ void __launch_bounds__(MD_MASK_THREADS) k_nb_masks(const md_nb_args *
   const int a = slot_atom[slot];
   const int q = (slot >> 3) & 7, il = slot & 7;
   const int xb = a >= 0 ? excl_start[a] : 0, xe = a >= 0 ? excl_start[a + 1] : 0;
+  // S's segments
+  for (int k = threadIdx.x, first = L.super_segs[S]; k * c.seg_len < count; k += MD_MASK_THREADS) {
+    if (first + k >= c.segment_capacity) break;
+    const int b = k * c.seg_len;
+    L.segments[first + k] = make_int4(S, eb + b, eb + min(b + c.seg_len, count), 0);
+  }
   for (int t0 = 0; t0 < count; t0 += MD_MASK_TILE) {
     const int nt = min(MD_MASK_TILE, count - t0);
     for (int k = threadIdx.x; k < nt; k += MD_MASK_THREADS) {
@@ -1870,7 +1977,6 @@ void md_nb_setup(md_system *s) {
   s->cell_rank = md_alloc<int>(s, nb.ncells);
   MD_HIP(hipMemcpyAsync(s->cell_rank, rank.data(), sizeof(int) * nb.ncells, hipMemcpyHostToDevice, s->stream));
   s->cell_count = md_alloc<int>(s, nb.ncells);
-  s->cell_cursor = md_alloc<int>(s, nb.ncells);
   s->cell_start = md_alloc<int>(s, nb.ncells + 1);
   s->atom_cell = md_alloc<int>(s, np);
   s->cell_member = md_alloc<int>(s, np);
@@ -1879,7 +1985,6 @@ void md_nb_setup(md_system *s) {
   MD_HIP(hipMemcpyAsync(s->slot_atom, pad.data(), sizeof(int) * nb.nslots, hipMemcpyHostToDevice, s->stream));
   MD_HIP(hipStreamSynchronize(s->stream));
   s->atom_slot = md_alloc<int>(s, np);
-  s->atom_folded = md_alloc<int64_t>(s, 3 * (size_t)np);
   s->build_pos = md_alloc<int64_t>(s, 3 * (size_t)np);
   s->slot_offset = md_alloc<int64_t>(s, 3 * (size_t)nb.nslots);
   s->slot_lj = md_alloc<float2>(s, nb.nslots);
@@ -1979,7 +2084,7 @@ static md_build_ctx build_ctx(md_system *s) {
 }
 
 // one replica's table entry
-static md_nb_args nb_args(md_system *s, int seg_len) {
+static md_nb_args nb_args(md_group *g, md_system *s, int seg_len) {
   auto &B = nbuf(s);
   md_nb_args a{};
   a.c = build_ctx(s);
@@ -2031,12 +2136,10 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   a.cell_rank = s->cell_rank;
   a.cell_count = s->cell_count;
   a.cell_start = s->cell_start;
-  a.cell_cursor = s->cell_cursor;
   a.atom_cell = s->atom_cell;
   a.cell_member = s->cell_member;
   a.slot_atom = s->slot_atom;
   a.atom_slot = s->atom_slot;
-  a.folded = s->atom_folded;
   a.build_pos = s->build_pos;
   a.slot_offset = s->slot_offset;
   a.cluster_center = B.cluster_center;
@@ -2052,16 +2155,20 @@ static md_nb_args nb_args(md_system *s, int seg_len) {
   a.cluster_hi = B.cluster_hi;
   a.totals = B.totals;
   a.ctl = s->ctl;
+  a.group_status = g->status;
+  a.energy = s->energy;
   return a;
 }
 
 // a group's launch tables for the nonbonded kernels
 struct md_nb_group {
   md_nb_args *table = nullptr;  // [R], device
-  md_launch atoms, scan, clusters, supers, slots;
+  md_launch atoms, scan, frames, supers, slots;
   md_launch seg;                // the pair kernel's segment numbering
   int pair_grid = 1;
   int seg_len = MD_SEGMENT;
+  size_t sort_lds = 0;  // k_nb_sort's LDS, 0: the sort as separate passes
+  int sort_cells = 0;
   bool compact = false;  // forces through the compacted schedule
 };
 
@@ -2071,18 +2178,30 @@ void md_nb_group_setup(md_group *g) {
   auto *G = new md_nb_group();
   g->nb = G;
   const int R = (int)g->reps.size();
-  std::vector<int> atoms, one, clusters, supers, slots;
+  std::vector<int> atoms, one, frames, supers, slots;
+  int most_atoms = 0, most_cells = 0;
   for (md_system *s : g->reps) {
     auto &B = nbuf(s);
     atoms.push_back((s->n + 255) / 256);
     one.push_back(1);
-    clusters.push_back((s->nb.nclusters + 63) / 64);
+    most_atoms = std::max(most_atoms, s->n);
+    most_cells = std::max(most_cells, s->nb.ncells);
+    frames.push_back((B.nsuper + MD_FRAME_WAVES - 1) / MD_FRAME_WAVES);
     supers.push_back(B.nsuper);
     slots.push_back((s->nb.nslots + 255) / 256);
   }
   G->atoms = md_make_launch(g, atoms);
   G->scan = md_make_launch(g, one);
-  G->clusters = md_make_launch(g, clusters);
+  // one workgroup sorts a replica while its rebuild costs less than the four
+  // launches it saves on every step, which a rebuild comes every six or so of
+  G->sort_cells = most_cells + 1;
+  if (most_atoms <= MD_SORT_THREADS * MD_SORT_ITEMS && most_cells < MD_SORT_CELLS) {
+    G->sort_lds = sizeof(int) * (size_t)(G->sort_cells + most_atoms);
+    if (G->sort_lds > 60 * 1024)
+      MD_HIP(hipFuncSetAttribute((const void *)k_nb_sort, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)G->sort_lds));
+  }
+  G->frames = md_make_launch(g, frames);
   G->supers = md_make_launch(g, supers);
   G->slots = md_make_launch(g, slots);
   G->seg.map.start = md_group_alloc<int>(g, R + 1);
@@ -2120,7 +2239,7 @@ bool md_nb_get_compact(md_group *g) { return nbg(g).compact; }
 
 void md_nb_group_refresh(md_group *g) {
   std::vector<md_nb_args> host;
-  for (md_system *s : g->reps) host.push_back(nb_args(s, nbg(g).seg_len));
+  for (md_system *s : g->reps) host.push_back(nb_args(g, s, nbg(g).seg_len));
   MD_HIP(hipMemcpyAsync(nbg(g).table, host.data(), sizeof(md_nb_args) * host.size(), hipMemcpyHostToDevice,
                         g->stream));
   MD_HIP(hipStreamSynchronize(g->stream));
@@ -2145,15 +2264,22 @@ void md_nb_group_free(md_group *g) {
   g->nb = nullptr;
 }
 
-void md_nb_build(md_group *g) {
+void md_nb_build(md_group *g, bool advance) {
   auto &G = nbg(g);
   hipStream_t st = g->stream;
   const md_nb_args *T = G.table;
-  k_nb_assign<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
-  k_nb_scan_cells<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
-  k_nb_scatter<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
-  k_nb_rank<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
-  k_nb_clusters<<<G.clusters.total, 64, 0, st>>>(T, G.clusters.map);
+  if (G.sort_lds) {
+    md_mark(g, MD_PHASE_BUILD);
+    k_nb_sort<<<(int)g->reps.size(), MD_SORT_THREADS, G.sort_lds, st>>>(T, advance ? 1 : 0, G.sort_cells);
+  } else {
+    md_step_prologue(g, advance);
+    md_mark(g, MD_PHASE_BUILD);
+    k_nb_assign<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
+    k_nb_scan_cells<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
+    k_nb_scatter<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
+    k_nb_rank<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
+    k_nb_clusters<<<G.frames.total, 64 * MD_FRAME_WAVES, 0, st>>>(T, G.frames.map);
+  }
   md_mark(g, MD_PHASE_SEARCH);
   k_nb_list<<<G.supers.total, 64 * MD_LIST_WAVES, 0, st>>>(T, G.supers.map);
   k_nb_starts<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
