@@ -515,6 +515,10 @@ static void create(md_system *s, const md_system_desc *d, const md_run_options *
         int ci = R.cl_cons[k][c];
         int li = (int)(std::find(at.begin(), at.end(), d->constraint_p1[ci]) - at.begin());
         int lj = (int)(std::find(at.begin(), at.end(), d->constraint_p2[ci]) - at.begin());
+        if (std::min(li, lj) != 0 || std::max(li, lj) != c + 1)
+          s->star_clusters = 0;
+        else if (li != 0)
+          s->star_clusters = std::min(s->star_clusters, 1);
         double dist = d->constraint_distance[ci];
         int64_t bits;
         std::memcpy(&bits, &dist, 8);
@@ -1654,6 +1658,11 @@ md_err md_shake_counts(md_system *s, int64_t *passes, int64_t *clusters) {
   md_control c;
   MD_HIP(hipSetDevice(s->device));
   MD_HIP(hipMemcpy(&c, s->ctl, sizeof c, hipMemcpyDeviceToHost));
+  // the last step's are still in parts
+  for (int k = 0; k < MD_STEP_PARTS; ++k) {
+    c.shake_passes += c.part[k][3];
+    c.shake_clusters += c.part[k][4];
+  }
   if (passes) *passes = c.shake_passes;
   if (clusters) *clusters = c.shake_clusters;
   MD_API_END

@@ -34,6 +34,8 @@ void md_set_last_error(const std::string &message);
                      std::string(#call) + ": " + hipGetErrorString(e_));            \
   } while (0)
 
+#define MD_STEP_PARTS 16
+
 // Device-resident control words, read and written by the kernels of a step.
 struct md_control {
   int64_t step_current;            // the step being integrated (thermostat counter)
@@ -45,7 +47,7 @@ struct md_control {
   uint32_t max_disp2_bits[2];      // [0] worst squared displacement since the build
   uint32_t cluster_radius_bits;    // largest cluster bounding-box half diagonal (f32 bits)
   uint32_t super_radius_bits;      // largest super-cluster radius (f32 bits)
-  int64_t momentum[2][3];          // sum m v in Q32.32, by step parity
+  int64_t momentum[3];             // sum m v in Q32.32, of the velocities the step starts from
   int64_t pair_census;             // in-cutoff pairs, when counted
   uint32_t force_pending;          // the host asks for a rebuild at the next step
   uint32_t diverged;               // the integrator's constraint solve failed: bit 0 SHAKE did not
@@ -55,26 +57,44 @@ struct md_control {
   int64_t pair_blocks;             // 8x8 cluster-pair blocks evaluated, when counted
   uint32_t barostat_error;         // a barostat move failed: 1 the trial box is too small for the
                                    // cutoff, 2 a scaled position left the fixed-point range
+  // what the integrator's waves add to since the last prologue, a 64-byte line
+  // each: sum m v [3], SHAKE passes, cluster-steps
+  alignas(64) int64_t part[MD_STEP_PARTS][8];
 };
 
-// The start of a step, by one thread per replica: advance the device step
+// The start of a step, by one wave per replica: advance the device step
 // counter, latch the rebuild request (the displacement test's, or the host's),
-// clear the momentum slot this step's integrator fills (or, not advancing, the
-// energies an evaluation sums), and raise the group's status word when an
-// earlier step left an error in the control block.
+// add up the momentum and SHAKE counts the last step's integrator left in parts
+// (or, not advancing, clear the energies an evaluation sums), and raise the
+// group's status word when an earlier step left an error in the control block.
 __device__ __forceinline__ void md_prologue(md_control *ctl, uint32_t *group_status, int64_t *energy, int advance) {
-  if (ctl->overflow | ctl->diverged | ctl->barostat_error) atomicOr(group_status, 1u);
+  const int lane = threadIdx.x & 63;
   if (advance) {
-    ctl->step_current = ctl->step_next;
-    ctl->step_next = ctl->step_next + 1;
-    const int64_t s = ctl->step_current;
-    for (int d = 0; d < 3; ++d) ctl->momentum[(s + 1) & 1][d] = 0;
-  } else {
-    for (int k = 0; k < MD_E_SLOTS; ++k) energy[k] = 0;
+    int64_t v[5];
+    for (int k = 0; k < 5; ++k) {
+      v[k] = 0;
+      if (lane < MD_STEP_PARTS) {
+        v[k] = ctl->part[lane][k];
+        ctl->part[lane][k] = 0;
+      }
+      v[k] = md_wave_sum_i64(v[k]);
+    }
+    if (lane == 0) {
+      for (int d = 0; d < 3; ++d) ctl->momentum[d] = v[d];
+      ctl->shake_passes += v[3];
+      ctl->shake_clusters += v[4];
+      ctl->step_current = ctl->step_next;
+      ctl->step_next = ctl->step_next + 1;
+    }
+  } else if (lane < MD_E_SLOTS) {
+    energy[lane] = 0;
   }
-  ctl->rebuild_active = ctl->rebuild_request[0] | ctl->force_pending;
-  ctl->rebuild_request[0] = 0;
-  ctl->force_pending = 0;
+  if (lane == 0) {
+    if (ctl->overflow | ctl->diverged | ctl->barostat_error) atomicOr(group_status, 1u);
+    ctl->rebuild_active = ctl->rebuild_request[0] | ctl->force_pending;
+    ctl->rebuild_request[0] = 0;
+    ctl->force_pending = 0;
+  }
 }
 
 // The per-group energies of the energy slots and the host constants
@@ -302,6 +322,10 @@ struct md_system {
   int4 *ccl_cons = nullptr;      // [n][8] (local i, local j, f64 distance bits)
   int *free_atoms = nullptr;
   int max_cluster_atoms = 0;
+  // 1: in every cluster one atom is in all constraints, comes first, and the
+  // others follow in the order of their constraints; 2: and it is each
+  // constraint's first atom
+  int star_clusters = 2;
 
   // ---- learned SHAKE warm start ------------------------------------------
   const md_ws_net *ws_net = nullptr;  // the network the integrator runs, or none

@@ -6,8 +6,8 @@
 // (src/gpu/kernels/integrate.wgsl:90-203), `settle_cluster`,
 // `settle_velocities` (settle.wgsl:74-249), `shake_cluster`, `rattle_cluster`
 // (shake.wgsl:124-229) and `momentum`/`subtract_com` (reduce.wgsl:61-105).
-// Upstream runs these as seven dispatches per step; here one thread owns one
-// constraint cluster (a rigid water, a SHAKE cluster of at most 8 atoms, or
+// Upstream runs these as seven dispatches per step; here one launch does, and
+// one thread owns one constraint cluster (a rigid water, a SHAKE cluster of at most 8 atoms, or
 // a single unconstrained atom) and carries it through the whole step in
 // registers, so the phases need no global synchronisation between them.
 //
@@ -53,6 +53,7 @@ struct md_int_args {
   const int4 *ccl_cons;
   const int *free_atoms;
   int n_waters, n_ccl, n_free;
+  int blocks_ccl, blocks_water;  // workgroups of a step's clusters and waters
   int n;  // atoms
   // learned SHAKE warm start: the network (null: plain SHAKE), and the
   // sample ring a recording run fills with (features, multipliers)
@@ -244,9 +245,8 @@ __device__ __forceinline__ double md_fx(int64_t v) { return (double)v * 2.328306
 // RATTLE (src/reference/constraints.ts:195-243): Jacobi, along the current
 // bond vectors, divided by the reference squared length
 // (false: not converged within MD_MAX_CONSTRAINT_ITERATIONS passes)
-template <int MAXA>
-__device__ __forceinline__ bool md_rattle(const md_int_args &A, md_item<MAXA> &it, int nc, const int4 *cons) {
-  constexpr int MAXC = md_max_constraints<MAXA>::value;
+template <int MAXA, int MAXC>
+__device__ __forceinline__ bool md_rattle(const md_int_args &A, md_item<MAXA> &it, int nc, const int4 (&cons)[MAXC]) {
   double rv[MAXC][3], l2[MAXC], mu[MAXC];
   double v[MAXA][3];
 #pragma unroll
@@ -312,11 +312,10 @@ __device__ __forceinline__ bool md_rattle(const md_int_args &A, md_item<MAXA> &i
 // bond vectors, converged when |r'|^2 lies in [(1-t)^2, (1+t)^2] d^2.
 // *passes receives the update passes applied, or -1 when the cluster did not
 // converge within MD_MAX_CONSTRAINT_ITERATIONS.
-template <int MAXA>
-__device__ __forceinline__ void md_shake(const md_int_args &A, md_item<MAXA> &it, int nc, const int4 *cons,
+template <int MAXA, int MAXC>
+__device__ __forceinline__ void md_shake(const md_int_args &A, md_item<MAXA> &it, int nc, const int4 (&cons)[MAXC],
                                          bool warm = false, const float *lam0 = nullptr,
                                          double *lam_total = nullptr, int *passes = nullptr) {
-  constexpr int MAXC = md_max_constraints<MAXA>::value;
   double rv[MAXC][3], mu[MAXC], t2[MAXC];
   double t[MAXA][3], moved[MAXA][3];
 #pragma unroll
@@ -459,7 +458,10 @@ __device__ __forceinline__ void md_shake(const md_int_args &A, md_item<MAXA> &it
   if (passes) *passes = converged ? applied : -1;
   if (lam_total) {
 #pragma unroll
-    for (int c = 0; c < MAXC && c < MD_WS_MAXC; ++c) lam_total[c] = mu[c] == 0.0 ? 0.0 : total[c] / mu[c];
+    for (int c = 0; c < MD_WS_MAXC; ++c) {
+      lam_total[c] = 0.0;
+      if (c < MAXC) lam_total[c] = mu[c < MAXC ? c : 0] == 0.0 ? 0.0 : total[c < MAXC ? c : 0] / mu[c < MAXC ? c : 0];
+    }
   }
 }
 
@@ -471,8 +473,8 @@ __device__ __forceinline__ void md_shake(const md_int_args &A, md_item<MAXA> &it
 // constraints that share an atom: +-m_shared^-1 / sqrt(the two inverse-mass
 // sums) times the cosine between their reference vectors.  All invariant
 // under rotation and translation.
-template <int MAXA>
-__device__ __forceinline__ void md_ws_features(const md_item<MAXA> &it, int nc, const int4 *cons, float *f) {
+template <int MAXA, int MAXC>
+__device__ __forceinline__ void md_ws_features(const md_item<MAXA> &it, int nc, const int4 (&cons)[MAXC], float *f) {
 #pragma unroll
   for (int k = 0; k < MD_WS_F; ++k) f[k] = 0.0f;
   double rv[MD_WS_MAXC][3], d2[MD_WS_MAXC], isum[MD_WS_MAXC];
@@ -481,8 +483,8 @@ __device__ __forceinline__ void md_ws_features(const md_item<MAXA> &it, int nc, 
   for (int c = 0; c < MD_WS_MAXC; ++c) {
     d2[c] = isum[c] = 0.0;
     rv[c][0] = rv[c][1] = rv[c][2] = 0.0;
-    if (c >= n) continue;
-    int li = cons[c].x, lj = cons[c].y;
+    if (c >= MAXC || c >= n) continue;
+    int li = cons[c < MAXC ? c : 0].x, lj = cons[c < MAXC ? c : 0].y;
     double rp[3], l2 = 0.0, pr = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -491,7 +493,7 @@ __device__ __forceinline__ void md_ws_features(const md_item<MAXA> &it, int nc, 
       l2 += rp[d] * rp[d];
       pr += rp[d] * rv[c][d];
     }
-    double dist = __hiloint2double(cons[c].w, cons[c].z);
+    double dist = __hiloint2double(cons[c < MAXC ? c : 0].w, cons[c < MAXC ? c : 0].z);
     d2[c] = dist * dist;
     const double imi = md_pick1(it.im, li), imj = md_pick1(it.im, lj);
     isum[c] = imi + imj;
@@ -505,8 +507,9 @@ __device__ __forceinline__ void md_ws_features(const md_item<MAXA> &it, int nc, 
   for (int c = 0; c < MD_WS_MAXC; ++c)
 #pragma unroll
     for (int e = c + 1; e < MD_WS_MAXC; ++e, ++pair) {
-      if (e >= n) continue;
-      int ci = cons[c].x, cj = cons[c].y, ei = cons[e].x, ej = cons[e].y;
+      if (e >= MAXC || e >= n) continue;
+      int ci = cons[c < MAXC ? c : 0].x, cj = cons[c < MAXC ? c : 0].y, ei = cons[e < MAXC ? e : 0].x,
+          ej = cons[e < MAXC ? e : 0].y;
       double shared = 0.0;
       if (ci == ei) shared += md_pick1(it.im, ci);
       if (cj == ej) shared += md_pick1(it.im, cj);
@@ -644,42 +647,60 @@ __device__ __forceinline__ void md_settle_velocities(md_item<3> &it, const float
 __device__ __forceinline__ void md_com_velocity(const md_int_args &A, uint32_t step, float *vcom) {
   vcom[0] = vcom[1] = vcom[2] = 0.0f;
   if (A.cmm_frequency > 0 && step % (uint32_t)A.cmm_frequency == 0) {
-    const int64_t *p = A.ctl->momentum[step & 1];
+    const int64_t *p = A.ctl->momentum;
 #pragma unroll
     for (int d = 0; d < 3; ++d) vcom[d] = (float)(md_fixed_to_double_dev(p[d]) * (double)A.inv_total_mass);
   }
 }
 
-__device__ __forceinline__ void md_reduce_out(const md_int_args &A, uint32_t step, const double *mom, float worst) {
-  // momentum for the next step's COM removal, and the displacement monitor
+// Momentum for the next step's COM removal, the SHAKE counts and the
+// displacement monitor, one wave's worth.  The sums go to MD_STEP_PARTS lines
+// that the next prologue adds up: with every wave adding to the control words
+// themselves, the integrator of 243k atoms waited 55 us for some 4,500 atomics
+// on one line.
+__device__ __forceinline__ void md_reduce_out(const md_int_args &A, const double *mom, float worst, int passes,
+                                              int clusters) {
+  int64_t *part = A.ctl->part[blockIdx.x % MD_STEP_PARTS];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     int64_t f = md_wave_sum_i64((int64_t)rint(mom[d] * 4294967296.0));
-    if ((threadIdx.x & 63) == 0) md_atomic_add_i64(&A.ctl->momentum[(step + 1) & 1][d], f);
+    if (threadIdx.x == 0) md_atomic_add_i64(&part[d], f);
+  }
+  const int64_t cs = md_wave_sum_i64(clusters);
+  if (cs) {  // wave-uniform
+    const int64_t ps = md_wave_sum_i64(passes);
+    if (threadIdx.x == 0) {
+      md_atomic_add_i64(&part[3], ps);
+      md_atomic_add_i64(&part[4], cs);
+    }
   }
   for (int off = 32; off > 0; off >>= 1) worst = fmaxf(worst, __shfl_xor(worst, off, 64));
-  if ((threadIdx.x & 63) == 0) {
-    atomicMax(&A.ctl->max_disp2_bits[0], __float_as_uint(worst));
+  if (threadIdx.x == 0) {
+    md_raise(&A.ctl->max_disp2_bits[0], worst);
     if (worst > A.half_skin2) A.ctl->rebuild_request[0] = 1;
   }
 }
 
-// SHAKE clusters run in workgroups of one wavefront: an ensemble has few
-// clusters per replica (~300 at 10k atoms), so 64 per workgroup spreads them
-// over four times as many CUs as 256 would, and a slow-converging cluster
-// holds up one wave, not four.
-#define MD_CLUSTER_BLOCK 64
+// One step of a replica's items in one launch, a wave per workgroup: first the
+// SHAKE clusters (the longest chain of work, so it starts first), then the
+// SETTLE waters, then the free atoms.  KIND 0: free atoms, 1: waters, 2:
+// clusters of at most MAXA atoms and MAXC constraints.  MODE (clusters only): 0
+// plain SHAKE; 1 plain SHAKE, recording each cluster's features and converged
+// multipliers as training samples; 2 SHAKE started from the network's predicted
+// multipliers.
+//
+// STAR: every cluster of the launch is a heavy atom, first, and its hydrogens
+// in the order of its constraints (X-H constraints of the usual topologies).
+// The constraints' atom numbers are then constants and the picks of a cluster's
+// atoms by number fall away: on a small system the clusters of a step are one
+// long chain of instructions in a wave or two, 41 us with the picks (71 KB of
+// straight code), 21 without.  As three launches, with every wave's sums on the
+// control words, a step's integration took 62 us at 2,168 atoms (so: 22), 111
+// at 243k (33) and 106 on 64 replicas (66).
+#define MD_INT_BLOCK 64
 
-// kind 0: free atoms, 1: SETTLE waters, 2: SHAKE clusters (MAXA atoms).
-// MODE (clusters only): 0 plain SHAKE; 1 plain SHAKE, recording each
-// cluster's features and converged multipliers as training samples; 2 SHAKE
-// started from the network's predicted multipliers.  Every cluster step adds
-// its SHAKE passes to the replica's counters.
-template <int KIND, int MAXA, int MODE = 0>
-__global__ void __launch_bounds__(256) k_integrate(const md_int_args *__restrict__ T, md_bmap map) {
-  int blk;
-  const md_int_args &A = T[md_locate(map, blockIdx.x, blk)];
-  int t = blk * blockDim.x + threadIdx.x;
+template <int KIND, int MAXA, int MAXC, int MODE, bool STAR>
+__device__ __forceinline__ void md_step_item(const md_int_args &A, int t, float *ws_lds) {
   uint32_t step = (uint32_t)A.ctl->step_current;
   float vcom[3];
   md_com_velocity(A, step, vcom);
@@ -689,9 +710,8 @@ __global__ void __launch_bounds__(256) k_integrate(const md_int_args *__restrict
   const bool live = t < count;
   md_item<MAXA> it;
   it.n = 0;
-  int nc = 0;
+  int nc = 0, passes = 0;
   uint32_t failed = 0;  // control-block divergence bits this thread raises
-  constexpr int MAXC = KIND == 2 ? md_max_constraints<MAXA>::value : 1;
   int4 cons[MAXC];
   if (live) {
     if (KIND == 0) {
@@ -709,8 +729,13 @@ __global__ void __launch_bounds__(256) k_integrate(const md_int_args *__restrict
       for (int a = 0; a < MAXA; ++a) it.atom[a] = a < it.n ? A.ccl_atoms[t * MD_MAX_CLUSTER_ATOMS + a] : 0;
       nc = A.ccl_ncons[t];
 #pragma unroll
-      for (int c = 0; c < MAXC; ++c)
+      for (int c = 0; c < MAXC; ++c) {
         cons[c] = c < nc ? A.ccl_cons[t * MD_MAX_CLUSTER_CONSTRAINTS + c] : make_int4(0, 0, 0, 0);
+        if (STAR) {
+          cons[c].x = 0;
+          cons[c].y = c + 1;
+        }
+      }
     }
     md_load_kick(A, it, vcom);
     if constexpr (KIND == 1) {
@@ -734,21 +759,19 @@ __global__ void __launch_bounds__(256) k_integrate(const md_int_args *__restrict
     bool warm = false;
     if constexpr (MODE == 2) {
       // every lane of the workgroup runs the network (its replica's, or none)
-      __shared__ float ws_lds[(MD_CLUSTER_BLOCK / 64) * MD_WS_TILE_LDS];
       if (A.ws) {
         float f[MD_WS_F], y[MD_WS_MAXC];
         if (covered)
           md_ws_features(it, nc, cons, f);
         else
           for (int k = 0; k < MD_WS_F; ++k) f[k] = 0.0f;
-        md_ws_infer(*A.ws, f, y, ws_lds + (threadIdx.x >> 6) * MD_WS_TILE_LDS);
+        md_ws_infer(*A.ws, f, y, ws_lds);
         if (covered) {
           for (int c = 0; c < MD_WS_MAXC; ++c) lam0[c] = y[c] * (1.0f / MD_WS_SCALE);
           warm = true;
         }
       }
     }
-    int passes = 0;
     if (live) {
       double total[MD_WS_MAXC];
       float f[MD_WS_F];
@@ -769,16 +792,28 @@ __global__ void __launch_bounds__(256) k_integrate(const md_int_args *__restrict
         }
       }
     }
-    // SHAKE passes and clusters of this step, for the warm start's gain
-    int64_t ps = md_wave_sum_i64((int64_t)passes), cs = md_wave_sum_i64(live ? 1 : 0);
-    if ((threadIdx.x & 63) == 0 && cs) {
-      md_atomic_add_i64(&A.ctl->shake_passes, ps);
-      md_atomic_add_i64(&A.ctl->shake_clusters, cs);
-    }
   }
   if (live) md_finish(A, it, mom, worst, failed);
   if (failed) atomicOr(&A.ctl->diverged, failed);
-  md_reduce_out(A, step, mom, worst);
+  md_reduce_out(A, mom, worst, passes, KIND == 2 && live ? 1 : 0);
+}
+
+template <int MAXA, int MAXC, int MODE, bool STAR>
+__global__ void __launch_bounds__(MD_INT_BLOCK) k_integrate(const md_int_args *__restrict__ T, md_bmap map) {
+  __shared__ float ws_lds[MODE == 2 ? MD_WS_TILE_LDS : 1];
+  int blk;
+  const md_int_args &A = T[md_locate(map, blockIdx.x, blk)];
+  if (blk < A.blocks_ccl) {
+    md_step_item<2, MAXA, MAXC, MODE, STAR>(A, blk * MD_INT_BLOCK + threadIdx.x, ws_lds);
+    return;
+  }
+  blk -= A.blocks_ccl;
+  if (blk < A.blocks_water) {
+    md_step_item<1, 3, 1, 0, false>(A, blk * MD_INT_BLOCK + threadIdx.x, nullptr);
+    return;
+  }
+  blk -= A.blocks_water;
+  md_step_item<0, 1, 1, 0, false>(A, blk * MD_INT_BLOCK + threadIdx.x, nullptr);
 }
 
 // Constraint projection outside a step (src/reference/constraints.ts:254-291):
@@ -859,33 +894,31 @@ __global__ void __launch_bounds__(256) k_constrain(const md_int_args *__restrict
   }
 }
 
-// the start of a step, where no other kernel runs it (md_nb_build)
-__global__ void k_step_prologue(const md_int_args *__restrict__ T, int R, int advance) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < R) md_prologue(T[r].ctl, T[r].group_status, T[r].energy, advance);
+// the start of a step, where no other kernel runs it (md_nb_build): one wave per
+// replica
+__global__ void __launch_bounds__(64) k_step_prologue(const md_int_args *__restrict__ T, int advance) {
+  const md_int_args &A = T[blockIdx.x];
+  md_prologue(A.ctl, A.group_status, A.energy, advance);
 }
 
-// momentum of the current velocities, into the slot the next step reads
+// momentum of the current velocities, in the parts the next prologue adds up
 __global__ void k_momentum(const md_int_args *__restrict__ T, md_bmap map) {
   int blk;
   const md_int_args &A = T[md_locate(map, blockIdx.x, blk)];
-  md_control *ctl = A.ctl;
   int i = blk * blockDim.x + threadIdx.x;
-  uint32_t slot = (uint32_t)(ctl->step_next & 1);
+  int64_t *part = A.ctl->part[blk % MD_STEP_PARTS];
   double m[3] = {0, 0, 0};
   if (i < A.n)
     for (int d = 0; d < 3; ++d) m[d] = (double)A.mass[i] * A.vel[d * A.np + i];
   for (int d = 0; d < 3; ++d) {
     int64_t f = md_wave_sum_i64((int64_t)rint(m[d] * 4294967296.0));
-    if ((threadIdx.x & 63) == 0) md_atomic_add_i64(&ctl->momentum[slot][d], f);
+    if ((threadIdx.x & 63) == 0) md_atomic_add_i64(&part[d], f);
   }
 }
 
-__global__ void k_clear_momentum(const md_int_args *__restrict__ T, int R) {
-  int r = blockIdx.x;
-  if (r >= R || threadIdx.x >= 3) return;
-  md_control *ctl = T[r].ctl;
-  ctl->momentum[ctl->step_next & 1][threadIdx.x] = 0;
+__global__ void k_clear_momentum(const md_int_args *__restrict__ T) {
+  const int k = threadIdx.x;
+  if (k < MD_STEP_PARTS * 3) T[blockIdx.x].ctl->part[k / 3][k % 3] = 0;
 }
 
 static md_int_args int_args(md_system *s) {
@@ -924,6 +957,8 @@ static md_int_args int_args(md_system *s) {
   A.n_waters = s->n_waters;
   A.n_ccl = s->n_clusters_c;
   A.n_free = s->n_free;
+  A.blocks_ccl = (s->n_clusters_c + MD_INT_BLOCK - 1) / MD_INT_BLOCK;
+  A.blocks_water = (s->n_waters + MD_INT_BLOCK - 1) / MD_INT_BLOCK;
   A.n = s->n;
   A.ws = s->ws_net;
   A.rec_x = s->rec_x;
@@ -935,8 +970,11 @@ static md_int_args int_args(md_system *s) {
 
 struct md_int_group {
   md_int_args *table = nullptr;
-  md_launch free_items, waters, clusters, atoms;
+  md_launch items, waters, clusters, atoms;  // a step's items; constraint projection; momentum
   int R = 0;
+  // every cluster a heavy atom and its hydrogens (md_step_item); for the network's
+  // features, which name a constraint's first atom, that one being the heavy atom
+  bool star = true, star_features = true;
 };
 
 static md_int_group &ig(md_group *g) { return *reinterpret_cast<md_int_group *>(g->integ); }
@@ -945,16 +983,20 @@ void md_int_group_setup(md_group *g) {
   auto *G = new md_int_group();
   g->integ = G;
   G->R = (int)g->reps.size();
-  std::vector<int> fr, wa, cl, at;
+  std::vector<int> items, wa, cl, at;
   g->max_cluster_atoms = 0;
   for (md_system *s : g->reps) {
-    fr.push_back((s->n_free + 255) / 256);
+    const int blocks[3] = {(s->n_clusters_c + MD_INT_BLOCK - 1) / MD_INT_BLOCK,
+                           (s->n_waters + MD_INT_BLOCK - 1) / MD_INT_BLOCK, (s->n_free + MD_INT_BLOCK - 1) / MD_INT_BLOCK};
+    items.push_back(blocks[0] + blocks[1] + blocks[2]);
     wa.push_back((s->n_waters + 255) / 256);
-    cl.push_back((s->n_clusters_c + MD_CLUSTER_BLOCK - 1) / MD_CLUSTER_BLOCK);
+    cl.push_back(blocks[0]);
+    G->star &= s->star_clusters >= 1;
+    G->star_features &= s->star_clusters == 2;
     at.push_back((s->n + 255) / 256);
     g->max_cluster_atoms = std::max(g->max_cluster_atoms, s->max_cluster_atoms);
   }
-  G->free_items = md_make_launch(g, fr);
+  G->items = md_make_launch(g, items);
   G->waters = md_make_launch(g, wa);
   G->clusters = md_make_launch(g, cl);
   G->atoms = md_make_launch(g, at);
@@ -987,34 +1029,30 @@ void md_int_group_free(md_group *g) {
 
 void md_step_prologue(md_group *g, bool advance) {
   auto &G = ig(g);
-  k_step_prologue<<<(G.R + 63) / 64, 64, 0, g->stream>>>(G.table, G.R, advance ? 1 : 0);
+  k_step_prologue<<<G.R, 64, 0, g->stream>>>(G.table, advance ? 1 : 0);
   MD_HIP(hipGetLastError());
+}
+
+template <int MAXA, int MAXC, bool STAR>
+static void launch_integrate(md_group *g) {
+  auto &G = ig(g);
+  const int n = G.items.total;
+  if (g->ws_mode == 2)
+    k_integrate<MAXA, MAXC, 2, STAR><<<n, MD_INT_BLOCK, 0, g->stream>>>(G.table, G.items.map);
+  else if (g->ws_mode == 1)
+    k_integrate<MAXA, MAXC, 1, STAR><<<n, MD_INT_BLOCK, 0, g->stream>>>(G.table, G.items.map);
+  else
+    k_integrate<MAXA, MAXC, 0, STAR><<<n, MD_INT_BLOCK, 0, g->stream>>>(G.table, G.items.map);
 }
 
 void md_integrate(md_group *g) {
   auto &G = ig(g);
-  hipStream_t st = g->stream;
-  const md_int_args *T = G.table;
-  if (G.free_items.total) k_integrate<0, 1><<<G.free_items.total, 256, 0, st>>>(T, G.free_items.map);
-  if (G.waters.total) k_integrate<1, 3><<<G.waters.total, 256, 0, st>>>(T, G.waters.map);
-  if (G.clusters.total) {
-    const int mode = g->ws_mode;
-    if (g->max_cluster_atoms <= 4) {
-      if (mode == 2)
-        k_integrate<2, 4, 2><<<G.clusters.total, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map);
-      else if (mode == 1)
-        k_integrate<2, 4, 1><<<G.clusters.total, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map);
-      else
-        k_integrate<2, 4, 0><<<G.clusters.total, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map);
-    } else {
-      if (mode == 2)
-        k_integrate<2, 8, 2><<<G.clusters.total, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map);
-      else if (mode == 1)
-        k_integrate<2, 8, 1><<<G.clusters.total, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map);
-      else
-        k_integrate<2, 8, 0><<<G.clusters.total, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map);
-    }
-  }
+  if (g->max_cluster_atoms <= 4 && (g->ws_mode == 0 ? G.star : G.star_features))
+    launch_integrate<4, 3, true>(g);
+  else if (g->max_cluster_atoms <= 4)
+    launch_integrate<4, md_max_constraints<4>::value, false>(g);
+  else
+    launch_integrate<8, md_max_constraints<8>::value, false>(g);
   MD_HIP(hipGetLastError());
 }
 
@@ -1032,14 +1070,14 @@ void md_constrain(md_group *g, int what, double tolerance) {
     int gsz = G.clusters.total;
     if (g->max_cluster_atoms <= 4) {
       if (what == 0)
-        k_constrain<2, 4, 0><<<gsz, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
+        k_constrain<2, 4, 0><<<gsz, MD_INT_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
       else
-        k_constrain<2, 4, 1><<<gsz, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
+        k_constrain<2, 4, 1><<<gsz, MD_INT_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
     } else {
       if (what == 0)
-        k_constrain<2, 8, 0><<<gsz, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
+        k_constrain<2, 8, 0><<<gsz, MD_INT_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
       else
-        k_constrain<2, 8, 1><<<gsz, MD_CLUSTER_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
+        k_constrain<2, 8, 1><<<gsz, MD_INT_BLOCK, 0, st>>>(T, G.clusters.map, tolerance);
     }
   }
   MD_HIP(hipGetLastError());
@@ -1047,7 +1085,7 @@ void md_constrain(md_group *g, int what, double tolerance) {
 
 void md_momentum(md_group *g) {
   auto &G = ig(g);
-  k_clear_momentum<<<G.R, 64, 0, g->stream>>>(G.table, G.R);
+  k_clear_momentum<<<G.R, 64, 0, g->stream>>>(G.table);
   k_momentum<<<G.atoms.total, 256, 0, g->stream>>>(G.table, G.atoms.map);
   MD_HIP(hipGetLastError());
 }

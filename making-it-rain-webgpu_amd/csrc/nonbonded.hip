@@ -454,10 +454,12 @@ __global__ void __launch_bounds__(MD_SORT_THREADS) k_nb_sort(const md_nb_args *_
   __shared__ int active, wave_sum[16];
   const md_nb_args &A = T[blockIdx.x];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  if (t == 0) {
+  if (wave == 0) {
     md_prologue(A.ctl, A.group_status, A.energy, advance);
-    active = (int)A.ctl->rebuild_active;
-    if (active) md_rebuild_begins(A.ctl);
+    if (lane == 0) {
+      active = (int)A.ctl->rebuild_active;
+      if (active) md_rebuild_begins(A.ctl);
+    }
   }
   __syncthreads();
   if (!active) return;
