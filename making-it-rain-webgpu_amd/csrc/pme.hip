@@ -56,6 +56,7 @@ struct md_pme_table {
   float *phi;
   int64_t *force;
   int64_t *energy;
+  int small_charges;  // every |charge| < MD_SMALL_FIXED
   md_pair_forces F;
   const int64_t *piece;  // the bonded terms' pieces, by atom
   const int *piece_start;
@@ -119,45 +120,78 @@ __device__ __forceinline__ int md_wrap(int i, int n) {
 // is at least the spline's order
 __device__ __forceinline__ int md_wrap_once(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
-// Charge spreading, one workgroup per 64-slot super-cluster of the nonbonded
-// list (spatially compact: its atoms' stencils overlap), one thread per
-// (slot, x-plane of the stencil).  Each thread's 25 contributions -- the
-// same Q32.32 values as one global atomic each would add -- go into an int64
-// tile in LDS covering the super-cluster's stencil box; the tile is then
-// added to the grid, one global atomic per non-zero point: about a quarter
-// of the global atomics of spreading atom by atom.  Integer sums do not
-// depend on order, so the grid is the same either way.  A super-cluster
-// whose box exceeds the tile spreads straight to the grid.
-#define MD_SPREAD_THREADS (64 * MD_PME_ORDER)
-#define MD_SPREAD_TILE 6144  // int64 points (48 KB of LDS)
+// md_to_fixed for |x| < 2^19: adding 1.5 * 2^20 in f64 rounds x to a multiple of
+// 2^-32, ties to even, and leaves that multiple in the sum's low bits.  Four
+// instructions instead of about twelve.
+__device__ __forceinline__ int64_t md_small_to_fixed(float x) {
+  return __double_as_longlong((double)x + 1572864.0) - 0x4138000000000000ll;
+}
+#define MD_SMALL_FIXED 524288.0f  // 2^19
 
+// idx / m for 0 <= idx < 2^20 by an f32 reciprocal (an integer division is some
+// 30 instructions, more than a radix-4 butterfly): (idx + 1/2) / m is at least
+// 1/(2m) from an integer, and the product is within 3.6e-7 of it relatively.
+__device__ __forceinline__ float md_inverse(int m) { return __builtin_amdgcn_rcpf((float)m); }
+__device__ __forceinline__ int md_div(int idx, float inv) { return (int)(((float)idx + 0.5f) * inv); }
+
+// the representative in [-n/2, n/2) of a difference of two bases
 __device__ __forceinline__ int md_wrap_near(int d, int n) {
-  d = md_wrap(d, n);
-  return d >= n / 2 ? d - n : d;  // the representative in [-n/2, n/2)
+  if (d < 0) d += n;  // bases lie in [-4, n]: now in [0, n + 4]
+  if (d >= n) d -= n;
+  return d >= n / 2 ? d - n : d;
 }
 
-__global__ void __launch_bounds__(MD_SPREAD_THREADS) k_pme_spread(const md_pme_table *__restrict__ T, md_bmap map) {
+// Charge spreading.  A workgroup takes `per` consecutive 64-slot super-clusters
+// of the nonbonded list (spatially compact: their atoms' stencils overlap); one
+// wave each finds the atoms' stencils, then wave a adds plane a of every stencil
+// to an int64 tile in LDS covering their stencil box, and the tile is added to
+// the grid, one global atomic per non-zero point: about a fifth of the atomics
+// of spreading atom by atom.  Contributions are Q32.32 and integer sums do not
+// depend on order, so the grid is the same however atoms are grouped.  Super-
+// clusters whose joint box exceeds the tile go one at a time; a single one that
+// exceeds it spreads straight to the grid.
+//
+// Bound by the atomic requests at memory, and on small launches by latency (64
+// replicas, 289 us before, with 4.6 M requests and 91 M wave instructions, 150
+// us of VALU issue): stencils are found once, not by each of the five waves,
+// contributions are rounded by md_small_to_fixed, the flush divides by
+// reciprocals, and two super-clusters share a tile where there are enough of
+// them to fill the chip.  Now 258 us there, 85 at 243k atoms (107), 15 at 31k
+// (18).
+#define MD_SPREAD_WAVES MD_PME_ORDER
+#define MD_SPREAD_THREADS (64 * MD_SPREAD_WAVES)
+#define MD_SPREAD_TILE 5632  // int64 points: 45 KB, with the stencils 54 KB, three workgroups to a CU
+#define MD_SPREAD_MOST 2     // super-clusters of a workgroup
+#define MD_SPREAD_PAIRED 1024  // super-clusters of a launch from which they go two to a workgroup
+
+struct md_spread_box {
+  int ref[3], lo[3], hi[3];  // a stencil base, and the lowest and highest offsets from it; lo > hi: no charge
+};
+
+__global__ void __launch_bounds__(MD_SPREAD_THREADS) k_pme_spread(const md_pme_table *__restrict__ T, md_bmap map, int per) {
   // super-clusters laid out XCD by XCD: neighbouring ones add into the same
   // mesh region from one L2
-  int S;
-  const md_pme_table &E = T[md_locate(map, md_xcd_block(blockIdx.x, gridDim.x), S)];
+  int blk;
+  const md_pme_table &E = T[md_locate(map, md_xcd_block(blockIdx.x, gridDim.x), blk)];
   const md_pme_args &P = E.P;
   int64_t *grid = E.grid;
   __shared__ unsigned long long tile[MD_SPREAD_TILE];
-  __shared__ int box[9];  // reference stencil base, then lowest and highest offsets from it
-  const int t = threadIdx.x, lane = t & 63, a = t >> 6;
-  const int i = E.slot_atom[S * 64 + lane];
-  const float q = i >= 0 ? E.param[i].w : 0.0f;
-  const bool live = q != 0.0f;
-  int base[3] = {0, 0, 0};
-  float w[3] = {0.0f, 0.0f, 0.0f};
-  if (live) md_mesh_coord(E.pos, E.np, i, P.inv, P.nx, P.ny, P.nz, base, w);
+  __shared__ md_spread_box boxes[MD_SPREAD_MOST];
+  __shared__ float theta[MD_SPREAD_MOST][2 * MD_PME_ORDER + MD_PME_ORDER][64];  // q tx, ty, tz
+  __shared__ int bases[MD_SPREAD_MOST][3][64];                                  // base[0] INT_MIN: no charge
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int n[3] = {P.nx, P.ny, P.nz};
-  // the first wave (plane 0 of every slot) finds the stencil box: offsets of
-  // each base from the first live slot's, taken to the nearest periodic
-  // representative (any representative lands on the same grid points; the
-  // nearest keeps the box small)
-  if (a == 0) {
+  const int S0 = blk * per, count = min(per, E.nslots / 64 - S0);
+  if (wave < count) {
+    const int i = E.slot_atom[(S0 + wave) * 64 + lane];
+    const float q = i >= 0 ? E.param[i].w : 0.0f;
+    const bool live = q != 0.0f;
+    int base[3] = {0, 0, 0};
+    float w[3] = {0.0f, 0.0f, 0.0f};
+    if (live) md_mesh_coord(E.pos, E.np, i, P.inv, P.nx, P.ny, P.nz, base, w);
+    // the stencil box: offsets of each base from the first live slot's, taken to
+    // the nearest periodic representative (any representative lands on the same
+    // grid points; the nearest keeps the box small)
     const uint64_t m = __ballot(live);
     const int first = m ? __ffsll((unsigned long long)m) - 1 : 0;
     for (int d = 0; d < 3; ++d) {
@@ -169,55 +203,116 @@ __global__ void __launch_bounds__(MD_SPREAD_THREADS) k_pme_spread(const md_pme_t
         hi = max(hi, __shfl_xor(hi, k, 64));
       }
       if (lane == 0) {
-        box[d] = ref;
-        box[3 + d] = m ? lo : 0;
-        box[6 + d] = m ? hi : -MD_PME_ORDER;  // no charge: an empty box
+        boxes[wave].ref[d] = ref;
+        boxes[wave].lo[d] = lo;
+        boxes[wave].hi[d] = hi;
+      }
+      bases[wave][d][lane] = base[d];
+    }
+    if (!live) bases[wave][0][lane] = INT_MIN;
+    float tx[5], ty[5], tz[5];
+    md_bspline5(w[0], tx, nullptr);
+    md_bspline5(w[1], ty, nullptr);
+    md_bspline5(w[2], tz, nullptr);
+    for (int c = 0; c < 5; ++c) {
+      theta[wave][c][lane] = q * tx[c];
+      theta[wave][5 + c][lane] = ty[c];
+      theta[wave][10 + c][lane] = tz[c];
+    }
+  }
+  __syncthreads();
+  // one pass over all of them if their joint box fits the tile
+  md_spread_box box = boxes[0];
+  int passes = 1;
+  int shift[3] = {0, 0, 0};  // the second one's reference base from the box's
+  if (count == 2) {
+    const md_spread_box other = boxes[1];
+    if (other.lo[0] <= other.hi[0]) {
+      if (box.lo[0] > box.hi[0]) {
+        box = other;
+      } else {
+        int joint = 1;
+        md_spread_box both = box;
+        for (int d = 0; d < 3; ++d) {
+          shift[d] = md_wrap_near(other.ref[d] - box.ref[d], n[d]);
+          both.lo[d] = min(box.lo[d], other.lo[d] + shift[d]);
+          both.hi[d] = max(box.hi[d], other.hi[d] + shift[d]);
+          joint *= min(both.hi[d] - both.lo[d] + MD_PME_ORDER, MD_SPREAD_TILE);
+          joint = min(joint, MD_SPREAD_TILE + 1);
+        }
+        if (joint <= MD_SPREAD_TILE) {
+          box = both;
+        } else {
+          passes = 2;
+          shift[0] = shift[1] = shift[2] = 0;
+        }
       }
     }
   }
-  __syncthreads();
-  int ext[3], off[3];
-  for (int d = 0; d < 3; ++d) {
-    ext[d] = box[6 + d] - box[3 + d] + MD_PME_ORDER;
-    off[d] = live ? md_wrap_near(base[d] - box[d], n[d]) - box[3 + d] : 0;
-  }
-  const int volume = ext[0] * ext[1] * ext[2];
-  if (volume == 0) return;  // no charged atom in this super-cluster (uniform)
-  float tx[5], ty[5], tz[5];
-  md_bspline5(w[0], tx, nullptr);
-  md_bspline5(w[1], ty, nullptr);
-  md_bspline5(w[2], tz, nullptr);
-  const float wx = q * tx[a];
-  if (volume > MD_SPREAD_TILE) {
-    if (!live) return;
-    const int gx = md_wrap(base[0] + a, P.nx);
-    for (int b = 0; b < 5; ++b) {
-      const int gy = md_wrap(base[1] + b, P.ny);
-      const float wxy = wx * ty[b];
-      int64_t *row = grid + ((size_t)gx * P.ny + gy) * P.nz;
-      for (int c = 0; c < 5; ++c) md_atomic_add_i64(&row[md_wrap(base[2] + c, P.nz)], md_to_fixed(wxy * tz[c]));
+  for (int pass = 0; pass < passes; ++pass) {
+    if (pass) box = boxes[pass];
+    if (box.lo[0] > box.hi[0]) continue;  // no charged atom (uniform)
+    int ext[3];
+    for (int d = 0; d < 3; ++d) ext[d] = box.hi[d] - box.lo[d] + MD_PME_ORDER;
+    const int volume = ext[0] * ext[1] * ext[2], first = passes == 2 ? pass : 0, last = passes == 2 ? pass + 1 : count;
+    if (volume > MD_SPREAD_TILE) {  // one super-cluster alone
+      const int base[3] = {bases[first][0][lane], bases[first][1][lane], bases[first][2][lane]};
+      if (base[0] == INT_MIN) continue;
+      const int gx = md_wrap(base[0] + wave, P.nx);
+      const float wx = theta[first][wave][lane];
+      for (int b = 0; b < 5; ++b) {
+        const int gy = md_wrap(base[1] + b, P.ny);
+        const float wxy = wx * theta[first][5 + b][lane];
+        int64_t *row = grid + ((size_t)gx * P.ny + gy) * P.nz;
+        for (int c = 0; c < 5; ++c)
+          md_atomic_add_i64(&row[md_wrap(base[2] + c, P.nz)], md_to_fixed(wxy * theta[first][10 + c][lane]));
+      }
+      continue;
     }
-    return;
-  }
-  for (int k = t; k < volume; k += MD_SPREAD_THREADS) tile[k] = 0;
-  __syncthreads();
-  if (live) {
-    const int plane = (off[0] + a) * ext[1];
-    for (int b = 0; b < 5; ++b) {
-      const float wxy = wx * ty[b];
-      unsigned long long *row = tile + (size_t)(plane + off[1] + b) * ext[2] + off[2];
-      for (int c = 0; c < 5; ++c) atomicAdd(&row[c], (unsigned long long)md_to_fixed(wxy * tz[c]));
+    for (int k = t; k < volume; k += MD_SPREAD_THREADS) tile[k] = 0;
+    __syncthreads();
+    for (int g = first; g < last; ++g) {
+      if (bases[g][0][lane] == INT_MIN) continue;
+      // the offset from its own super-cluster's reference, as its box was found
+      int off[3];
+      for (int d = 0; d < 3; ++d)
+        off[d] = md_wrap_near(bases[g][d][lane] - boxes[g].ref[d], n[d]) + (g ? shift[d] : 0) - box.lo[d];
+      const float wx = theta[g][wave][lane];
+      float tz[5];
+      for (int c = 0; c < 5; ++c) tz[c] = theta[g][10 + c][lane];
+      unsigned long long *at = tile + ((off[0] + wave) * ext[1] + off[1]) * ext[2] + off[2];
+      for (int b = 0; b < 5; ++b, at += ext[2]) {
+        const float wxy = wx * theta[g][5 + b][lane];
+        if (E.small_charges) {
+          for (int c = 0; c < 5; ++c) atomicAdd(&at[c], (unsigned long long)md_small_to_fixed(wxy * tz[c]));
+        } else {
+          for (int c = 0; c < 5; ++c) atomicAdd(&at[c], (unsigned long long)md_to_fixed(wxy * tz[c]));
+        }
+      }
     }
-  }
-  __syncthreads();
-  const int yz = ext[1] * ext[2];
-  for (int k = t; k < volume; k += MD_SPREAD_THREADS) {
-    const long long v = (long long)tile[k];
-    if (v == 0) continue;
-    const int lx = k / yz, r = k - lx * yz, ly = r / ext[2], lz = r - ly * ext[2];
-    const int gx = md_wrap(box[0] + box[3] + lx, P.nx), gy = md_wrap(box[1] + box[4] + ly, P.ny),
-              gz = md_wrap(box[2] + box[5] + lz, P.nz);
-    md_atomic_add_i64(grid + ((size_t)gx * P.ny + gy) * P.nz + gz, v);
+    __syncthreads();
+    const int x0 = md_wrap(box.ref[0] + box.lo[0], P.nx), y0 = md_wrap(box.ref[1] + box.lo[1], P.ny),
+              z0 = md_wrap(box.ref[2] + box.lo[2], P.nz);
+    const float inv_z = md_inverse(ext[2]), inv_y = md_inverse(ext[1]);
+    // a box wider than the mesh (a stencil box of a tiny mesh) wraps more than once
+    const bool once = ext[0] <= P.nx && ext[1] <= P.ny && ext[2] <= P.nz;
+    for (int k = t; k < volume; k += MD_SPREAD_THREADS) {
+      const long long v = (long long)tile[k];
+      if (v == 0) continue;
+      const int row = md_div(k, inv_z), lx = md_div(row, inv_y);
+      int gx = x0 + lx, gy = y0 + row - lx * ext[1], gz = z0 + k - row * ext[2];
+      if (once) {
+        gx = gx >= P.nx ? gx - P.nx : gx;
+        gy = gy >= P.ny ? gy - P.ny : gy;
+        gz = gz >= P.nz ? gz - P.nz : gz;
+      } else {
+        gx %= P.nx;
+        gy %= P.ny;
+        gz %= P.nz;
+      }
+      md_atomic_add_i64(grid + ((size_t)gx * P.ny + gy) * P.nz + gz, v);
+    }
+    if (pass + 1 < passes) __syncthreads();  // the next pass clears the tile
   }
 }
 
@@ -226,12 +321,6 @@ __global__ void __launch_bounds__(MD_SPREAD_THREADS) k_pme_spread(const md_pme_t
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
-
-// idx / m for 0 <= idx < 2^20 by an f32 reciprocal (an integer division is some
-// 30 instructions, more than a radix-4 butterfly): (idx + 1/2) / m is at least
-// 1/(2m) from an integer, and the product is within 3.6e-7 of it relatively.
-__device__ __forceinline__ float md_inverse(int m) { return __builtin_amdgcn_rcpf((float)m); }
-__device__ __forceinline__ int md_div(int idx, float inv) { return (int)(((float)idx + 0.5f) * inv); }
 
 // Where a stage finds its input and puts its output: lines of LDS (element e
 // of line l at l * line + e * elem; a transposed read swaps the strides), or
@@ -842,6 +931,9 @@ static md_pme_table pme_table(md_system *s) {
   E.phi = s->pme_phi;
   E.force = s->force;
   E.energy = s->energy;
+  E.small_charges = 1;
+  for (double q : s->charge)
+    if (!(std::fabs(q) < MD_SMALL_FIXED)) E.small_charges = 0;
   E.F = md_nb_pair_forces(s);
   E.piece = s->term_piece;
   E.piece_start = s->atom_piece_start;
@@ -851,6 +943,7 @@ static md_pme_table pme_table(md_system *s) {
 struct md_pme_group {
   md_pme_table *table = nullptr;
   md_launch spread, zrows, ylines, xlines, gather, planes;
+  int spread_per = 1;             // super-clusters of a spreading workgroup
   size_t lz = 0, ly = 0, lx = 0;  // dynamic LDS of the three passes
   size_t lyz = 0;                 // dynamic LDS of a whole x-plane
   bool fused_yz = false;          // the y and z passes per x-plane in one launch
@@ -863,10 +956,13 @@ void md_pme_group_setup(md_group *g) {
   g->pme = G;
   std::vector<int> spread, zrows, ylines, xlines, gather, planes;
   int mx = 0, my = 0, mz = 0;
+  long supers = 0;
+  for (md_system *s : g->reps) supers += s->has_nonbonded ? s->nb.nslots / 64 : 0;
+  G->spread_per = supers >= MD_SPREAD_PAIRED ? 2 : 1;
   for (md_system *s : g->reps) {
     bool on = s->has_nonbonded;
     int nx = s->pme_nx, ny = s->pme_ny, nz = s->pme_nz, kzb = md_kz_runs(s->pme_nzc);
-    spread.push_back(on ? s->nb.nslots / 64 : 0);
+    spread.push_back(on ? (s->nb.nslots / 64 + G->spread_per - 1) / G->spread_per : 0);
     zrows.push_back(on ? (nx * ny + PME_BATCH - 1) / PME_BATCH : 0);
     ylines.push_back(on ? nx * kzb : 0);
     xlines.push_back(on ? ny * kzb : 0);
@@ -934,7 +1030,7 @@ void md_pme(md_group *g, bool energy) {
   if (G.spread.total == 0) return;
   hipStream_t st = g->stream;
   const md_pme_table *T = G.table;
-  k_pme_spread<<<G.spread.total, MD_SPREAD_THREADS, 0, st>>>(T, G.spread.map);
+  k_pme_spread<<<G.spread.total, MD_SPREAD_THREADS, 0, st>>>(T, G.spread.map, G.spread_per);
   md_mark(g, MD_PHASE_FFT);
   if (G.fused_yz) {
     k_pme_yz_forward<<<G.planes.total, MD_PLANE_THREADS, G.lyz, st>>>(T, G.planes.map);
