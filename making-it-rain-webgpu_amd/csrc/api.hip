@@ -645,9 +645,7 @@ static void launch_step(md_group *g) {
   md_mark(g, -1);
 }
 
-static void check_control(md_system *s) {
-  md_control c;
-  MD_HIP(hipMemcpy(&c, s->ctl, sizeof c, hipMemcpyDeviceToHost));
+static void raise_errors(const md_errors &c) {
   const std::string when = " (at or before step " + std::to_string(c.step_current) + ")";
   if (c.overflow == 2)
     throw md_error(MD_ERR_CUTOFF_TOO_LARGE,
@@ -674,6 +672,12 @@ static void check_control(md_system *s) {
                        ((c.diverged & 2) ? ": RATTLE did not converge within its passes" : "") +
                        ((c.diverged & 4) ? ": a velocity became non-finite" : "") +
                        "; the time step is too long for this system, or its starting geometry is strained");
+}
+
+static void check_control(md_system *s) {
+  md_control c;
+  MD_HIP(hipMemcpy(&c, s->ctl, sizeof c, hipMemcpyDeviceToHost));
+  raise_errors({c.step_current, c.overflow, c.barostat_error, c.diverged});
 }
 
 // host state of each replica onto the device before its first step: the
@@ -807,15 +811,8 @@ static void run_steps(md_system *s, int64_t steps) {
   run_group(s->self, steps);
 }
 
-static void evaluate(md_system *s, double *forces, double *groups, double *total, bool census) {
-  MD_HIP(hipSetDevice(s->device));
-  fault_tick(s, 1);
+static void launch_evaluation(md_system *s) {
   md_group *grp = s->self;
-  group_prepare(grp);
-  if (census) {
-    MD_HIP(hipMemsetAsync(&s->ctl->pair_census, 0, sizeof(int64_t), s->stream));
-    MD_HIP(hipMemsetAsync(&s->ctl->pair_blocks, 0, sizeof(int64_t), s->stream));
-  }
   if (s->has_nonbonded) {
     md_nb_build(grp, false);
     md_nb_pairs(grp, true);
@@ -827,6 +824,18 @@ static void evaluate(md_system *s, double *forces, double *groups, double *total
     md_pme(grp, true);
   else
     md_bonded_forces(grp);
+}
+
+static void evaluate(md_system *s, double *forces, double *groups, double *total, bool census) {
+  MD_HIP(hipSetDevice(s->device));
+  fault_tick(s, 1);
+  md_group *grp = s->self;
+  group_prepare(grp);
+  if (census) {
+    MD_HIP(hipMemsetAsync(&s->ctl->pair_census, 0, sizeof(int64_t), s->stream));
+    MD_HIP(hipMemsetAsync(&s->ctl->pair_blocks, 0, sizeof(int64_t), s->stream));
+  }
+  launch_evaluation(s);
   int64_t e[MD_E_SLOTS];
   MD_HIP(hipMemcpyAsync(e, s->energy, sizeof e, hipMemcpyDeviceToHost, s->stream));
   std::vector<int64_t> f;
@@ -870,15 +879,27 @@ struct lbfgs_state {
 };
 }  // namespace
 
-static double min_objective(lbfgs_state &L, const double *x, double *g) {
+// The objective and its gradient g at x + step d (at x itself without d): one
+// read-back, of the energies, the errors and the gradient's products.
+static const md_min_report &min_objective(lbfgs_state &L, const double *x, const double *d, double step, double *trial,
+                                          double *g, double &value) {
   md_system *s = L.s;
-  if (!md_min_positions_in(s, L.w, x))
-    throw md_error(MD_ERR_FIXED_POINT_OVERFLOW, "the minimiser moved a coordinate outside the fixed-point range");
-  MD_HIP(hipMemsetAsync(&s->ctl->overflow, 0, sizeof(uint32_t), s->stream));
+  MD_HIP(hipSetDevice(s->device));
+  md_min_trial(s, L.w, x, d, step, trial);
   s->need_rebuild = true;
-  double total = 0.0;
-  evaluate(s, nullptr, nullptr, &total, false);
-  return total + md_min_gradient(s, L.w, x, L.kspring, g);
+  fault_tick(s, 1);
+  if (s->momentum_dirty) group_prepare(s->self);
+  launch_evaluation(s);
+  s->need_rebuild = false;
+  const md_min_report &r = md_min_gradient(s, L.w, d ? trial : x, d, L.kspring, g);
+  if (r.bad) {
+    s->need_rebuild = true;
+    throw md_error(MD_ERR_FIXED_POINT_OVERFLOW, "the minimiser moved a coordinate outside the fixed-point range");
+  }
+  raise_errors(r.errors);
+  double groups[MD_GROUP_COUNT];
+  value = md_energy_groups(r.energy, md_energy_constants(s), box_volume(s->box), groups) + r.spring;
+  return r;
 }
 
 // returns the iterations taken; L.x holds the last accepted point
@@ -886,33 +907,31 @@ static int min_lbfgs(lbfgs_state &L, int max_iterations, double rms_tolerance, d
   md_system *s = L.s;
   const double max_move = 0.5, armijo = 1e-4, curvature = 0.9;
   const int max_line_search = 40;
-  auto done = [&](const double *grad) { return std::sqrt(md_min_dot(s, L.w, grad, grad) / s->n) <= rms_tolerance; };
-  value = min_objective(L, L.x, L.g);
-  if (done(L.g)) return 0;
-  double rho[MD_MIN_MEMORY];
+  auto done = [&](double gg) { return std::sqrt(gg / s->n) <= rms_tolerance; };
+  double gg = min_objective(L, L.x, nullptr, 0.0, nullptr, L.g, value).gg;
+  if (done(gg)) return 0;
   int count = 0, head = 0;  // pairs held; the slot the next pair goes to
-  md_min_lincomb(s, L.d, -1.0, L.g, 0.0, nullptr);
-  double step = 1.0 / std::sqrt(md_min_dot(s, L.w, L.d, L.d));
+  const md_min_report *r = &md_min_steepest(s, L.w, L.g, L.d);
+  double slope0 = r->slope, dmax = r->most;
+  double step = 1.0 / std::sqrt(gg);  // 1 / |d|
   int iteration = 0;
   for (;;) {
     ++iteration;
-    const double slope0 = md_min_dot(s, L.w, L.g, L.d);
     if (slope0 >= 0.0) return iteration - 1;
     bool accepted = false;
     double v = 0.0;
-    const double dmax = md_min_absmax(s, L.w, L.d);
     for (int trial = 0; trial < max_line_search; ++trial) {
       if (step * dmax > max_move) {
         step *= 0.5;
         continue;
       }
-      md_min_lincomb(s, L.trial, 1.0, L.x, step, L.d);
-      v = min_objective(L, L.trial, L.gt);
+      r = &min_objective(L, L.x, L.d, step, L.trial, L.gt, v);
+      const double slope = r->slope;
+      gg = r->gg;
       if (!(v <= value + armijo * step * slope0)) {
         step *= 0.5;
         continue;
       }
-      const double slope = md_min_dot(s, L.w, L.gt, L.d);
       if (slope < curvature * slope0) {
         if (2.1 * step * dmax > max_move) {
           accepted = true;  // still steep, but at the displacement cap
@@ -927,39 +946,31 @@ static int min_lbfgs(lbfgs_state &L, int max_iterations, double rms_tolerance, d
       }
     }
     if (!accepted) return iteration - 1;
-    // the correction pair of this step, into the next slot of the ring
-    md_min_lincomb(s, L.S[head], 1.0, L.trial, -1.0, L.x);
-    md_min_lincomb(s, L.Y[head], 1.0, L.gt, -1.0, L.g);
+    value = v;
+    const bool stop = done(gg) || (max_iterations > 0 && iteration >= max_iterations);
+    if (!stop) {
+      // the correction pair of this step, into the next slot of the ring, and
+      // the two-loop recursion q = -H g
+      md_min_loop loop{};
+      loop.head = head;
+      loop.count = count;
+      loop.g = L.gt;
+      loop.q = L.q;
+      std::copy(L.S, L.S + MD_MIN_MEMORY, loop.S);
+      std::copy(L.Y, L.Y + MD_MIN_MEMORY, loop.Y);
+      r = &md_min_direction(s, L.w, loop, L.x, L.trial, L.g);
+      slope0 = r->slope;
+      dmax = r->most;
+      if (r->kept) {
+        head = (head + 1) % MD_MIN_MEMORY;
+        count = std::min(count + 1, MD_MIN_MEMORY);
+      }
+      std::swap(L.d, L.q);
+      step = 1.0;
+    }
     std::swap(L.x, L.trial);
     std::swap(L.g, L.gt);
-    value = v;
-    if (done(L.g) || (max_iterations > 0 && iteration >= max_iterations)) return iteration;
-    const double sy = md_min_dot(s, L.w, L.S[head], L.Y[head]);
-    if (sy > 0.0) {
-      rho[head] = 1.0 / sy;
-      head = (head + 1) % MD_MIN_MEMORY;
-      count = std::min(count + 1, MD_MIN_MEMORY);
-    }
-    // two-loop recursion: q = -H g
-    md_min_lincomb(s, L.q, -1.0, L.g, 0.0, nullptr);
-    double alpha[MD_MIN_MEMORY];
-    for (int k = 0; k < count; ++k) {  // newest to oldest
-      const int slot = (head - 1 - k + 2 * MD_MIN_MEMORY) % MD_MIN_MEMORY;
-      alpha[k] = rho[slot] * md_min_dot(s, L.w, L.S[slot], L.q);
-      md_min_lincomb(s, L.q, 1.0, L.q, -alpha[k], L.Y[slot]);
-    }
-    if (count) {
-      const int newest = (head - 1 + MD_MIN_MEMORY) % MD_MIN_MEMORY;
-      md_min_lincomb(s, L.q, 1.0 / (rho[newest] * md_min_dot(s, L.w, L.Y[newest], L.Y[newest])), L.q, 0.0,
-                     nullptr);
-    }
-    for (int k = count - 1; k >= 0; --k) {  // oldest to newest
-      const int slot = (head - 1 - k + 2 * MD_MIN_MEMORY) % MD_MIN_MEMORY;
-      const double beta = rho[slot] * md_min_dot(s, L.w, L.Y[slot], L.q);
-      md_min_lincomb(s, L.q, 1.0, L.q, alpha[k] - beta, L.S[slot]);
-    }
-    std::swap(L.d, L.q);
-    step = 1.0;
+    if (stop) return iteration;
   }
 }
 

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -442,27 +443,68 @@ int &md_baro_step(md_system *s);            // steps since the last attempt
 // L-BFGS work vectors: MD_MIN_VECTORS f64 3N-vectors in planes [3][np]
 #define MD_MIN_MEMORY 6
 #define MD_MIN_VECTORS (6 + 2 * MD_MIN_MEMORY)
+// what a control block says went wrong
+struct md_errors {
+  int64_t step_current;
+  uint32_t overflow, barostat_error, diverged;
+};
+// the host's view of a trial point or of a search direction, in pinned memory
+struct md_min_report {
+  double slope;   // gradient . direction
+  double gg;      // gradient . gradient
+  double spring;  // the constraint springs' energy
+  double most;    // the direction's largest component
+  int kept;       // the last correction pair was kept
+  int bad;        // a coordinate outside the fixed-point range
+  md_errors errors;
+  int64_t energy[MD_E_SLOTS];
+};
+// the recursion's coefficients: by slot 1 / S.Y and Y.Y, by pair alpha
+struct md_min_state {
+  double rho[MD_MIN_MEMORY], yy[MD_MIN_MEMORY], alpha[MD_MIN_MEMORY];
+  int kept;
+};
+// the recursion's vectors; head the slot of the pair being formed, count the
+// pairs held before it, g the new gradient
+struct md_min_loop {
+  int n, np, head, count;
+  const double *g;
+  double *q, *S[MD_MIN_MEMORY], *Y[MD_MIN_MEMORY];
+  double *partial;
+  md_min_state *state;
+};
 struct md_min_work {
   double *vec = nullptr;      // [MD_MIN_VECTORS][3][np]
-  double *partial = nullptr;  // reduction partials
+  double *partial = nullptr;  // eight sets of reduction partials
   double *scalar = nullptr;   // one reduced scalar
+  md_min_state *state = nullptr;
+  md_min_report *report = nullptr;  // pinned host memory
   int *bad = nullptr;         // a coordinate outside the fixed-point range
   int nc = 0;                 // live constraints (springs)
   int *p1 = nullptr, *p2 = nullptr;
   double *dist = nullptr;
-  double *spring_f = nullptr;  // [nc][3]: each spring's pull on its first atom
   int *cstart = nullptr;       // [np + 1]: by atom, its springs in clist
   int *clist = nullptr;        // spring c as c (first atom) or -c - 1 (second)
+  md_min_work() = default;
+  md_min_work(const md_min_work &) = delete;
+  ~md_min_work() {
+    if (report) (void)hipHostFree(report);
+  }
 };
 md_min_work *md_min_work_create(md_system *s, const std::vector<int> &p1, const std::vector<int> &p2,
                                 const std::vector<double> &dist);
 double *md_min_vec(md_system *s, md_min_work *w, int k);
-double md_min_dot(md_system *s, md_min_work *w, const double *a, const double *b);
-double md_min_absmax(md_system *s, md_min_work *w, const double *a);
-void md_min_lincomb(md_system *s, double *out, double a, const double *x, double b, const double *y);
 void md_min_positions_out(md_system *s, double *x);
 bool md_min_positions_in(md_system *s, md_min_work *w, const double *x);
-double md_min_gradient(md_system *s, md_min_work *w, const double *x, double kspring, double *g);
+// positions trial = x + step d (x itself without d), ready for an evaluation
+void md_min_trial(md_system *s, md_min_work *w, const double *x, const double *d, double step, double *trial);
+// after the evaluation: the objective's gradient at x, and the trial's report
+const md_min_report &md_min_gradient(md_system *s, md_min_work *w, const double *x, const double *d, double kspring,
+                                     double *g);
+// d = -g, or (x, g -> trial, L.g) L.q = -H L.g, and the direction's report
+const md_min_report &md_min_steepest(md_system *s, md_min_work *w, const double *g, double *d);
+const md_min_report &md_min_direction(md_system *s, md_min_work *w, md_min_loop L, const double *x,
+                                      const double *trial, const double *g);
 double md_min_constraint_error(md_system *s, md_min_work *w, const double *x);
 
 // ---- learned SHAKE warm start (warmstart.hip) ---------------------------------
