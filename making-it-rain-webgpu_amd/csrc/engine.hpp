@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -61,6 +62,26 @@ struct md_control {
   // what the integrator's waves add to since the last prologue, a 64-byte line
   // each: sum m v [3], SHAKE passes, cluster-steps
   alignas(64) int64_t part[MD_STEP_PARTS][8];
+};
+
+// what a control block says went wrong
+struct md_errors {
+  int64_t step_current;
+  uint32_t overflow, barostat_error, diverged;
+};
+
+// What the host and the device tell each other of a replica at the ends of a
+// call, in pinned memory: the host's step count and request for a rebuild ahead
+// of it, the errors and the energies after it.
+struct md_replica_io {
+  int64_t step;
+  uint32_t rebuild;
+  md_errors errors;
+  int64_t energy[MD_E_SLOTS];
+};
+struct md_replica_words {
+  md_control *ctl;
+  const int64_t *energy;
 };
 
 // The start of a step, by one wave per replica: advance the device step
@@ -213,6 +234,9 @@ struct md_group {
   // error (list or frame overflow, diverged constraints); read after every
   // stride so a failing run stops within one stride
   uint32_t *status = nullptr;
+  md_replica_io *io = nullptr;         // [R], pinned
+  md_replica_words *words = nullptr;   // [R], device: where the replicas' words are
+  uint32_t *status_out = nullptr;      // the status word as last reported, pinned
   int ws_mode = 0;          // cluster integrator: 0 plain, 1 recording, 2 learned
   bool graph_stale = false; // the captured stride no longer matches the kernels
   // profiling: events recorded by md_mark while `profiling` is set
@@ -336,6 +360,11 @@ struct md_system {
   // ---- the device barostat, when attached ------------------------------------
   md_baro *baro = nullptr;
 
+  // 3 np f64 in pinned memory: positions, velocities or forces on their way, and
+  // whose turn it is
+  double *transfer = nullptr;
+  std::mutex transfer_lock;
+
   // ---- the minimiser's work vectors, made on the first md_minimise ----------
   md_min_work *min_work = nullptr;
   std::vector<int> con_p1, con_p2;    // the constraints (host copies)
@@ -443,11 +472,6 @@ int &md_baro_step(md_system *s);            // steps since the last attempt
 // L-BFGS work vectors: MD_MIN_VECTORS f64 3N-vectors in planes [3][np]
 #define MD_MIN_MEMORY 6
 #define MD_MIN_VECTORS (6 + 2 * MD_MIN_MEMORY)
-// what a control block says went wrong
-struct md_errors {
-  int64_t step_current;
-  uint32_t overflow, barostat_error, diverged;
-};
 // the host's view of a trial point or of a search direction, in pinned memory
 struct md_min_report {
   double slope;   // gradient . direction

@@ -340,12 +340,12 @@ class NativeSystem:
         check(library().md_set_velocities(self.handle, _d(a)))
 
     def positions(self) -> np.ndarray:
-        out = np.zeros(3 * self.n)
+        out = np.empty(3 * self.n)
         check(library().md_get_positions(self.handle, _d(out)))
         return out
 
     def velocities(self) -> np.ndarray:
-        out = np.zeros(3 * self.n)
+        out = np.empty(3 * self.n)
         check(library().md_get_velocities(self.handle, _d(out)))
         return out
 
@@ -365,7 +365,7 @@ class NativeSystem:
 
     def evaluate(self, forces=True):
         """(total, groups[6], forces[3N] or None)."""
-        f = np.zeros(3 * self.n) if forces else None
+        f = np.empty(3 * self.n) if forces else None
         g = np.zeros(6)
         t = C.c_double()
         check(library().md_evaluate(self.handle, _d(f) if forces else None, _d(g), C.byref(t)))
