@@ -111,8 +111,7 @@ static void group_release(md_group *g) {
   if (g->bonded) md_bonded_group_free(g);
   if (g->pme) md_pme_group_free(g);
   if (g->integ) md_int_group_free(g);
-  if (g->io) hipHostFree(g->io);
-  if (g->status_out) hipHostFree(g->status_out);
+  if (g->io && g->own_stream) hipHostFree(g->io);
   for (void *p : g->allocations) hipFree(p);
   if (g->own_stream && g->stream) hipStreamDestroy(g->stream);
   for (md_system *s : g->reps) {
@@ -179,8 +178,11 @@ static md_group *group_create(const std::vector<md_system *> &reps, hipStream_t 
     std::vector<md_replica_words> words;
     for (md_system *s : reps) words.push_back({s->ctl, s->energy});
     g->words = md_group_upload(g, words);
-    MD_HIP(hipHostMalloc(&g->io, sizeof(md_replica_io) * reps.size()));
-    MD_HIP(hipHostMalloc(&g->status_out, sizeof(uint32_t)));
+    if (stream)
+      g->io = reps[0]->io;  // the system's own group
+    else
+      MD_HIP(hipHostMalloc(&g->io, sizeof(md_replica_io) * (reps.size() + 1)));
+    g->status_out = &g->io[reps.size()].rebuild;
     if (any_nb) {
       md_nb_group_setup(g);
       apply_tuned_schedule(g);
@@ -562,7 +564,8 @@ static void create(md_system *s, const md_system_desc *d, const md_run_options *
   s->mass_f = upload(s, mf);
   s->atom_param = upload(s, ap);
   s->energy = md_alloc<int64_t>(s, MD_E_SLOTS);
-  MD_HIP(hipHostMalloc(&s->transfer, sizeof(double) * 3 * (size_t)s->np));
+  MD_HIP(hipHostMalloc(&s->io, 2 * sizeof(md_replica_io) + sizeof(double) * 3 * (size_t)s->np));
+  s->transfer = reinterpret_cast<double *>(s->io + 2);
   s->ctl = md_alloc<md_control>(s, 1);
   s->term_atoms = upload(s, ta);
   s->term_param = upload(s, tp);
@@ -614,7 +617,7 @@ static void release(md_system *s) {
   delete s->min_work;  // its device memory is among the system's allocations
   md_baro_release(s);
   for (void *p : s->allocations) hipFree(p);
-  if (s->transfer) hipHostFree(s->transfer);
+  if (s->io) hipHostFree(s->io);
   if (s->stream) hipStreamDestroy(s->stream);
   delete s;
 }
@@ -899,10 +902,10 @@ static void run_steps(md_system *s, int64_t steps) {
   run_group(s->self, steps);
 }
 
-static void launch_evaluation(md_system *s) {
+static void launch_evaluation(md_system *s, bool rebuild) {
   md_group *grp = s->self;
   if (s->has_nonbonded) {
-    md_nb_build(grp, false);
+    md_nb_build(grp, false, rebuild);
     md_nb_pairs(grp, true);
   } else {
     md_step_prologue(grp, false);
@@ -918,12 +921,13 @@ static void evaluate(md_system *s, double *forces, double *groups, double *total
   MD_HIP(hipSetDevice(s->device));
   fault_tick(s, 1);
   md_group *grp = s->self;
+  const bool rebuild = s->need_rebuild;
   group_prepare(grp);
   if (census) {
     MD_HIP(hipMemsetAsync(&s->ctl->pair_census, 0, sizeof(int64_t), s->stream));
     MD_HIP(hipMemsetAsync(&s->ctl->pair_blocks, 0, sizeof(int64_t), s->stream));
   }
-  launch_evaluation(s);
+  launch_evaluation(s, rebuild);
   if (forces) {
     std::lock_guard<std::mutex> turn(s->transfer_lock);
     if (s->n > 0) k_export<int64_t><<<(3 * s->n + 255) / 256, 256, 0, s->stream>>>(s->force, s->transfer, s->n, s->np);
@@ -975,7 +979,7 @@ static const md_min_report &min_objective(lbfgs_state &L, const double *x, const
   s->need_rebuild = true;
   fault_tick(s, 1);
   if (s->momentum_dirty) group_prepare(s->self);
-  launch_evaluation(s);
+  launch_evaluation(s, true);
   s->need_rebuild = false;
   const md_min_report &r = md_min_gradient(s, L.w, d ? trial : x, d, L.kspring, g);
   if (r.bad) {

@@ -234,9 +234,9 @@ struct md_group {
   // error (list or frame overflow, diverged constraints); read after every
   // stride so a failing run stops within one stride
   uint32_t *status = nullptr;
-  md_replica_io *io = nullptr;         // [R], pinned
+  md_replica_io *io = nullptr;         // [R + 1], pinned
   md_replica_words *words = nullptr;   // [R], device: where the replicas' words are
-  uint32_t *status_out = nullptr;      // the status word as last reported, pinned
+  uint32_t *status_out = nullptr;      // the status word as last reported, in the last io
   int ws_mode = 0;          // cluster integrator: 0 plain, 1 recording, 2 learned
   bool graph_stale = false; // the captured stride no longer matches the kernels
   // profiling: events recorded by md_mark while `profiling` is set
@@ -360,8 +360,9 @@ struct md_system {
   // ---- the device barostat, when attached ------------------------------------
   md_baro *baro = nullptr;
 
-  // 3 np f64 in pinned memory: positions, velocities or forces on their way, and
-  // whose turn it is
+  // pinned memory: the own group's words (2), then 3 np f64 for positions,
+  // velocities or forces on their way, and whose turn it is
+  md_replica_io *io = nullptr;
   double *transfer = nullptr;
   std::mutex transfer_lock;
 
@@ -438,7 +439,9 @@ void md_nb_set_schedule(md_group *g, int seg_len, int waves);  // pair-kernel sc
 void md_nb_get_schedule(md_group *g, int *seg_len, int *waves);
 void md_nb_set_compact(md_group *g, bool compact);  // forces through the compacted pair schedule
 bool md_nb_get_compact(md_group *g);
-void md_nb_build(md_group *g, bool advance);    // the step's prologue, then the rebuild, gated per replica
+// the step's prologue, then the rebuild, gated per replica (`rebuild`: one of
+// the group's replicas is known to rebuild)
+void md_nb_build(md_group *g, bool advance, bool rebuild = false);
 void md_nb_pairs(md_group *g, bool energy);
 void md_bonded(md_group *g, bool energy);       // bonded.hip
 void md_bonded_forces(md_group *g);             // the terms' forces alone (no NonbondedForce)

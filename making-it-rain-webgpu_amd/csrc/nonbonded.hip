@@ -449,6 +449,10 @@ __global__ void __launch_bounds__(64 * MD_FRAME_WAVES) k_nb_clusters(const md_nb
 #define MD_SORT_THREADS 1024
 #define MD_SORT_ITEMS 12  // atoms a thread holds
 #define MD_SORT_CELLS 12288
+// A call that is known to rebuild pays the rebuild and not the waiting: past this
+// size the separate passes are quicker (9k atoms: 62 us, and 25 in six launches; 2,168:
+// 23 and 20, less than the launches).
+#define MD_SORT_SURE 4096
 __global__ void __launch_bounds__(MD_SORT_THREADS) k_nb_sort(const md_nb_args *__restrict__ T, int advance, int cells) {
   extern __shared__ int sort_lds[];
   __shared__ int active, wave_sum[16];
@@ -685,17 +689,28 @@ __device__ __forceinline__ void md_candidate(const md_build_ctx &c, const md_lis
 // Write the list entries of one super-cluster into its own region of the
 // entry arrays (entries_per_super entries from S * entries_per_super) and
 // their count, and count each J's entries for the transposed list.  One
-// workgroup of MD_LIST_WAVES wavefronts per S, lanes over candidate J
+// workgroup of WAVES wavefronts per S, lanes over candidate J
 // clusters, each wave a chunk of 64; a prefix count over the round's waves
 // puts the entries in the order of one wave's scan (ascending J), so the list
 // does not depend on the number of waves.  The search of one S is a chain of
 // dependent loads and int64 arithmetic per chunk and the replica waits for
 // its slowest S, so the chunks run side by side (a rebuild's search with one wave per S, the
 // images in lockstep and int64 box tests: 157 us at 2,168 atoms, 241 at 243k;
-// so: 50 and 136).
+// so: 45 and 137, of which keeping the images found while counting, where a
+// second pass found them again, gave 61 to 45, and 197 to 172 on 64 replicas).
 // A count past the region reports a list overflow.
-#define MD_LIST_WAVES 4
-__global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args *__restrict__ T, md_bmap map) {
+//
+// WAVES: on a small launch more waves put more of the chunks side by side (9k
+// atoms, 142 super-clusters: 39 us with 4, 29 with 8, 22 with 16; 31k, 490: 53,
+// 44, 52), on one that fills the chip they only wait for each other at the
+// counts (243k: 137, 167, 228; 64 replicas: 172, 218, 342), and below eight
+// super-clusters a wave there are no chunks for them (2,168 atoms, 34: 45, 46,
+// 50).
+#define MD_LIST_RESIDENT 4096  // waves of a launch that still counts as small
+#define MD_LIST_KEPT 3        // images of a candidate kept from the counting pass
+#define MD_LIST_BAD (1 << 30)  // in a kept entry: past the frame's range
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) k_nb_list(const md_nb_args *__restrict__ T, md_bmap map) {
   int S;
   const md_nb_args &A = md_nb_entry(T, map, S);
   md_control *ctl = A.ctl;
@@ -705,7 +720,7 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (S >= c.nsuper) return;
   __shared__ md_super_boxes boxes;
-  __shared__ int wave_count[MD_LIST_WAVES];
+  __shared__ int wave_count[WAVES];
   md_super_view V;
   const int first = S * 8;
   V.first = first;
@@ -727,7 +742,7 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
     if (lane == 0) wave_count[wave] = mine;
     __syncthreads();
     before = all = 0;
-    for (int w = 0; w < MD_LIST_WAVES; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const int u = wave_count[w];
       if (w < wave) before += u;
       all += u;
@@ -775,6 +790,7 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
   // the same order as a scan of every J >= S's first cluster, so the list is
   // the one that scan builds.
   __shared__ int cand[MD_LIST_CANDIDATES];
+  __shared__ int4 kept[MD_LIST_KEPT][64 * WAVES];
   int ncand = 0;
   const float rs = V.rs;
   int Kp[3] = {c.box.rectangular ? 0 : 1, c.box.rectangular ? 0 : 1, c.box.rectangular ? 0 : 1};
@@ -788,7 +804,7 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
     }
   }
   if (prefilter) {
-    for (int sb = 0; sb < c.nsuper; sb += 64 * MD_LIST_WAVES) {
+    for (int sb = 0; sb < c.nsuper; sb += 64 * WAVES) {
       const int SJ = sb + (int)threadIdx.x;
       bool near = false;
       if (SJ < c.nsuper && (SJ == S || md_lists_pair(S, SJ))) {
@@ -834,7 +850,7 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
   const int chunks = scan_all ? (c.nclusters + 63) / 64 : (ncand + 7) / 8;
   int written = 0;
   const int base_out = S * c.entries_per_super, region_end = base_out + c.entries_per_super;
-  for (int round = 0; round < chunks; round += MD_LIST_WAVES) {
+  for (int round = 0; round < chunks; round += WAVES) {
     const int chunk = round + wave;
     int J = c.nclusters;
     if (chunk >= chunks) {
@@ -847,18 +863,28 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
       J = k < ncand ? cand[k] * 8 + (lane & 7) : c.nclusters;
     }
     bool valid = J < c.nclusters;
-    // the count, and the entry itself when there is just one (always, without
-    // image enumeration): only several images need a second pass to write
-    int count = 0, one_mask = 0;
-    int64_t one_shift[3] = {0, 0, 0};
-    if (valid)
+    // the count, and the first few entries themselves (a candidate of a small
+    // box has two or three images within reach): only more images than that
+    // need a second pass to write
+    int count = 0;
+    int64_t jox = 0, joy = 0, joz = 0;  // J's frame origin from S's
+    auto entry = [&](int imask, int self, int64_t shx, int64_t shy, int64_t shz) {
+      bool bad = false;
+      int4 e = make_int4(md_frame_coord(jox + shx, bad), md_frame_coord(joy + shy, bad), md_frame_coord(joz + shz, bad),
+                         imask | (self << 8));
+      if (bad) e.w |= MD_LIST_BAD;
+      return e;
+    };
+    if (valid) {
+      const int SJ = J / 8;
+      jox = L.super_origin[SJ] - ox;
+      joy = L.super_origin[c.nsuper + SJ] - oy;
+      joz = L.super_origin[2 * c.nsuper + SJ] - oz;
       md_candidate(c, L, V, J, enumerate, K, [&](int imask, int self, int64_t shx, int64_t shy, int64_t shz) {
+        if (count < MD_LIST_KEPT) kept[count][threadIdx.x] = entry(imask, self, shx, shy, shz);
         ++count;
-        one_mask = imask | (self << 8);
-        one_shift[0] = shx;
-        one_shift[1] = shy;
-        one_shift[2] = shz;
       });
+    }
     int incl = count;
     for (int off = 1; off < 64; off <<= 1) {
       int v = __shfl_up(incl, off, 64);
@@ -868,27 +894,23 @@ __global__ void __launch_bounds__(64 * MD_LIST_WAVES) k_nb_list(const md_nb_args
     round_counts(__shfl(incl, 63, 64), before, all);
     if (valid && count) {
       int at = base_out + written + before + incl - count;
-      int SJ = J / 8;
-      int64_t jox = L.super_origin[SJ], joy = L.super_origin[c.nsuper + SJ], joz = L.super_origin[2 * c.nsuper + SJ];
-      auto write = [&](int meta, int64_t shx, int64_t shy, int64_t shz) {
+      const int listed = min(count, region_end - at);
+      auto write = [&](const int4 &e) {
         if (at < region_end) {
           L.entry_j[at] = J;
-          L.entry_imask[at] = meta;
-          // J's frame origin, moved into this image, in S's frame
-          bool bad = false;
-          L.entry_shift[at] = make_int4(md_frame_coord(jox + shx - ox, bad), md_frame_coord(joy + shy - oy, bad),
-                                        md_frame_coord(joz + shz - oz, bad), 0);
-          if (bad) ctl->overflow = 3;
-          atomicAdd(&L.j_count[J], 1);
+          L.entry_imask[at] = e.w & ~MD_LIST_BAD;
+          L.entry_shift[at] = make_int4(e.x, e.y, e.z, 0);  // J's frame origin in this image, in S's frame
+          if (e.w & MD_LIST_BAD) ctl->overflow = 3;
         }
         ++at;
       };
-      if (count == 1)
-        write(one_mask, one_shift[0], one_shift[1], one_shift[2]);
+      if (count <= MD_LIST_KEPT)
+        for (int u = 0; u < count; ++u) write(kept[u][threadIdx.x]);
       else
         md_candidate(c, L, V, J, enumerate, K, [&](int imask, int self, int64_t shx, int64_t shy, int64_t shz) {
-          write(imask | (self << 8), shx, shy, shz);
+          write(entry(imask, self, shx, shy, shz));
         });
+      if (listed > 0) atomicAdd(&L.j_count[J], listed);
     }
     written += all;
   }
@@ -2170,7 +2192,8 @@ struct md_nb_group {
   int pair_grid = 1;
   int seg_len = MD_SEGMENT;
   size_t sort_lds = 0;  // k_nb_sort's LDS, 0: the sort as separate passes
-  int sort_cells = 0;
+  int sort_cells = 0, most_atoms = 0;
+  int list_waves = 4;    // waves of a super-cluster's list search
   bool compact = false;  // forces through the compacted schedule
 };
 
@@ -2197,6 +2220,7 @@ void md_nb_group_setup(md_group *g) {
   // one workgroup sorts a replica while its rebuild costs less than the four
   // launches it saves on every step, which a rebuild comes every six or so of
   G->sort_cells = most_cells + 1;
+  G->most_atoms = most_atoms;
   if (most_atoms <= MD_SORT_THREADS * MD_SORT_ITEMS && most_cells < MD_SORT_CELLS) {
     G->sort_lds = sizeof(int) * (size_t)(G->sort_cells + most_atoms);
     if (G->sort_lds > 60 * 1024)
@@ -2205,6 +2229,9 @@ void md_nb_group_setup(md_group *g) {
   }
   G->frames = md_make_launch(g, frames);
   G->supers = md_make_launch(g, supers);
+  const int most_supers = *std::max_element(supers.begin(), supers.end());
+  for (int waves = 8; waves <= 16; waves *= 2)
+    if (G->supers.total * waves <= MD_LIST_RESIDENT && 8 * waves <= most_supers) G->list_waves = waves;
   G->slots = md_make_launch(g, slots);
   G->seg.map.start = md_group_alloc<int>(g, R + 1);
   G->seg.map.R = R;
@@ -2266,11 +2293,11 @@ void md_nb_group_free(md_group *g) {
   g->nb = nullptr;
 }
 
-void md_nb_build(md_group *g, bool advance) {
+void md_nb_build(md_group *g, bool advance, bool rebuild) {
   auto &G = nbg(g);
   hipStream_t st = g->stream;
   const md_nb_args *T = G.table;
-  if (G.sort_lds) {
+  if (G.sort_lds && !(rebuild && G.most_atoms > MD_SORT_SURE)) {
     md_mark(g, MD_PHASE_BUILD);
     k_nb_sort<<<(int)g->reps.size(), MD_SORT_THREADS, G.sort_lds, st>>>(T, advance ? 1 : 0, G.sort_cells);
   } else {
@@ -2283,7 +2310,11 @@ void md_nb_build(md_group *g, bool advance) {
     k_nb_clusters<<<G.frames.total, 64 * MD_FRAME_WAVES, 0, st>>>(T, G.frames.map);
   }
   md_mark(g, MD_PHASE_SEARCH);
-  k_nb_list<<<G.supers.total, 64 * MD_LIST_WAVES, 0, st>>>(T, G.supers.map);
+  switch (G.list_waves) {
+    case 16: k_nb_list<16><<<G.supers.total, 64 * 16, 0, st>>>(T, G.supers.map); break;
+    case 8: k_nb_list<8><<<G.supers.total, 64 * 8, 0, st>>>(T, G.supers.map); break;
+    default: k_nb_list<4><<<G.supers.total, 64 * 4, 0, st>>>(T, G.supers.map);
+  }
   k_nb_starts<<<G.scan.total, 1024, 0, st>>>(T, G.scan.map);
   md_mark(g, MD_PHASE_MASKS);
   k_nb_masks<<<G.supers.total, MD_MASK_THREADS, 0, st>>>(T, G.supers.map);
