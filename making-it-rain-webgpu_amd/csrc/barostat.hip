@@ -204,21 +204,6 @@ __global__ void k_baro_restore(const md_baro_dev *B, int64_t *pos, const int64_t
   for (int d = 0; d < 3; ++d) pos[(size_t)d * np + i] = saved[(size_t)d * np + i];
 }
 
-// the step's force kernels with energies on, into the energy slots
-static void baro_energy(md_group *g, bool nb) {
-  if (nb) {
-    md_nb_build(g, false);
-    md_nb_pairs(g, true);
-  } else {
-    md_step_prologue(g, false);
-  }
-  md_bonded(g, true);
-  if (nb)
-    md_pme(g, true);
-  else
-    md_bonded_forces(g);
-}
-
 static void baro_box_constants(md_group *g, const double *box, bool nb) {
   md_bonded_box_from_device(g, box);
   if (nb) {
@@ -233,12 +218,12 @@ void md_baro_attempt(md_system *s) {
   const bool nb = g->nb != nullptr;
   const md_energy_consts ek = md_energy_constants(s);
   k_baro_prepare<<<1, 1, 0, g->stream>>>(s->ctl);
-  baro_energy(g, nb);
+  md_force_kernels(g, false, true, false);
   k_baro_propose<<<1, 1, 0, g->stream>>>(B.dev, s->energy, ek, B.seed, s->has_nonbonded ? s->cutoff : 0.0, s->ctl);
   k_baro_scale<<<(B.nmol + 63) / 64, 64, 0, g->stream>>>(B.dev, B.mol_start, B.mol_atoms, B.nmol, s->pos, B.saved,
                                                         s->resid, s->np, s->ctl);
   baro_box_constants(g, dev_box(B), nb);
-  baro_energy(g, nb);
+  md_force_kernels(g, false, true, false);
   k_baro_decide<<<1, 1, 0, g->stream>>>(B.dev, s->energy, ek, B.seed, B.pressure, B.kt, B.nmol, s->ctl);
   k_baro_restore<<<(s->n + 255) / 256, 256, 0, g->stream>>>(B.dev, s->pos, B.saved, s->n, s->np);
   baro_box_constants(g, dev_box(B), nb);

@@ -292,13 +292,13 @@ void md_bonded_group_free(md_group *g) {
   g->bonded = nullptr;
 }
 
-void md_bonded(md_group *g, bool energy) {
+void md_bonded(md_group *g, bool energy, hipStream_t st) {
   auto &G = bg(g);
   if (G.terms.total == 0) return;
   if (energy)
-    k_terms<true><<<G.terms.total, 256, 0, g->stream>>>(G.table, G.terms.map);
+    k_terms<true><<<G.terms.total, 256, 0, st>>>(G.table, G.terms.map);
   else
-    k_terms<false><<<G.terms.total, 256, 0, g->stream>>>(G.table, G.terms.map);
+    k_terms<false><<<G.terms.total, 256, 0, st>>>(G.table, G.terms.map);
   MD_HIP(hipGetLastError());
 }
 

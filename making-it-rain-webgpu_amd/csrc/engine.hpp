@@ -215,6 +215,8 @@ struct md_group {
   int device = 0;
   hipStream_t stream = nullptr;
   bool own_stream = false;
+  hipStream_t side = nullptr;  // the mesh's and the bonded terms' stream
+  hipEvent_t forked = nullptr, joined = nullptr;
   std::vector<md_system *> reps;
   md_group **owner = nullptr;  // cleared when the group is released
   int max_cluster_atoms = 0;
@@ -439,13 +441,17 @@ void md_nb_set_schedule(md_group *g, int seg_len, int waves);  // pair-kernel sc
 void md_nb_get_schedule(md_group *g, int *seg_len, int *waves);
 void md_nb_set_compact(md_group *g, bool compact);  // forces through the compacted pair schedule
 bool md_nb_get_compact(md_group *g);
-// the step's prologue, then the rebuild, gated per replica (`rebuild`: one of
-// the group's replicas is known to rebuild)
-void md_nb_build(md_group *g, bool advance, bool rebuild = false);
+// the step's prologue, then the rebuild, gated per replica: the cell sort
+// (`rebuild`: one of the group's replicas is known to rebuild) and the list
+void md_nb_sort(md_group *g, bool advance, bool rebuild);
+void md_nb_search(md_group *g);
 void md_nb_pairs(md_group *g, bool energy);
-void md_bonded(md_group *g, bool energy);       // bonded.hip
+void md_bonded(md_group *g, bool energy, hipStream_t st);  // bonded.hip
 void md_bonded_forces(md_group *g);             // the terms' forces alone (no NonbondedForce)
-void md_pme(md_group *g, bool energy);          // pme.hip: the mesh, then every atom's force
+void md_pme(md_group *g, bool energy, hipStream_t st);  // pme.hip: the mesh
+void md_forces(md_group *g, bool energy);               // pme.hip: every atom's force
+// api.hip: the force kernels of one step or evaluation
+void md_force_kernels(md_group *g, bool advance, bool energy, bool rebuild);
 // integrate.hip: advance the step counters (or, for an evaluation, clear the
 // energies) and latch each replica's rebuild request (its own displacement
 // test, or `force_pending` set by the host)

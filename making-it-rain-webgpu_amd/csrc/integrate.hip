@@ -894,7 +894,7 @@ __global__ void __launch_bounds__(256) k_constrain(const md_int_args *__restrict
   }
 }
 
-// the start of a step, where no other kernel runs it (md_nb_build): one wave per
+// the start of a step, where no other kernel runs it (md_nb_sort): one wave per
 // replica
 __global__ void __launch_bounds__(64) k_step_prologue(const md_int_args *__restrict__ T, int advance) {
   const md_int_args &A = T[blockIdx.x];

@@ -2293,7 +2293,7 @@ void md_nb_group_free(md_group *g) {
   g->nb = nullptr;
 }
 
-void md_nb_build(md_group *g, bool advance, bool rebuild) {
+void md_nb_sort(md_group *g, bool advance, bool rebuild) {
   auto &G = nbg(g);
   hipStream_t st = g->stream;
   const md_nb_args *T = G.table;
@@ -2309,6 +2309,13 @@ void md_nb_build(md_group *g, bool advance, bool rebuild) {
     k_nb_rank<<<G.atoms.total, 256, 0, st>>>(T, G.atoms.map);
     k_nb_clusters<<<G.frames.total, 64 * MD_FRAME_WAVES, 0, st>>>(T, G.frames.map);
   }
+  MD_HIP(hipGetLastError());
+}
+
+void md_nb_search(md_group *g) {
+  auto &G = nbg(g);
+  hipStream_t st = g->stream;
+  const md_nb_args *T = G.table;
   md_mark(g, MD_PHASE_SEARCH);
   switch (G.list_waves) {
     case 16: k_nb_list<16><<<G.supers.total, 64 * 16, 0, st>>>(T, G.supers.map); break;

@@ -1025,10 +1025,9 @@ void md_pme_group_free(md_group *g) {
   g->pme = nullptr;
 }
 
-void md_pme(md_group *g, bool energy) {
+void md_pme(md_group *g, bool energy, hipStream_t st) {
   auto &G = pg(g);
   if (G.spread.total == 0) return;
-  hipStream_t st = g->stream;
   const md_pme_table *T = G.table;
   k_pme_spread<<<G.spread.total, MD_SPREAD_THREADS, 0, st>>>(T, G.spread.map, G.spread_per);
   md_mark(g, MD_PHASE_FFT);
@@ -1048,7 +1047,13 @@ void md_pme(md_group *g, bool energy) {
     k_pme_y<<<G.ylines.total, 256, G.ly, st>>>(T, G.ylines.map, 1.0f);
     k_pme_z_inverse<<<G.zrows.total, 256, G.lz, st>>>(T, G.zrows.map);
   }
+  MD_HIP(hipGetLastError());
+}
+
+void md_forces(md_group *g, bool energy) {
+  auto &G = pg(g);
+  if (G.spread.total == 0) return;
   md_mark(g, MD_PHASE_FORCES);
-  k_forces<<<G.gather.total, MD_FORCES_THREADS, 0, st>>>(T, G.gather.map, energy ? 1 : 0);
+  k_forces<<<G.gather.total, MD_FORCES_THREADS, 0, g->stream>>>(G.table, G.gather.map, energy ? 1 : 0);
   MD_HIP(hipGetLastError());
 }
