@@ -242,8 +242,9 @@ md_err md_batch_profile_steps(md_batch *batch, int32_t steps, double *ms);
 
 /* The pair kernel's autotuner.  No counterpart upstream: the WebGPU loop
  * has fixed workgroup shapes (src/gpu/loop.ts:171).  It times the pair
- * kernel's schedules -- list entries per work unit (8 to 32), waves per
- * launch, and the direct or the compacted evaluation (the in-cutoff pairs of two entries packed densely into full waves) -- on the
+ * kernel's schedules -- list entries per segment (8 to 32), waves per launch
+ * (each takes a fixed run of segments), and the direct or the compacted
+ * evaluation (the in-cutoff pairs packed densely into full waves) -- on the
  * group's own replicas, `steps` steps each, keeps the fastest, and caches it
  * per (replica count, atom-count bucket, triclinic or not) for launch groups
  * created later in the process.  No schedule changes any bit; the timed

@@ -128,7 +128,7 @@ static void group_release(md_group *g) {
 
 // ---- the pair-kernel autotuner's cache ----------------------------------------
 //
-// Tuned schedules (entries per work unit, resident waves) keyed by what sets
+// Tuned schedules (entries per segment, waves) keyed by what sets
 // the best one: the number of replicas, the launch's atom count in
 // half-octave buckets, and whether any cell is triclinic.  A new launch group
 // whose key has an entry starts from it.

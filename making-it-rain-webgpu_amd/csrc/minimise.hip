@@ -21,7 +21,7 @@
 // order), the two-loop recursion takes one launch per correction vector with
 // its coefficients kept on the device, and a trial point's values come back
 // together.  Ten iterations a round at 9k atoms, 98 evaluations: 57.7 ms before,
-// 29.3 now.
+// 29.3 so (and 21.2 with what the evaluation has gained since).
 #include "engine.hpp"
 
 #define MD_MIN_BLOCK 256

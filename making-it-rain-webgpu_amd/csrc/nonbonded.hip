@@ -2245,10 +2245,10 @@ void md_nb_group_setup(md_group *g) {
   md_nb_group_refresh(g);
 }
 
-// The pair kernel's schedule: list entries per work unit (a multiple of
+// The pair kernel's schedule: list entries per segment (a multiple of
 // MD_SEGMENT; the i-force rounding happens per MD_SEGMENT entries, so any
-// length gives the same bits) and the resident grid of waves that draws units
-// from the counter.  waves <= 0 keeps the current grid.
+// length gives the same bits) and the launch's waves, each of which takes a
+// fixed run of segments.  waves <= 0 keeps the current number.
 void md_nb_set_schedule(md_group *g, int seg_len, int waves) {
   auto &G = nbg(g);
   if (seg_len % MD_SEGMENT || seg_len < MD_SEGMENT || seg_len > 32 * MD_SEGMENT)
