@@ -50,11 +50,11 @@ FP32_PEAK_TFLOPS = 157.3   # MI355X published FP32 vector peak
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E
 PAIR_FLOPS = 76            # algorithmic FP32 flops per in-cutoff pair
 # HBM bytes per launch of the batched pair kernel on this ensemble, by the
-# work-unit length in use (the autotuner picks 64 or 128 entries here):
+# segment length in use (the autotuner picks 16 entries here, 8 is the default):
 # FETCH_SIZE + WRITE_SIZE from two rocprofv3 --pmc passes over
 # `bench.py --traffic-probe 3 --pair-segment N`, each scaled by its reading
 # for a 256 MiB device copy (profiles/k_nb_pairs_ensemble64_traffic.md)
-PAIR_TRAFFIC_BYTES = {64: 465.0e6, 128: 436.7e6}
+PAIR_TRAFFIC_BYTES = {8: 402.2e6, 16: 397.1e6}
 DT_PS = 0.002
 METRIC = "aggregate ns/day at 2 fs (batched+learned vs plain, same GPU, fixed force error)"
 
