@@ -223,13 +223,14 @@ __global__ void __launch_bounds__(MD_SPREAD_THREADS) k_pme_spread(const md_pme_t
   __syncthreads();
   // one pass over all of them if their joint box fits the tile
   md_spread_box box = boxes[0];
-  int passes = 1;
+  int passes = 1, from = 0;  // a single pass starts with super-cluster `from`, the box's if it is only one's
   int shift[3] = {0, 0, 0};  // the second one's reference base from the box's
   if (count == 2) {
     const md_spread_box other = boxes[1];
     if (other.lo[0] <= other.hi[0]) {
       if (box.lo[0] > box.hi[0]) {
         box = other;
+        from = 1;
       } else {
         int joint = 1;
         md_spread_box both = box;
@@ -254,8 +255,9 @@ __global__ void __launch_bounds__(MD_SPREAD_THREADS) k_pme_spread(const md_pme_t
     if (box.lo[0] > box.hi[0]) continue;  // no charged atom (uniform)
     int ext[3];
     for (int d = 0; d < 3; ++d) ext[d] = box.hi[d] - box.lo[d] + MD_PME_ORDER;
-    const int volume = ext[0] * ext[1] * ext[2], first = passes == 2 ? pass : 0, last = passes == 2 ? pass + 1 : count;
-    if (volume > MD_SPREAD_TILE) {  // one super-cluster alone
+    const int volume = ext[0] * ext[1] * ext[2], first = passes == 2 ? pass : from, last = passes == 2 ? pass + 1 : count;
+    // one super-cluster alone: with two in the pass the box fits, or the other has no charge
+    if (volume > MD_SPREAD_TILE) {
       const int base[3] = {bases[first][0][lane], bases[first][1][lane], bases[first][2][lane]};
       if (base[0] == INT_MIN) continue;
       const int gx = md_wrap(base[0] + wave, P.nx);
