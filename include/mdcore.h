@@ -112,7 +112,8 @@ typedef struct {
   uint32_t seed;
   int32_t integrator;          /* 0 LangevinMiddle, 1 Verlet (NVE gate) */
   double verlet_skin;          /* nm; < 0 picks the default (0.15, nonbonded.ts:227) */
-  int32_t mesh[3];             /* PME mesh override; 0 = from the system or the box */
+  int32_t mesh[3];             /* PME mesh override; 0 = from the system or the box; 13-smooth,
+                                  5 to 640 points an axis */
   int32_t device;              /* HIP device ordinal */
   int32_t max_batch;           /* steps per captured HIP graph (maxBatch,
                                   src/gpu/loop.ts:151-158); 0 = 50, 1 = every

@@ -470,6 +470,9 @@ static void create(md_system *s, const md_system_desc *d, const md_run_options *
       if (r != 1)
         throw md_error(MD_ERR_NOT_SMOOTH, "PME mesh size " + std::to_string(g) + " has a prime factor above 13 (" +
                                               std::to_string(r) + " is left); mesh sizes must be 13-smooth");
+      if (g > MD_PME_MOST_POINTS)
+        throw md_error(MD_ERR_INVALID_ARGUMENT, "PME mesh size " + std::to_string(g) + ": an axis takes at most " +
+                                                    std::to_string(MD_PME_MOST_POINTS) + " points");
       s->grid[a] = g;
     }
   }

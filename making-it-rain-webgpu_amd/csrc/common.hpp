@@ -24,6 +24,7 @@
 #define MD_BAROSTAT_DOMAIN 0x6a09e667u
 #define MD_VELOCITY_DOMAIN 0xbb67ae85u
 #define MD_PME_ORDER 5
+#define MD_PME_MOST_POINTS 640  // of a mesh axis
 #define MD_CLUSTER 8            // atoms per cluster
 #define MD_SUPER 64             // atoms per super-cluster (one wavefront: 8 clusters)
 #define MD_SEGMENT 8            // list entries per wavefront work unit, at least

@@ -23,7 +23,8 @@
 #include "engine.hpp"
 
 #define PME_MAX_STAGES 12
-#define PME_BATCH 16
+#define PME_BATCH 16          // lines of a workgroup, at most (md_lines)
+#define PME_LDS (160 * 1024)  // a CU's LDS
 #define MD_PHI_PAD 4  // values a row of the potential repeats past its end (md_row5)
 
 struct md_fft_plan {
@@ -31,6 +32,8 @@ struct md_fft_plan {
   int nstages;
   int radix[PME_MAX_STAGES];
   int tw;  // offset of this length's twiddle table
+  int lines;      // lines of a workgroup
+  int runs, per;  // for lines along y or x: a row's runs of consecutive kz, and the kz of a run
 };
 
 struct md_pme_args {
@@ -415,6 +418,15 @@ __device__ __forceinline__ void md_fft_stage(const md_fft_io &io, Ext &ext, int 
 // consecutive lines meets each bank once
 __host__ __device__ inline int md_pitch(int n) { return n | 1; }
 
+// A line pass's LDS: two buffers of `lines` lines and the twiddles.  PME_BATCH
+// lines of up to 616 points fit; of more points as many as fit (15 of 640).
+static size_t md_lines_lds(int n, int lines) { return sizeof(float2) * (2 * (size_t)lines * md_pitch(n) + n); }
+static int md_lines(int n) {
+  int lines = PME_BATCH;
+  while (lines > 1 && md_lines_lds(n, lines) > PME_LDS) --lines;
+  return lines;
+}
+
 // `nlines` lines of length P.n, transformed with sign -1 (forward) or +1
 // (inverse) through the LDS buffers a and b.  The input is `src` (one of the
 // two, with its line and element strides) or, with a null src, the kernel's
@@ -514,28 +526,30 @@ struct md_ext_potential {
 };
 
 // z pass, forward: int64 rows -> f32 -> complex FFT -> first nz/2+1 values.
-// Clears the integer grid behind it.  Block = PME_BATCH rows.
+// Clears the integer grid behind it.  Block = P.pz.lines rows.
 __global__ void __launch_bounds__(256) k_pme_z_forward(const md_pme_table *__restrict__ T, md_bmap map) {
   extern __shared__ float2 lds[];
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  const int rows = P.nx * P.ny, r0 = blk * PME_BATCH, nl = min(PME_BATCH, rows - r0);
-  float2 *a = lds, *b = a + PME_BATCH * md_pitch(P.nz), *tw = b + PME_BATCH * md_pitch(P.nz);
+  const int rows = P.nx * P.ny, lines = P.pz.lines, r0 = blk * lines, nl = min(lines, rows - r0);
+  float2 *a = lds, *b = a + lines * md_pitch(P.nz), *tw = b + lines * md_pitch(P.nz);
   md_load_twiddles(tw, P.pz, P.tw);
   __syncthreads();
   md_ext_charge ext{E.grid + (size_t)r0 * P.nz, E.cgrid + (size_t)r0 * P.nzc, P.nz, P.nzc};
   md_fft(a, b, nullptr, 0, 0, true, ext, nl, P.pz, tw, -1.0f);
 }
 
-// Lines along y or x are taken a run of consecutive kz at a time, at most
-// PME_BATCH, the runs of one row of equal length (33 values as three runs of
-// 11, not 16, 16 and 1).
-__host__ __device__ inline int md_kz_runs(int nzc) { return (nzc + PME_BATCH - 1) / PME_BATCH; }
-__device__ __forceinline__ void md_kz_run(int nzc, int run, int &z0, int &nl) {
-  const int runs = md_kz_runs(nzc), per = (nzc + runs - 1) / runs;
-  z0 = run * per;
-  nl = max(0, min(per, nzc - z0));
+// Lines along y or x are taken a run of consecutive kz at a time, at most as
+// many as a workgroup holds, the runs of one row of equal length (33 values as
+// three runs of 11, not 16, 16 and 1).
+static void md_set_runs(md_fft_plan &p, int nzc) {
+  p.runs = (nzc + p.lines - 1) / p.lines;
+  p.per = (nzc + p.runs - 1) / p.runs;
+}
+__device__ __forceinline__ void md_kz_run(const md_fft_plan &p, int nzc, int run, int &z0, int &nl) {
+  z0 = run * p.per;
+  nl = max(0, min(p.per, nzc - z0));
 }
 
 // y pass: lines along y at fixed (x, kz)
@@ -544,10 +558,10 @@ __global__ void __launch_bounds__(256) k_pme_y(const md_pme_table *__restrict__ 
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  const int runs = md_kz_runs(P.nzc), x = blk / runs;
+  const int runs = P.py.runs, x = blk / runs;
   int z0, nl;
-  md_kz_run(P.nzc, blk - x * runs, z0, nl);
-  float2 *a = lds, *b = a + PME_BATCH * md_pitch(P.ny), *tw = b + PME_BATCH * md_pitch(P.ny);
+  md_kz_run(P.py, P.nzc, blk - x * runs, z0, nl);
+  float2 *a = lds, *b = a + P.py.lines * md_pitch(P.ny), *tw = b + P.py.lines * md_pitch(P.ny);
   md_load_twiddles(tw, P.py, P.tw);
   __syncthreads();
   float2 *plane = E.cgrid + (size_t)x * P.ny * P.nzc + z0;
@@ -566,11 +580,11 @@ __global__ void __launch_bounds__(256) k_pme_x_convolve(const md_pme_table *__re
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
   int64_t *energy = E.energy;
-  const int runs = md_kz_runs(P.nzc), y = blk / runs;
+  const int runs = P.px.runs, y = blk / runs;
   int z0, nl;
-  md_kz_run(P.nzc, blk - y * runs, z0, nl);
+  md_kz_run(P.px, P.nzc, blk - y * runs, z0, nl);
   const int pitch = md_pitch(P.nx);
-  float2 *a = lds, *b = a + PME_BATCH * pitch, *tw = b + PME_BATCH * pitch;
+  float2 *a = lds, *b = a + P.px.lines * pitch, *tw = b + P.px.lines * pitch;
   md_load_twiddles(tw, P.px, P.tw);
   __syncthreads();
   float2 *const at = E.cgrid + (size_t)y * P.nzc + z0;
@@ -618,8 +632,8 @@ __global__ void __launch_bounds__(256) k_pme_z_inverse(const md_pme_table *__res
   int blk;
   const md_pme_table &E = md_pme_entry(T, map, blk);
   const md_pme_args &P = E.P;
-  const int rows = P.nx * P.ny, r0 = blk * PME_BATCH, nl = min(PME_BATCH, rows - r0);
-  float2 *a = lds, *b = a + PME_BATCH * md_pitch(P.nz), *tw = b + PME_BATCH * md_pitch(P.nz);
+  const int rows = P.nx * P.ny, lines = P.pz.lines, r0 = blk * lines, nl = min(lines, rows - r0);
+  float2 *a = lds, *b = a + lines * md_pitch(P.nz), *tw = b + lines * md_pitch(P.nz);
   md_load_twiddles(tw, P.pz, P.tw);
   __syncthreads();
   md_ext_potential ext{E.cgrid + (size_t)r0 * P.nzc, P.nzc, 1, E.phi + (size_t)r0 * (P.nz + MD_PHI_PAD), P.nz, P.nzc};
@@ -808,6 +822,7 @@ static md_fft_plan make_plan(int n, int tw_offset) {
   md_fft_plan p{};
   p.n = n;
   p.tw = tw_offset;
+  p.lines = md_lines(n);
   int r = n;
   // radix 4 first, then 2, 3, 5, 7, then any remaining prime (direct DFT)
   while (r % 4 == 0) {
@@ -869,6 +884,8 @@ void md_pme_setup(md_system *s) {
   H.px = make_plan(nx, off[0]);
   H.py = make_plan(ny, off[1]);
   H.pz = make_plan(nz, off[2]);
+  md_set_runs(H.px, s->pme_nzc);
+  md_set_runs(H.py, s->pme_nzc);
   std::vector<float> mod;
   for (int d = 0; d < 3; ++d)
     for (double v : moduli(lens[d])) mod.push_back((float)v);
@@ -957,23 +974,25 @@ void md_pme_group_setup(md_group *g) {
   auto *G = new md_pme_group();
   g->pme = G;
   std::vector<int> spread, zrows, ylines, xlines, gather, planes;
-  int mx = 0, my = 0, mz = 0;
+  int my = 0, mz = 0;
   long supers = 0;
   for (md_system *s : g->reps) supers += s->has_nonbonded ? s->nb.nslots / 64 : 0;
   G->spread_per = supers >= MD_SPREAD_PAIRED ? 2 : 1;
   for (md_system *s : g->reps) {
     bool on = s->has_nonbonded;
-    int nx = s->pme_nx, ny = s->pme_ny, nz = s->pme_nz, kzb = md_kz_runs(s->pme_nzc);
+    int nx = s->pme_nx, ny = s->pme_ny, nz = s->pme_nz;
     spread.push_back(on ? (s->nb.nslots / 64 + G->spread_per - 1) / G->spread_per : 0);
-    zrows.push_back(on ? (nx * ny + PME_BATCH - 1) / PME_BATCH : 0);
-    ylines.push_back(on ? nx * kzb : 0);
-    xlines.push_back(on ? ny * kzb : 0);
+    zrows.push_back(on ? (nx * ny + pme_host(s).pz.lines - 1) / pme_host(s).pz.lines : 0);
+    ylines.push_back(on ? nx * pme_host(s).py.runs : 0);
+    xlines.push_back(on ? ny * pme_host(s).px.runs : 0);
     gather.push_back(on ? s->nb.nslots / MD_FORCES_THREADS : 0);
     planes.push_back(on ? nx : 0);
     if (on) {
-      mx = std::max(mx, nx);
       my = std::max(my, ny);
       mz = std::max(mz, nz);
+      G->lx = std::max(G->lx, md_lines_lds(nx, md_lines(nx)));
+      G->ly = std::max(G->ly, md_lines_lds(ny, md_lines(ny)));
+      G->lz = std::max(G->lz, md_lines_lds(nz, md_lines(nz)));
     }
   }
   G->spread = md_make_launch(g, spread);
@@ -985,9 +1004,6 @@ void md_pme_group_setup(md_group *g) {
   // planes of up to about 64^2 in LDS, two workgroups to a CU
   G->lyz = sizeof(float2) * (2 * (size_t)md_plane_buffer(my, mz) + my + mz);
   G->fused_yz = G->lyz <= 68 * 1024;
-  G->lz = sizeof(float2) * (2 * PME_BATCH * md_pitch(mz) + mz);
-  G->ly = sizeof(float2) * (2 * PME_BATCH * md_pitch(my) + my);
-  G->lx = sizeof(float2) * (2 * PME_BATCH * md_pitch(mx) + mx);
   auto allow = [](std::initializer_list<const void *> kernels, size_t lds) {
     if (lds > 64 * 1024)
       for (auto *k : kernels) MD_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
