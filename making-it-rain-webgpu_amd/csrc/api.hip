@@ -1107,6 +1107,8 @@ static void minimise_system(md_system *s, int max_iterations, double tolerance, 
     L.S[k] = md_min_vec(s, w, 6 + k);
     L.Y[k] = md_min_vec(s, w, 6 + MD_MIN_MEMORY + k);
   }
+  // a search that ended between a trial point and its report left its flag
+  MD_HIP(hipMemsetAsync(w->bad, 0, sizeof(int), s->stream));
   const double ctol = s->opt.constraint_tolerance, work = std::max(1e-4, ctol);
   L.kspring = 100.0 / work;
   md_constrain(s->self, 0, work);
