@@ -217,13 +217,16 @@ void md_baro_attempt(md_system *s) {
   md_group *g = s->self;
   const bool nb = g->nb != nullptr;
   const md_energy_consts ek = md_energy_constants(s);
+  // Both evaluations rebuild the list for certain, and the sort is told (its one
+  // workgroup is the slower way to a rebuild past 4,096 atoms): an attempt takes
+  // 15 us less at 4,140 atoms, 75 at 9k, 120 at 12,270.
   k_baro_prepare<<<1, 1, 0, g->stream>>>(s->ctl);
-  md_force_kernels(g, false, true, false);
+  md_force_kernels(g, false, true, true);
   k_baro_propose<<<1, 1, 0, g->stream>>>(B.dev, s->energy, ek, B.seed, s->has_nonbonded ? s->cutoff : 0.0, s->ctl);
   k_baro_scale<<<(B.nmol + 63) / 64, 64, 0, g->stream>>>(B.dev, B.mol_start, B.mol_atoms, B.nmol, s->pos, B.saved,
                                                         s->resid, s->np, s->ctl);
   baro_box_constants(g, dev_box(B), nb);
-  md_force_kernels(g, false, true, false);
+  md_force_kernels(g, false, true, true);
   k_baro_decide<<<1, 1, 0, g->stream>>>(B.dev, s->energy, ek, B.seed, B.pressure, B.kt, B.nmol, s->ctl);
   k_baro_restore<<<(s->n + 255) / 256, 256, 0, g->stream>>>(B.dev, s->pos, B.saved, s->n, s->np);
   baro_box_constants(g, dev_box(B), nb);

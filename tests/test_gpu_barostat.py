@@ -196,3 +196,25 @@ def test_device_barostat_leaves_tables_matching_its_box(npt):
     assert max(gerr) < 1e-5
     assert rel.max() < 2e-6
     t.destroy()
+
+
+def test_device_attempt_past_the_one_workgroup_sort():
+    """Past 4,096 atoms an attempt's evaluations sort in separate passes and the
+    steps around it, up to 12,288, in one workgroup: decision, box and positions
+    as the host's attempt, with the tolerances of a first attempt above."""
+    b = synthetic.build(0, 1380, 0, "cube", 78, barostat=True)
+    e = HipEngine(b.system, b.state, RunOptions(seed=4))
+    e.minimise(50, 100.0)
+    e.setVelocitiesToTemperature(300.0, 4)
+    dev = _twin(b, e, barostat="device")
+    host = _twin(b, e, barostat="host")
+    dev.run(25)
+    host.run(25)
+    d, h = dev.lastBarostat, host.lastBarostat
+    assert dev.barostatAttempts == host.barostatAttempts == 1
+    assert d["last_accepted"] == h["last_accepted"]
+    assert abs(d["last_energy_before"] - h["last_energy_before"]) < 1e-12 * abs(h["last_energy_before"])
+    np.testing.assert_allclose(np.asarray(dev.boxVectors()), np.asarray(host.boxVectors()), rtol=1e-14, atol=0)
+    assert np.max(np.abs(dev.positions() - host.positions())) < 1e-8
+    for x in (e, dev, host):
+        x.destroy()
