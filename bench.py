@@ -278,7 +278,7 @@ def run_ensemble(args):
         log(f"pair schedule set to {args.pair_schedule}, {args.pair_segment or 'unchanged'} entries per unit")
     if tune:
         log(f"autotuned pair schedule: {tune['segment_entries']} entries per unit, {tune['pair_waves']} waves "
-            f"({tune['ms_per_step']:.3f} ms/step phase by phase) vs the default {tune['default_segment_entries']}, "
+            f"({tune['ms_per_step']:.3f} ms/step) vs the default {tune['default_segment_entries']}, "
             f"{tune['default_pair_waves']} ({tune['default_ms_per_step']:.3f} ms/step)")
     # the work-unit length the timed run uses (its measured traffic, if any)
     unit_entries = args.pair_segment or (tune["segment_entries"] if tune else None)

@@ -246,13 +246,14 @@ md_err md_batch_profile_steps(md_batch *batch, int32_t steps, double *ms);
  * kernel's schedules -- list entries per segment (8 to 32), waves per launch
  * (each takes a fixed run of segments), and the direct or the compacted
  * evaluation (the in-cutoff pairs packed densely into full waves) -- on the
- * group's own replicas, `steps` steps each, keeps the fastest, and caches it
+ * group's own replicas, `steps` steps each as a run takes them (without a
+ * barostat's attempts), keeps the fastest, and caches it
  * per (replica count, atom-count bucket, triclinic or not) for launch groups
  * created later in the process.  No schedule changes any bit; the timed
  * steps are ordinary steps. */
 typedef struct {
   int32_t segment_entries, pair_waves;                 /* the schedule picked */
-  double ms_per_step;                                  /* its mean step, phase by phase */
+  double ms_per_step;                                  /* its mean step, as a run takes it */
   int32_t default_segment_entries, default_pair_waves; /* the schedule before tuning */
   double default_ms_per_step;
   int32_t candidates;                                  /* schedules timed */

@@ -9,6 +9,8 @@
 * A batch can be destroyed and its replicas go on alone; a replica
   destroyed first leaves the batch refusing to run.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -164,3 +166,25 @@ def test_autotuner_picks_a_schedule_and_the_batch_goes_on(replicas):
         err, _ = edge.rel_rms_edge(f, of, r.built.system, x, r.built.system.boxVectors, o.alpha())
         assert err < 2e-6
         e.destroy()
+
+
+def test_autotuner_times_steps_as_they_run():
+    """The reported times are those of a run's steps, which put the mesh beside
+    the pairs and replay a graph.  Steps timed phase by phase take 1.7 times as
+    long at this size; a quarter is left for noise and for rebuilds."""
+    b = synthetic.build(0, 700, 0, "cube", 3)
+    e = HipEngine(b.system, b.state, RunOptions(timeStep=0.001, friction=10.0, seed=1))
+    e.minimise(15, 100.0)
+    e.setVelocitiesToTemperature(300.0, 1)
+    e.run(400)
+    best = e._native.autotune(50)
+    e._native.set_pair_schedule(best["default_segment_entries"], best["default_pair_waves"], False)
+    e.run(400)
+    took = []
+    for _ in range(5):
+        start = time.perf_counter()
+        e.run(400)
+        took.append((time.perf_counter() - start) / 400 * 1e3)
+    print("reported", best["default_ms_per_step"], "as run", took)
+    assert 0.75 * min(took) < best["default_ms_per_step"] < 1.25 * min(took)
+    e.destroy()
