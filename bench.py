@@ -50,11 +50,11 @@ FP32_PEAK_TFLOPS = 157.3   # MI355X published FP32 vector peak
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E
 PAIR_FLOPS = 76            # algorithmic FP32 flops per in-cutoff pair
 # HBM bytes per launch of the batched pair kernel on this ensemble, by the
-# segment length in use (the autotuner picks 16 entries here, 8 is the default):
+# segment length in use (the autotuner picks among these, 8 is the default):
 # FETCH_SIZE + WRITE_SIZE from two rocprofv3 --pmc passes over
 # `bench.py --traffic-probe 3 --pair-segment N`, each scaled by its reading
 # for a 256 MiB device copy (profiles/k_nb_pairs_ensemble64_traffic.md)
-PAIR_TRAFFIC_BYTES = {8: 402.2e6, 16: 397.1e6}
+PAIR_TRAFFIC_BYTES = {8: 402.2e6, 16: 397.1e6, 32: 391.7e6}
 DT_PS = 0.002
 METRIC = "aggregate ns/day at 2 fs (batched+learned vs plain, same GPU, fixed force error)"
 
@@ -351,30 +351,34 @@ def run_ensemble(args):
 
     # ---- roofline of the dominant kernel, measured inside the batched step -----
     phases = batch.profileStep(args.profile_steps)
-    pairs = 0
+    pairs = entries = 0
     for e in engines:
         p, _ = e._native.pair_census()
         pairs += p
+        entries += e._native.list_flags()["tiles"]
     log("batched phases (ms): " + ", ".join(f"{k} {v:.4f}" for k, v in phases.items()))
     integ_gbs = 124.0 * total_atoms / (phases["integrate"] * 1e-3) / 1e9 if phases["integrate"] > 0 else 0.0
     meshes = [tuple(e.mesh) for e in engines]
     points = float(sum(m[0] * m[1] * m[2] for m in meshes))
 
-    def hbm(phase, nbytes):
-        ms = phases.get(phase, 0.0)
+    def hbm(ms, nbytes):
         gbs = nbytes / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
         return {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
                 "bytes": nbytes, "ms": ms}
 
     # algorithmic bytes per launch, per unit of work: spreading 28 B/atom + 8 B
     # per grid point; the five transform passes (C2C forward + inverse, 3 axes
-    # each) 96 B/point plus the convolution's 16; gathering 28 B/atom + 8 B per
-    # point + 24 B/atom of force
+    # each) 96 B/point plus the convolution's 16; the one pass that makes the
+    # forces (timed whole: the profile halves it between its two phases) 28
+    # B/atom in, 24 B/atom out, 48 B/atom of i forces read and cleared, 96 B of
+    # j forces per list entry, 4 B/point (without the bonded terms' pieces)
     pme_roofline = {
-        "pme_spread": hbm("pme_spread", 28.0 * total_atoms + 8.0 * points),
-        "pme_fft_convolve": hbm("pme_fft_convolve", (96.0 + 16.0) * points),
-        "pme_gather": hbm("pme_gather", (28.0 + 24.0) * total_atoms + 8.0 * points),
+        "pme_spread": hbm(phases["pme_spread"], 28.0 * total_atoms + 8.0 * points),
+        "pme_fft_convolve": hbm(phases["pme_fft_convolve"], (96.0 + 16.0) * points),
+        "forces": hbm(phases["pme_gather"] + phases["pair_forces"],
+                      (28.0 + 24.0 + 48.0) * total_atoms + 96.0 * entries + 4.0 * points),
         "grid_points": points,
+        "list_entries": entries,
     }
 
     result = {

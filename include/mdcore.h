@@ -226,8 +226,8 @@ md_err md_set_step(md_system *sys, int64_t step);
  * runs one system per device, and this attaches to its per-system state and
  * step ring (loop.ts:171, 434-445, 715-751).  A batch advances several
  * independent systems of any sizes together: each phase of a step is ONE
- * kernel launch covering every replica (the pair kernel's waves draw list
- * segments of all replicas from one counter), and strides of steps are
+ * kernel launch covering every replica (the pair kernel's waves take fixed
+ * runs of all replicas' list segments), and strides of steps are
  * captured as HIP graphs.  Each replica keeps its own state, options
  * (temperature, seed, ...) and every per-system call above; the batch borrows
  * the systems, which must all use the same device and outlive it.  Calls on

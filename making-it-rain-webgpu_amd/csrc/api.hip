@@ -655,7 +655,9 @@ void md_mark(md_group *g, int phase) {
 // other uses; the order of integer sums is no matter, so every bit is the same.
 // Fork and join cost less than they give at all sizes measured: a step of 2,168
 // atoms 120 to 103 us, of 31k 195 to 178, of 243k 684 to 644, of 64 replicas
-// 2,026 to 1,925.  A profiled step runs in one line, so that phases can be timed.
+// 2,026 to 1,925.  At the last two the mesh's branch is the longer one: beside
+// the pairs its spreading takes about four times as long as by itself (84 to 334
+// us, 258 to 1,016).  A profiled step runs in one line, so that phases can be timed.
 void md_force_kernels(md_group *g, bool advance, bool energy, bool rebuild) {
   md_mark(g, MD_PHASE_PROLOGUE);
   if (!g->nb) {

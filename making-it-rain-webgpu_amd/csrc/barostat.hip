@@ -21,7 +21,6 @@
 //                         the proposal width adapted every 10 attempts
 //   k_baro_restore        a rejected trial's positions put back
 //   box constants         from the box that won
-//   zero forces           the next step starts from clean accumulators
 //
 // The arithmetic follows the host path (mdcore/barostat.py) operation for
 // operation, with contraction into fused multiply-adds off, so a device
